@@ -153,6 +153,18 @@ template <typename R>
 hipError_t launch_chunk_sums(const void *psi, int n, uint64_t chunk, double *d_out,
                              hipStream_t s);
 
+// One inverse-CDF sample: the chunk it lies in, the sum of the chunks before
+// it, and the value the running sum has to exceed.
+struct SampleShot {
+  uint64_t chunk;
+  double run, tau;
+};
+
+// d_out[j] = the basis index of shot j (count < 2^31).
+template <typename R>
+hipError_t launch_sample(const void *psi, uint64_t chunk, const SampleShot *d_shots,
+                         uint64_t count, uint64_t *d_out, hipStream_t s);
+
 // ---- fused sweep engine (qs_sweep.hip) --------------------------------------
 struct SweepPlan;  // defined in qs_sweep.h
 }  // namespace qs

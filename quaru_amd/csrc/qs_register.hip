@@ -18,7 +18,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -119,6 +118,8 @@ constexpr size_t kRingBytes = 8u << 20;
 // so they allocate nothing after the first call.
 constexpr int kReadoutBits = 22;
 constexpr uint64_t kReadoutAmps = 1ull << kReadoutBits;
+// Shots of qs_sample_cdf scanned per launch (2 MiB of work buffer).
+constexpr size_t kSamplePiece = 1u << 16;
 constexpr size_t kRedDoubles = 4 * qs::kReduceBlocks + 64;
 
 bool valid_dtype(int d) { return d == QS_C128 || d == QS_C64; }
@@ -1238,9 +1239,14 @@ int qs_sample_cdf(qs_register *r, const double *uniforms, size_t count, uint64_t
   if (count == 0) return QS_OK;
   const uint64_t chunk = std::min<uint64_t>(r->len, 1ull << 16);
   const uint64_t nchunks = (r->len + chunk - 1) / chunk;
+  const size_t piece = std::min<size_t>(count, kSamplePiece);
   std::vector<double> sums(nchunks);
   double *d_sums = nullptr;
-  QS_HIP(ensure_big(r, std::max<uint64_t>(nchunks, chunk) * sizeof(double), &d_sums));
+  QS_HIP(ensure_big(r, nchunks * sizeof(double) +
+                           piece * (sizeof(qs::SampleShot) + sizeof(uint64_t)),
+                    &d_sums));
+  qs::SampleShot *d_shots = reinterpret_cast<qs::SampleShot *>(d_sums + nchunks);
+  uint64_t *d_idx = reinterpret_cast<uint64_t *>(d_shots + piece);
   hipError_t e = by_dtype(r, [&](auto z) {
     return qs::launch_chunk_sums<decltype(z)>(r->psi, r->n, chunk, d_sums, r->stream);
   });
@@ -1252,44 +1258,29 @@ int qs_sample_cdf(qs_register *r, const double *uniforms, size_t count, uint64_t
   std::vector<double> prefix(nchunks + 1, 0.0);
   for (uint64_t c = 0; c < nchunks; ++c) prefix[c + 1] = prefix[c] + sums[c];
   const double total = prefix[nchunks];
-  std::map<uint64_t, std::vector<double>> chunk_probs;
-  for (size_t j = 0; j < count && e == hipSuccess; ++j) {
-    const double tau = uniforms[j] * total;
-    // first chunk whose running sum exceeds tau
-    uint64_t c = (uint64_t)(std::upper_bound(prefix.begin() + 1, prefix.end(), tau) -
-                            (prefix.begin() + 1));
-    if (c >= nchunks) c = nchunks - 1;
-    auto it = chunk_probs.find(c);
-    if (it == chunk_probs.end()) {
-      std::vector<double> pr(chunk);
+  std::vector<qs::SampleShot> shots(piece);
+  for (size_t off = 0; off < count; off += piece) {
+    const size_t cnt = std::min(piece, count - off);
+    for (size_t j = 0; j < cnt; ++j) {
+      const double tau = uniforms[off + j] * total;
+      // first chunk whose running sum exceeds tau
+      uint64_t c = (uint64_t)(std::upper_bound(prefix.begin() + 1, prefix.end(), tau) -
+                              (prefix.begin() + 1));
+      if (c >= nchunks) c = nchunks - 1;
+      shots[j] = {c, prefix[c], tau};
+    }
+    e = hipMemcpyAsync(d_shots, shots.data(), cnt * sizeof(qs::SampleShot),
+                       hipMemcpyHostToDevice, r->stream);
+    if (e == hipSuccess)
       e = by_dtype(r, [&](auto z) {
-        using R = decltype(z);
-        const size_t ab = r->amp_bytes();
-        return qs::launch_probabilities<R>((const char *)r->psi + c * chunk * ab,
-                                           (int)(63 - __builtin_clzll(chunk)), d_sums, r->stream);
+        return qs::launch_sample<decltype(z)>(r->psi, chunk, d_shots, cnt, d_idx, r->stream);
       });
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(pr.data(), d_sums, chunk * sizeof(double), hipMemcpyDeviceToHost,
-                           r->stream);
-      if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
-      it = chunk_probs.emplace(c, std::move(pr)).first;
-    }
-    const std::vector<double> &pr = it->second;
-    double run = prefix[c];
-    uint64_t x = c * chunk + chunk - 1, last_nz = x;
-    bool found = false;
-    for (uint64_t i = 0; i < chunk; ++i) {
-      if (pr[i] > 0.0) last_nz = c * chunk + i;
-      run += pr[i];
-      if (run > tau) {
-        x = c * chunk + i;
-        found = true;
-        break;
-      }
-    }
-    indices[j] = found ? x : last_nz;
+    if (e == hipSuccess)
+      e = hipMemcpyAsync(indices + off, d_idx, cnt * sizeof(uint64_t), hipMemcpyDeviceToHost,
+                         r->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
+    if (e != hipSuccess) return hip_fail(e, "qs_sample_cdf");
   }
-  if (e != hipSuccess) return hip_fail(e, "qs_sample_cdf");
   return QS_OK;
 }
 

@@ -539,6 +539,44 @@ def test_sample_cdf():
     assert np.array_equal(got, exp)
 
 
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+@pytest.mark.parametrize("n", [0, 1, 5, 9, 10, 11, 16, 17, 18])
+def test_sample_cdf_exact_sums(n, dtype):
+    # amplitudes that are small integers: every sum is exact in any order, so
+    # ties (tau on a prefix sum) and the ends of the range are decided exactly
+    rng = np.random.default_rng(80 + n)
+    psi = rng.integers(0, 4, 1 << n) * np.where(rng.random(1 << n) < 0.5, 1, 1j)
+    psi[rng.random(1 << n) < 0.3] = 0
+    psi[-3:] = 0
+    psi[0] = 2
+    r = Register.from_int(n, 0, dtype=dtype, seed=1)
+    r.state = psi
+    p = np.abs(psi).round().astype(np.int64) ** 2
+    cdf = np.cumsum(p)
+    total = int(cdf[-1])
+    # cdf / total * total need not be exact: keep the u that hit their tau
+    u = np.concatenate([np.arange(0, 64) / 64, cdf[:: max(1, cdf.size // 200)] / total])
+    u = u[(u < 1) & ((u * total == np.round(u * total)) | (u * 64 == np.round(u * 64)))]
+    got = r.sample(u)
+    exp = np.searchsorted(cdf, u * float(total), side="right")
+    assert np.array_equal(got, exp)
+    # at and past the total: the last chunk's last amplitude above 0
+    chunk = min(1 << n, 1 << 16)
+    tail = p[-chunk:]
+    end = (1 << n) - chunk + (np.nonzero(tail)[0][-1] if tail.any() else chunk - 1)
+    assert np.array_equal(r.sample([1.0, 1.5, -0.25]), [end, end, 0])
+
+
+def test_sample_cdf_many_shots():
+    # more shots than one launch takes
+    n = 4
+    psi = np.ones(1 << n) / 4.0
+    r = Register.from_int(n, 0, dtype="c128", seed=1)
+    r.state = psi
+    u = (np.arange(70001) % 16) / 16
+    assert np.array_equal(r.sample(u), np.arange(70001) % 16)
+
+
 # ---- reductions and equality ---------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", ["c128", "c64"])
