@@ -34,6 +34,7 @@
 #include "../../include/quaru_hip.h"
 #include "qs_internal.h"
 #include "qs_sweep.h"
+#include "qs_sweep_kernel.h"
 
 namespace {
 
@@ -65,6 +66,10 @@ int fail_arg(const char *msg) { return qs::set_error(QS_ERR_ARGUMENT, 0, 0, msg)
 __device__ __forceinline__ uint64_t insert0(uint64_t p, int q) {
   const uint64_t lo = p & ((1ull << q) - 1ull);
   return ((p ^ lo) << 1) | lo;
+}
+
+__device__ __forceinline__ uint32_t insert0_32(uint32_t p, uint32_t q) {
+  return p + (p & ~((1u << q) - 1u));
 }
 
 template <typename R>
@@ -259,202 +264,417 @@ __global__ __launch_bounds__(kBlock) void k_fill_zero(double *p, uint64_t count)
     p[i] = 0.0;
 }
 
-// ---- fused reverse pass.  The reverse sweep runs in blocks of consecutive
-// operations whose pair targets fit one tile of T qubits (the low qubits
-// always among them, for contiguous loads).  A workgroup loads its tile of
-// psi and of lambda into LDS, runs the block's reverse steps there (each
-// rotation: the tile's share of Im <lambda|sigma|psi>, then U^dagger on
-// both; each fixed gate: its inverse on both) and writes the tile back:
-// one pass over psi and lambda per block instead of one per operation.
-// Diagonal and phase gates act on any qubits (their bits off the tile are
-// the same for the whole tile).
-enum : uint32_t { REV_ROT = 1, REV_PHASE = 2, REV_DIAG = 3, REV_U1 = 4 };
-
-struct RevRec {
-  uint32_t kind;
-  uint32_t k;      // tile bit of the target (REV_ROT, REV_U1)
-  uint32_t axis;   // REV_ROT: rotation axis; REV_DIAG: number of act bits
-  uint32_t rslot;  // REV_ROT: rotation slot of the matrix table
-  uint32_t out;    // REV_ROT: row of the partial sums
-  uint32_t moff;   // values at vals[moff..] as {re, im} pairs
-  int32_t a0, a1;  // REV_DIAG: act bits: tile bit (>= 0) or -1 - global qubit
-  uint64_t umask, uval;  // pattern bits off the tile (global index bits)
-  uint64_t lmask, lval;  // pattern bits on the tile (tile bits)
-};
-
-constexpr int kRevMaxOps = 64;
+// ---- fused reverse pass.  The reverse sweep runs in blocks of operations
+// whose pair targets fit one tile of T qubits (the low qubits always among
+// them, for contiguous loads), taken out of order where they commute
+// (reverse_blocks).  A workgroup loads its tile of psi and of lambda into
+// LDS, runs the block's reverse steps there (each rotation: the tile's share
+// of Im <lambda|sigma|psi>, then U^dagger on both; each fixed gate: its
+// inverse on both) and writes the tile back: one pass over psi and lambda per
+// block instead of one per operation.  The records of a block come in passes
+// over the tile:
+//  * a diagonal pass: any run of phases, diagonals and Z rotations, on tile
+//    qubits or not.  All of them multiply psi and lambda by the same factor
+//    of modulus 1, so w(x) = Im(conj(lambda_x) psi_x) is the same before and
+//    after each, and the gradient of the Z rotation on qubit q is the sum of
+//    (-1)^(x_q) w(x): wave_signed gives the sums of all six lane qubits and
+//    the total at once.
+//  * a pair pass: one X or Y rotation, or two on different tile qubits, on
+//    pairs or quads of amplitudes.
+//  * a 2x2 pass: the inverse of a (controlled) fixed 2x2.
+constexpr int kRevMaxOps = 192;  // records per block
+constexpr int kRevMaxRows = 64;  // rotations per block
+constexpr int kRevMaxSlots = 32;  // rotations per block summed by RowSums
+constexpr int kRevMaxOff = 16;   // Z rotations off the tile per diagonal pass
 constexpr int kRevMaxTile = 16;
 constexpr int kRevMaxBits = 11;  // tile of at most 2^11 amplitudes
+constexpr uint32_t kRevNone = 255;
 
-struct RevHeader {
-  uint32_t T, nops, nrot, nvals;
-  uint32_t tq[kRevMaxTile];  // tile qubits, ascending
+// One pass.  REV_ROT: k = first | second << 8 tile bit | X flags << 16 (bit
+// 16 the first is an X rotation, bit 17 the second) | a second one << 18;
+// rows = row | row2 << 8 | slot << 16, the second's slot the next one.
+// REV_U1: rows = index of its record.  REV_DIAGS: rows = index of its RevDiag.
+enum : uint32_t { REV_ROT = 1, REV_U1 = 2, REV_DIAGS = 3, REV_PHASE = 4, REV_DIAG = 5, REV_RZ = 6 };
+
+struct RevPass {
+  uint32_t kind, k, rows, pad;
 };
 
-// One reverse step of a rotation on the pair (x0, x1) of psi and (l0, l1) of
-// lambda: acc += Im(conj(l0) s0 + conj(l1) s1) with s = sigma . psi, then
-// U^dagger = [[conj m0, conj m2], [conj m1, conj m3]] on both pairs.
-template <typename R>
+// A diagonal pass: rz[k] = the row of the Z rotation on tile bit k (kRevNone:
+// none); lane_row: word offset of 64 bytes, the row that each lane's sum goes
+// to (kRevNone: none); the Z rotations off the tile, off[o0 .. o0 + noff) = row |
+// qubit << 8; sign: word offset of the tile's sign table, one bit per
+// amplitude, the parity of the phases of -1 with patterns on the tile alone
+// (~0: none); and records first .. first + count for everything else.
+struct RevDiag {
+  uint32_t nrz, sign, o0, noff, first, count, lane_row, pad;
+  uint32_t rz[kRevMaxTile];
+};
+
+// A phase, a diagonal, a further Z rotation on a qubit, or a 2x2.
+struct RevRec {
+  uint32_t kind;
+  uint32_t k;      // tile bit of the target (REV_U1, REV_RZ: kRevNone off the tile)
+  uint32_t axis;   // REV_DIAG: number of act bits
+  uint32_t out;    // REV_RZ: row of the partial sums
+  uint32_t moff;   // values at vals[moff..] as {re, im} pairs
+  int32_t a0, a1;  // REV_DIAG: act bits: tile bit (>= 0) or -1 - global qubit; REV_RZ: qubit
+  uint32_t slot;   // REV_RZ in complex64
+  uint32_t lmask, lval;  // pattern bits on the tile (tile bits)
+  uint32_t pad2[2];
+  uint64_t umask, uval;  // pattern bits off the tile (global index bits)
+};
+
+// The descriptor: header, passes, diagonal passes, records, then values; the
+// tables that threads read by their index (row slots, parameters, off-tile Z
+// rotations, signs) behind them, at word offset `tab`.
+struct RevHeader {
+  uint32_t T, npass, nrot, nslot;
+  uint32_t ndiag, nrec, tab, params;  // params: word offset of the parameter table
+  uint32_t tq[kRevMaxTile];       // tile qubits, ascending
+  uint32_t row_of[kRevMaxSlots];  // row of the rotation with that slot
+};
+
+// One reverse step of an X or Y rotation on the pair (x0, x1) of psi and
+// (l0, l1) of lambda: acc += Im(conj(l0) s0 + conj(l1) s1) with s = sigma .
+// psi, then U^dagger on both up to a real factor.  U^dagger is [[c, i s],
+// [i s, c]] (X) or [[c, s], [-s, c]] (Y); its entries are divided by the
+// larger of c and s in modulus (by s: kSwap), so that each output is one
+// multiply-add per component: t = s / c or c / s, |t| <= 1.  The factor is
+// the same for the whole tile: it is applied once, when the tile is stored.
+template <typename R, bool kX, bool kSwap>
 __device__ __forceinline__ void rot_reverse_pair(typename AV2<R>::T &x0, typename AV2<R>::T &x1,
                                                  typename AV2<R>::T &l0, typename AV2<R>::T &l1,
-                                                 uint32_t axis, const typename AV2<R>::T *m,
-                                                 double &acc) {
+                                                 R t, double &acc) {
   using T = typename AV2<R>::T;
-  double s0r, s0i, s1r, s1i;
-  if (axis == 0) {
-    s0r = x1.x; s0i = x1.y; s1r = x0.x; s1i = x0.y;
-  } else if (axis == 1) {
-    s0r = x1.y; s0i = -(double)x1.x; s1r = -(double)x0.y; s1i = x0.x;
+  if constexpr (kX)
+    acc += (double)l0.x * x1.y - (double)l0.y * x1.x + (double)l1.x * x0.y - (double)l1.y * x0.x;
+  else
+    acc += (double)l1.x * x0.x + (double)l1.y * x0.y - (double)l0.x * x1.x - (double)l0.y * x1.y;
+  auto turn = [t](T &a, T &b) {
+    T u, v;
+    if constexpr (kX) {
+      if constexpr (kSwap) {
+        u.x = fma(t, a.x, -b.y);
+        u.y = fma(t, a.y, b.x);
+        v.x = fma(t, b.x, -a.y);
+        v.y = fma(t, b.y, a.x);
+      } else {
+        u.x = fma(-t, b.y, a.x);
+        u.y = fma(t, b.x, a.y);
+        v.x = fma(-t, a.y, b.x);
+        v.y = fma(t, a.x, b.y);
+      }
+    } else {
+      if constexpr (kSwap) {
+        u.x = fma(t, a.x, b.x);
+        u.y = fma(t, a.y, b.y);
+        v.x = fma(t, b.x, -a.x);
+        v.y = fma(t, b.y, -a.y);
+      } else {
+        u.x = fma(t, b.x, a.x);
+        u.y = fma(t, b.y, a.y);
+        v.x = fma(-t, a.x, b.x);
+        v.y = fma(-t, a.y, b.y);
+      }
+    }
+    a = u;
+    b = v;
+  };
+  turn(x0, x1);
+  turn(l0, l1);
+}
+
+// The same in complex64: every product and sum rounded as k_rot_reverse
+// rounds it (cs = {c, s}, no factor taken out), so that a gradient does not
+// depend on how the operations fall into blocks.
+template <bool kX>
+__device__ __forceinline__ void rot_reverse_pair_f(float2 &x0, float2 &x1, float2 &l0, float2 &l1,
+                                                   float2 cs, double &acc) {
+  if constexpr (kX)
+    acc += (double)l0.x * x1.y - (double)l0.y * x1.x + (double)l1.x * x0.y - (double)l1.y * x0.x;
+  else
+    acc += (double)l1.x * x0.x + (double)l1.y * x0.y - (double)l0.x * x1.x - (double)l0.y * x1.y;
+  const float c = cs.x, s = cs.y;
+  auto turn = [c, s](float2 &a, float2 &b) {
+    float2 u, v;
+    if constexpr (kX) {
+      u.x = fmaf(-s, b.y, __fmul_rn(c, a.x));
+      u.y = fmaf(s, b.x, __fmul_rn(c, a.y));
+      v.x = fmaf(c, b.x, __fmul_rn(-s, a.y));
+      v.y = fmaf(c, b.y, __fmul_rn(s, a.x));
+    } else {
+      u.x = fmaf(s, b.x, __fmul_rn(c, a.x));
+      u.y = fmaf(s, b.y, __fmul_rn(c, a.y));
+      v.x = fmaf(c, b.x, __fmul_rn(-s, a.x));
+      v.y = fmaf(c, b.y, __fmul_rn(-s, a.y));
+    }
+    a = u;
+    b = v;
+  };
+  turn(x0, x1);
+  turn(l0, l1);
+}
+
+// U^dagger of a Z rotation on one amplitude, in complex64, rounded as
+// k_rot_reverse rounds the bit-clear (s > 0) and the bit-set side.
+__device__ __forceinline__ float2 rz_reverse_f(float2 a, float2 cs, bool bit) {
+  const float c = cs.x, s = cs.y;
+  float2 u;
+  if (!bit) {
+    u.x = fmaf(c, a.x, __fmul_rn(-s, a.y));
+    u.y = fmaf(c, a.y, __fmul_rn(s, a.x));
   } else {
-    s0r = x0.x; s0i = x0.y; s1r = -(double)x1.x; s1i = -(double)x1.y;
+    u.x = fmaf(s, a.y, __fmul_rn(c, a.x));
+    u.y = fmaf(-s, a.x, __fmul_rn(c, a.y));
   }
-  acc += (double)l0.x * s0i - (double)l0.y * s0r + (double)l1.x * s1i - (double)l1.y * s1r;
-  const T m0 = m[0], m1 = m[1], m2 = m[2], m3 = m[3];
-  T y0, y1, k0, k1;
-  y0.x = m0.x * x0.x + m0.y * x0.y + m2.x * x1.x + m2.y * x1.y;
-  y0.y = m0.x * x0.y - m0.y * x0.x + m2.x * x1.y - m2.y * x1.x;
-  y1.x = m1.x * x0.x + m1.y * x0.y + m3.x * x1.x + m3.y * x1.y;
-  y1.y = m1.x * x0.y - m1.y * x0.x + m3.x * x1.y - m3.y * x1.x;
-  k0.x = m0.x * l0.x + m0.y * l0.y + m2.x * l1.x + m2.y * l1.y;
-  k0.y = m0.x * l0.y - m0.y * l0.x + m2.x * l1.y - m2.y * l1.x;
-  k1.x = m1.x * l0.x + m1.y * l0.y + m3.x * l1.x + m3.y * l1.y;
-  k1.y = m1.x * l0.y - m1.y * l0.x + m3.x * l1.y - m3.y * l1.x;
-  x0 = y0;
-  x1 = y1;
-  l0 = k0;
-  l1 = k1;
+  return u;
 }
 
-// Sum over the 64 lanes of a wave, every lane receiving the total: an xor
-// butterfly on VALU cross-lane moves (DPP within rows of 16, gfx950's
-// permlane swaps across them) instead of LDS-crossbar shuffles.
-__device__ __forceinline__ int dpp_i(int v, int ctrl) {
-  switch (ctrl) {
-    case 0: return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
-    case 1: return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
-    case 2: return __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, false);  // row_half_mirror
-    default: return __builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, false); // row_mirror
+// The pair step of either precision; cs is the rotation's entry of the
+// kernel's table.
+template <typename R, bool kX, bool kSwap>
+__device__ __forceinline__ void rot_pair(typename AV2<R>::T &x0, typename AV2<R>::T &x1,
+                                         typename AV2<R>::T &l0, typename AV2<R>::T &l1,
+                                         typename AV2<R>::T cs, double &acc) {
+  if constexpr (sizeof(R) == 4)
+    rot_reverse_pair_f<kX>(x0, x1, l0, l1, cs, acc);
+  else
+    rot_reverse_pair<R, kX, kSwap>(x0, x1, l0, l1, cs.x, acc);
+}
+
+// Calls f(integral_constant kX, integral_constant kSwap); form bit 0: X, bit
+// 1: swapped (the same for the whole wave).
+template <typename F>
+__device__ __forceinline__ void rot_form(uint32_t form, F &&f) {
+  using std::integral_constant;
+  if (form & 1u) {
+    if (form & 2u)
+      f(integral_constant<bool, true>{}, integral_constant<bool, true>{});
+    else
+      f(integral_constant<bool, true>{}, integral_constant<bool, false>{});
+  } else {
+    if (form & 2u)
+      f(integral_constant<bool, false>{}, integral_constant<bool, true>{});
+    else
+      f(integral_constant<bool, false>{}, integral_constant<bool, false>{});
   }
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-  // steps 1, 2: lane ^ 1, lane ^ 2; then every quad is uniform, so the half
-  // mirror adds the other quad of each 8 and the row mirror the other 8
+// Lane l ^ 2^K's value by VALU cross-lane moves.
+template <int K>
+__device__ __forceinline__ double lane_x(double v) {
+  return qs::sweep::lane_xor<K>(v, (threadIdx.x >> K) & 1);
+}
+
+// Sums over the lanes for up to 32 rotations of a block, by matrix
+// instructions: a 4 x 4 matrix whose row `slot` is ones times a 4 x 4 matrix
+// of 16 lanes' values (lanes 16 k + c for k < 4 a column) adds the sums of
+// the columns to row `slot` of a 4 x 4 FP64 accumulator; four such products
+// side by side take the wave's 64 values.  The 16 columns are added once, at
+// the end of the block, so a rotation's share costs one 16-cycle instruction
+// instead of a six-step exchange over the wave.
+struct RowSums {
+  double d[kRevMaxSlots / 4];
+};
+
+__device__ __forceinline__ void row_add(RowSums &rs, uint32_t slot, double v) {
+  const double a = (threadIdx.x & 3u) == (slot & 3u) ? 1.0 : 0.0;
+  const uint32_t g = slot >> 2;  // the same for the whole wave
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {
-    const long long b = __double_as_longlong(v);
-    const int lo = dpp_i((int)(b & 0xffffffffll), c), hi = dpp_i((int)(b >> 32), c);
-    v += __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-  }
-  // rows: every row of 16 is uniform; the swaps hand each lane the value of
-  // the row 16 (then 32) lanes away
-  const long long b16 = __double_as_longlong(v);
-  const auto l16 = __builtin_amdgcn_permlane16_swap((int)(b16 & 0xffffffffll),
-                                                    (int)(b16 & 0xffffffffll), false, false);
-  const auto h16 = __builtin_amdgcn_permlane16_swap((int)(b16 >> 32), (int)(b16 >> 32), false,
-                                                    false);
-  const bool r16 = (threadIdx.x >> 4) & 1;
-  const int lo16 = r16 ? l16[0] : l16[1], hi16 = r16 ? h16[0] : h16[1];
-  v += __longlong_as_double(((long long)hi16 << 32) | (unsigned int)lo16);
-  const long long b32 = __double_as_longlong(v);
-  const auto l32 = __builtin_amdgcn_permlane32_swap((int)(b32 & 0xffffffffll),
-                                                    (int)(b32 & 0xffffffffll), false, false);
-  const auto h32 = __builtin_amdgcn_permlane32_swap((int)(b32 >> 32), (int)(b32 >> 32), false,
-                                                    false);
-  const bool r32 = (threadIdx.x >> 5) & 1;
-  const int lo32 = r32 ? l32[0] : l32[1], hi32 = r32 ? h32[0] : h32[1];
-  return v + __longlong_as_double(((long long)hi32 << 32) | (unsigned int)lo32);
+  for (uint32_t i = 0; i < kRevMaxSlots / 4; ++i)
+    if (g == i) rs.d[i] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, v, rs.d[i], 0, 0, 0);
 }
 
-// One workgroup per tile (grid = ntiles); dynamic LDS 2 x 2^T amplitudes;
-// PER = max(1, 2^T / 256).  part[out * ntiles + tile] = the tile's share of
-// rotation `out`'s gradient.
+template <int K>
+__device__ __forceinline__ double wht_step(double v) {
+  const double o = lane_x<K>(v);
+  return ((threadIdx.x >> K) & 1) ? o - v : v + o;
+}
+
+// Sums over the wave signed by one lane bit: lane 0 receives the total, lane
+// 2^k the sum of (-1)^(bit k of lane) v.  Lane bits 4 and 5 by one matrix
+// instruction (rows of ones, of the signs of bit 4 and of bit 5 times the 4 x
+// 16 matrix of the lanes' values), bits 0 to 3 by a Walsh-Hadamard butterfly
+// over each of those rows.
+__device__ __forceinline__ double wave_signed(double v) {
+  const uint32_t i = threadIdx.x & 3u, k = (threadIdx.x >> 4) & 3u;
+  const double a = i == 3 ? 0.0 : ((i & k) ? -1.0 : 1.0);
+  v = __builtin_amdgcn_mfma_f64_4x4x4f64(a, v, 0.0, 0, 0, 0);
+  v = wht_step<0>(v);
+  v = wht_step<1>(v);
+  v = wht_step<2>(v);
+  return wht_step<3>(v);
+}
+
+// LDS position of tile amplitude j: the low three bits are XORed with the
+// next three, so that the strided reads of a pair pass on a low tile bit
+// spread over the banks.  Linear over XOR: pos(j ^ b) = pos(j) ^ pos(b).
+__device__ __forceinline__ uint32_t rev_pos(uint32_t j) { return j ^ ((j >> 3) & 7u); }
+
+// One workgroup per tile (grid = ntiles); dynamic LDS 2 x 2^T amplitudes (at
+// least 256); PER = max(1, 2^T / 256).  part[tile * nrot + row] = the tile's
+// share of the gradient of the rotation with that row.
+//
+// Bound by vector and LDS work beside the memory pass.  Backward of the
+// 20-qubit, 10-layer, batch-64 ansatz, complex128 (15 blocks, 4 GiB of
+// traffic each, 0.81 ms at the card's copy rate): 24.2 ms, 1.24 ms per block
+// with the vector units 51% busy (1490 instructions per wave).  Steps there:
+// 66 ms (55 blocks of 1.11 ms, operations in strict order, one exchange and
+// one descriptor fetch per rotation); 34.5 ms with commuting blocks and
+// diagonal passes (2280 instructions); 28.4 ms with descriptors fetched
+// ahead, cosines and sines in LDS and sums on the matrix cores (by 16 x 16
+// FP64 products instead of 4 x 4: 35.7 ms); 24.2 ms with one multiply-add per
+// component and tables for signs and lane sums.  Complex64: 45 to 17.8 ms.
+// Tiles of 2^11 complex128 amplitudes, two workgroups per CU: 27.3 ms.
 template <typename R, int PER>
-__global__ __launch_bounds__(kBlock) void k_reverse_tile(typename AV2<R>::T *__restrict__ psi,
+__global__ __launch_bounds__(kBlock)
+__attribute__((amdgpu_waves_per_eu(PER < 8 ? 4 : (sizeof(R) == 8 ? 2 : 3)))) void k_reverse_tile(typename AV2<R>::T *__restrict__ psi,
                                                          typename AV2<R>::T *__restrict__ lam,
-                                                         int n, const char *__restrict__ blob,
+                                                         int n, const char *__restrict__ blob_g,
                                                          const typename AV2<R>::T *__restrict__ rot,
-                                                         uint64_t Bp, double *__restrict__ part,
-                                                         uint64_t ntiles) {
+                                                         uint64_t Bp, double *__restrict__ part) {
   using T = typename AV2<R>::T;
+  constexpr int PB = PER == 1 ? 0 : (PER == 2 ? 1 : (PER == 4 ? 2 : 3));  // bits of i
+  constexpr bool kExact = sizeof(R) == 4;  // complex64: see rot_reverse_pair_f
   extern __shared__ unsigned char rev_smem[];
-  __shared__ double red[4][kBlock / 64];
-  const RevHeader &h = *(const RevHeader *)blob;
-  const RevRec *recs = (const RevRec *)(blob + sizeof(RevHeader));
-  const R *vals = (const R *)(blob + sizeof(RevHeader) + h.nops * sizeof(RevRec));
+  __shared__ double rows[kRevMaxRows][kBlock / 64];  // per wave, summed at the end
+  // per rotation: X and Y {t, factor} and form (rot_reverse_pair), Z {cos, sin}
+  // of half the angle; scale[s]: the square of the factors of the slots below
+  __shared__ T cs[kRevMaxRows];
+  __shared__ uint32_t form[kRevMaxRows];
+  __shared__ double scale[kRevMaxSlots + 1];
+  // what is the same for every lane is read through the constant address
+  // space, on scalar loads
+  const QS_CONST char *blob = (const QS_CONST char *)blob_g;
+  const QS_CONST RevHeader &h = *(const QS_CONST RevHeader *)blob;
+  const QS_CONST RevPass *passes = (const QS_CONST RevPass *)(blob + sizeof(RevHeader));
+  const QS_CONST RevDiag *diags = (const QS_CONST RevDiag *)(passes + h.npass);
+  const QS_CONST RevRec *recs = (const QS_CONST RevRec *)(diags + h.ndiag);
+  const QS_CONST R *vals = (const QS_CONST R *)(recs + h.nrec);
+  const uint32_t *tab = (const uint32_t *)blob_g + h.tab;
   const int Tt = (int)h.T;
   const uint32_t E = 1u << Tt;
+  const uint32_t tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
+  constexpr uint32_t EO = (uint32_t)PER * kBlock;  // lambda lies EO amplitudes behind psi
   T *ps = (T *)rev_smem;
-  T *ls = ps + E;
+  T *ls = ps + EO;
   const uint64_t tile = blockIdx.x;
   uint64_t base = tile;
   for (int i = 0; i < Tt; ++i) base = insert0(base, (int)h.tq[i]);
   const uint64_t b = base >> n;
-  // Amplitude j = threadIdx.x + 256 i of the tile: the thread index gives
-  // its low 8 tile bits, i the rest (the same for the whole workgroup).  All
-  // loads of the tile are issued before the first is waited for.
+  // Amplitude j = tid + 256 i of the tile: the thread index gives its low 8
+  // tile bits, i the rest (the same for the whole workgroup).  All loads of
+  // the tile are issued before the first is waited for.
   const int tb = Tt < 8 ? Tt : 8;
   uint64_t toff = 0;
   for (int i = 0; i < tb; ++i)
-    if ((threadIdx.x >> i) & 1u) toff |= 1ull << h.tq[i];
+    if ((tid >> i) & 1u) toff |= 1ull << h.tq[i];
   // PER amplitudes per thread (2^T / 256, at least 1: a tile of fewer than
   // 256 amplitudes leaves the other threads idle)
-  const bool active = threadIdx.x < E;
+  const bool active = tid < E;
   uint64_t ioff[PER];
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     uint64_t o = 0;
-    for (int k = 8; k < Tt; ++k)
-      if ((i >> (k - 8)) & 1) o |= 1ull << h.tq[k];
+#pragma unroll
+    for (int k = 0; k < PB; ++k)
+      if ((i >> k) & 1) o |= 1ull << h.tq[8 + k];
     ioff[i] = base | toff | o;
   }
+  const uint32_t tpos = rev_pos(tid);
   typedef R V __attribute__((ext_vector_type(2)));
   const V *psv = reinterpret_cast<const V *>(psi), *lav = reinterpret_cast<const V *>(lam);
   V *psl = reinterpret_cast<V *>(ps), *lsl = reinterpret_cast<V *>(ls);
-  if (active) {
+  {
     V xv[PER], lv[PER];
+    if (active) {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      xv[i] = psv[ioff[i]];
-      lv[i] = lav[ioff[i]];
+      for (int i = 0; i < PER; ++i) {
+        xv[i] = psv[ioff[i]];
+        lv[i] = lav[ioff[i]];
+      }
     }
+    // a thread per rotation fetches its angle's cosine and sine: m[0] = c (X,
+    // Y) or c - i s (Z); m[2] = -i s (X) or s (Y)
+    if (tid < h.nrot) {
+      const uint32_t a = tab[tid] >> 30;  // axis
+      const R *m = (const R *)(rot + ((uint64_t)(tab[tid] & 0x3fffffffu) * Bp + b) * 4);
+      const R c = m[0], s = a == 0 ? -m[5] : (a == 1 ? m[4] : -m[1]);
+      const bool swap = !kExact && !(fabs(c) >= fabs(s));
+      T v;
+      v.x = kExact || a == 2 ? c : (swap ? c / s : s / c);
+      v.y = kExact || a == 2 || swap ? s : c;
+      cs[tid] = v;
+      form[tid] = (a == 0 ? 1u : 0u) | (swap ? 2u : 0u);
+    }
+    if (active) {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      psl[threadIdx.x + i * kBlock] = xv[i];
-      lsl[threadIdx.x + i * kBlock] = lv[i];
+      for (int i = 0; i < PER; ++i) {
+        psl[tpos + i * kBlock] = xv[i];
+        lsl[tpos + i * kBlock] = lv[i];
+      }
     }
   }
   __syncthreads();
-  for (uint32_t o = 0; o < h.nops; ++o) {
-    const RevRec &r = recs[o];
+  // the factor of the whole tile, and the squares by which the sums taken
+  // before it is applied are off: the product over the slots, by one wave
+  R whole = 1;
+  if constexpr (!kExact) {
+    const uint32_t row = (uint32_t)lane < h.nslot ? h.row_of[lane & (kRevMaxSlots - 1)] : 0u;
+    double f = 1.0;
+    if ((uint32_t)lane < h.nslot) f = cs[row].y;
+    double pre = f;  // inclusive products
+#pragma unroll
+    for (int d = 1; d < kRevMaxSlots; d <<= 1) {
+      const double o = __shfl_up(pre, d);
+      if (lane >= d) pre *= o;
+    }
+    whole = (R)__shfl(pre, kRevMaxSlots - 1);
+    if (wave == 0 && lane < kRevMaxSlots) {
+      scale[lane + 1] = pre * pre;
+      if (lane == 0) scale[0] = 1.0;
+    }
+  }
+  RowSums sums = {};
+  const uint32_t npass = h.npass;
+  RevPass nx = {passes[0].kind, passes[0].k, passes[0].rows, 0};
+  for (uint32_t o = 0; o < npass; ++o) {
+    const RevPass r = nx;
+    // the next pass's record, fetched during this one (behind the last pass
+    // lies more of the descriptor)
+    nx.kind = passes[o + 1].kind;
+    nx.k = passes[o + 1].k;
+    nx.rows = passes[o + 1].rows;
     if (r.kind == REV_ROT) {
-      // two consecutive rotations on different tile bits run in one pass
-      // over quads of amplitudes; rows use four buffers by row number, so a
-      // buffer is rewritten only after a barrier that thread 0 passes after
-      // reading it
-      const bool two = o + 1 < h.nops && recs[o + 1].kind == REV_ROT && recs[o + 1].k != r.k;
-      const RevRec &r2 = two ? recs[o + 1] : r;
-      const T *mm = rot + ((uint64_t)r.rslot * Bp + b) * 4;
-      const T *mm2 = rot + ((uint64_t)r2.rslot * Bp + b) * 4;
-      const T m[4] = {mm[0], mm[1], mm[2], mm[3]};
-      const T n2[4] = {mm2[0], mm2[1], mm2[2], mm2[3]};
+      const uint32_t k1 = r.k & 255u, k2 = (r.k >> 8) & 255u;
+      const uint32_t row1 = r.rows & 255u, slot1 = (r.rows >> 16) & 255u;
+      const T c1 = cs[row1];
+      const uint32_t f1 = __builtin_amdgcn_readfirstlane(form[row1]);
       double acc = 0.0, acc2 = 0.0;
-      if (two) {
-        const uint32_t b1 = 1u << r.k, b2 = 1u << r2.k;
-        const int klo = r.k < r2.k ? (int)r.k : (int)r2.k;
-        const int khi = r.k < r2.k ? (int)r2.k : (int)r.k;
+      if ((r.k >> 18) & 1u) {
+        const uint32_t row2 = (r.rows >> 8) & 255u;
+        const T c2 = cs[row2];
+        const uint32_t f2 = __builtin_amdgcn_readfirstlane(form[row2]);
+        const uint32_t b1 = rev_pos(1u << k1), b2 = rev_pos(1u << k2);
+        const uint32_t klo = k1 < k2 ? k1 : k2, khi = k1 < k2 ? k2 : k1;
 #pragma unroll
         for (int qi = 0; qi < (PER + 3) / 4; ++qi) {
-          const uint32_t q = threadIdx.x + (uint32_t)qi * kBlock;
-          if (q >= E / 4) break;
-          const uint32_t j00 = (uint32_t)insert0(insert0(q, klo), khi);
-          const uint32_t j01 = j00 | b1, j10 = j00 | b2, j11 = j00 | b1 | b2;
+          const uint32_t q = tid + (uint32_t)qi * kBlock;
+          if (PER < 4 && q >= E / 4) break;
+          const uint32_t j00 = rev_pos(insert0_32(insert0_32(q, klo), khi));
+          const uint32_t j01 = j00 ^ b1, j10 = j00 ^ b2, j11 = j01 ^ b2;
           T x00 = ps[j00], x01 = ps[j01], x10 = ps[j10], x11 = ps[j11];
           T l00 = ls[j00], l01 = ls[j01], l10 = ls[j10], l11 = ls[j11];
-          rot_reverse_pair<R>(x00, x01, l00, l01, r.axis, m, acc);
-          rot_reverse_pair<R>(x10, x11, l10, l11, r.axis, m, acc);
-          rot_reverse_pair<R>(x00, x10, l00, l10, r2.axis, n2, acc2);
-          rot_reverse_pair<R>(x01, x11, l01, l11, r2.axis, n2, acc2);
+          rot_form(f1, [&](auto kx, auto ksw) {
+            rot_pair<R, decltype(kx)::value, decltype(ksw)::value>(x00, x01, l00, l01, c1, acc);
+            rot_pair<R, decltype(kx)::value, decltype(ksw)::value>(x10, x11, l10, l11, c1, acc);
+          });
+          rot_form(f2, [&](auto kx, auto ksw) {
+            rot_pair<R, decltype(kx)::value, decltype(ksw)::value>(x00, x10, l00, l10, c2, acc2);
+            rot_pair<R, decltype(kx)::value, decltype(ksw)::value>(x01, x11, l01, l11, c2, acc2);
+          });
           ps[j00] = x00;
           ps[j01] = x01;
           ps[j10] = x10;
@@ -464,55 +684,105 @@ __global__ __launch_bounds__(kBlock) void k_reverse_tile(typename AV2<R>::T *__r
           ls[j10] = l10;
           ls[j11] = l11;
         }
+        // (sums of the second rotation are off by the first one's factor too)
+        row_add(sums, slot1, acc);
+        row_add(sums, slot1 + 1, acc2);
       } else {
-        const uint32_t bk = 1u << r.k;
+        const uint32_t bk = rev_pos(1u << k1);
 #pragma unroll
         for (int pi = 0; pi < (PER + 1) / 2; ++pi) {
-          const uint32_t p = threadIdx.x + (uint32_t)pi * kBlock;
-          if (p >= E / 2) break;
-          const uint32_t j0 = (uint32_t)insert0(p, (int)r.k), j1 = j0 | bk;
-          T x0 = ps[j0], x1 = ps[j1], l0 = ls[j0], l1 = ls[j1];
-          rot_reverse_pair<R>(x0, x1, l0, l1, r.axis, m, acc);
+          const uint32_t p = tid + (uint32_t)pi * kBlock;
+          if (PER < 2 && p >= E / 2) break;
+          const uint32_t j0 = rev_pos(insert0_32(p, k1)), j1 = j0 ^ bk;
+          T x0 = ps[j0], x1v = ps[j1], l0 = ls[j0], l1 = ls[j1];
+          rot_form(f1, [&](auto kx, auto ksw) {
+            rot_pair<R, decltype(kx)::value, decltype(ksw)::value>(x0, x1v, l0, l1, c1, acc);
+          });
           ps[j0] = x0;
-          ps[j1] = x1;
+          ps[j1] = x1v;
           ls[j0] = l0;
           ls[j1] = l1;
         }
+        row_add(sums, slot1, acc);
       }
-      acc = wave_sum(acc);
-      double *rb = red[r.out & 3u];
-      double *rb2 = red[r2.out & 3u];
-      if ((threadIdx.x & 63u) == 0) rb[threadIdx.x >> 6] = acc;
-      if (two) {
-        acc2 = wave_sum(acc2);
-        if ((threadIdx.x & 63u) == 0) rb2[threadIdx.x >> 6] = acc2;
-      }
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        double t = 0.0, t2 = 0.0;
-        for (int w = 0; w < kBlock / 64; ++w) {
-          t += rb[w];
-          t2 += rb2[w];
-        }
-        part[(uint64_t)r.out * ntiles + tile] = t;
-        if (two) part[(uint64_t)r2.out * ntiles + tile] = t2;
-      }
-      if (two) ++o;
-    } else if (r.kind == REV_PHASE || r.kind == REV_DIAG) {
-      // a run of consecutive phase and diagonal records: one LDS pass, each
-      // amplitude multiplied by every factor whose pattern it meets
-      uint32_t e = o + 1;
-      while (e < h.nops && (recs[e].kind == REV_PHASE || recs[e].kind == REV_DIAG)) ++e;
+    } else if (r.kind == REV_U1) {
+      const QS_CONST RevRec &d = recs[r.rows];
+      if ((base & d.umask) == d.uval) {  // the same for the whole workgroup
+        const QS_CONST R *v = vals + d.moff;  // row-major 2x2 of the inverse gate
+        const uint32_t bk = rev_pos(1u << d.k);
 #pragma unroll
-      for (int ji = 0; ji < PER; ++ji) {
-        const uint32_t j = threadIdx.x + (uint32_t)ji * kBlock;
-        if (j >= E) break;
-        T x = ps[j], l = ls[j];
-        for (uint32_t t = o; t < e; ++t) {
-          const RevRec &d = recs[t];
-          if ((base & d.umask) != d.uval || (j & (uint32_t)d.lmask) != (uint32_t)d.lval) continue;
+        for (int pi = 0; pi < (PER + 1) / 2; ++pi) {
+          const uint32_t p = tid + (uint32_t)pi * kBlock;
+          if (p >= E / 2) break;
+          const uint32_t l0 = insert0_32(p, d.k);
+          if ((l0 & d.lmask) != d.lval) continue;
+          const uint32_t j0 = rev_pos(l0), j1 = j0 ^ bk;
+          T z[2][2] = {{ps[j0], ps[j1]}, {ls[j0], ls[j1]}};
+          for (int s = 0; s < 2; ++s) {
+            const T x0 = z[s][0], x1 = z[s][1];
+            T y0, y1;
+            y0.x = v[0] * x0.x - v[1] * x0.y + v[2] * x1.x - v[3] * x1.y;
+            y0.y = v[0] * x0.y + v[1] * x0.x + v[2] * x1.y + v[3] * x1.x;
+            y1.x = v[4] * x0.x - v[5] * x0.y + v[6] * x1.x - v[7] * x1.y;
+            y1.y = v[4] * x0.y + v[5] * x0.x + v[6] * x1.y + v[7] * x1.x;
+            z[s][0] = y0;
+            z[s][1] = y1;
+          }
+          ps[j0] = z[0][0];
+          ps[j1] = z[0][1];
+          ls[j0] = z[1][0];
+          ls[j1] = z[1][1];
+        }
+      }
+    } else if constexpr (kExact) {
+      // a diagonal pass in complex64: the records one by one, on the thread's
+      // amplitudes in registers; the phases of -1 (exact, in any order) first
+      const QS_CONST RevDiag &g = diags[r.rows];
+      T x[PER], l[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        x[i] = active ? ps[tpos + (uint32_t)i * kBlock] : T{0, 0};
+        l[i] = active ? ls[tpos + (uint32_t)i * kBlock] : T{0, 0};
+      }
+      if (g.sign != ~0u) {
+        const uint32_t *st = tab + g.sign + (tid >> 5);
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+          if (active && ((st[i * (kBlock / 32)] >> (tid & 31u)) & 1u)) {
+            x[i].x = -x[i].x;
+            x[i].y = -x[i].y;
+            l[i].x = -l[i].x;
+            l[i].y = -l[i].y;
+          }
+      }
+      const uint32_t e = g.first + g.count;
+      for (uint32_t t = g.first; t < e; ++t) {
+        const QS_CONST RevRec &d = recs[t];
+        if (d.kind == REV_RZ) {
+          const T v = cs[d.out];
+          const bool tbit =
+              d.k == kRevNone ? (bool)((base >> d.a0) & 1ull) : (bool)((tid >> (d.k & 7u)) & 1u);
+          double acc = 0.0;
+#pragma unroll
+          for (int i = 0; i < PER; ++i) {
+            const bool bit = d.k >= 8 && d.k != kRevNone ? (bool)((i >> (d.k - 8)) & 1) : tbit;
+            const double w = (double)l[i].x * x[i].y - (double)l[i].y * x[i].x;
+            acc += bit ? -w : w;
+            x[i] = rz_reverse_f(x[i], v, bit);
+            l[i] = rz_reverse_f(l[i], v, bit);
+          }
+          row_add(sums, d.slot, acc);
+          continue;
+        }
+        if ((base & d.umask) != d.uval) continue;  // the same for the whole workgroup
+        const bool on = (tid & (d.lmask & 255u)) == (d.lval & 255u);
+        const uint32_t im = d.lmask >> 8, iv = d.lval >> 8;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+          if (!on || ((uint32_t)i & im) != iv) continue;
           uint32_t vo = d.moff;
           if (d.kind == REV_DIAG) {
+            const uint32_t j = tid + (uint32_t)i * kBlock;
             const uint32_t i0 =
                 d.a0 >= 0 ? (j >> d.a0) & 1u : (uint32_t)((base >> (-1 - d.a0)) & 1ull);
             const uint32_t i1 =
@@ -520,81 +790,288 @@ __global__ __launch_bounds__(kBlock) void k_reverse_tile(typename AV2<R>::T *__r
                            : (d.a1 >= 0 ? (j >> d.a1) & 1u : (uint32_t)((base >> (-1 - d.a1)) & 1ull));
             vo += 2u * (i0 + 2u * i1);
           }
-          const R vr = vals[vo], vi = vals[vo + 1];
+          const R *vg = (const R *)vals + vo;
+          const R vr = vg[0], vi = vg[1];
+          T y, k;
+          y.x = fmaf(vr, x[i].x, -__fmul_rn(vi, x[i].y));
+          y.y = fmaf(vr, x[i].y, __fmul_rn(vi, x[i].x));
+          k.x = fmaf(vr, l[i].x, -__fmul_rn(vi, l[i].y));
+          k.y = fmaf(vr, l[i].y, __fmul_rn(vi, l[i].x));
+          x[i] = y;
+          l[i] = k;
+        }
+      }
+      if (active) {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+          ps[tpos + (uint32_t)i * kBlock] = x[i];
+          ls[tpos + (uint32_t)i * kBlock] = l[i];
+        }
+      }
+    } else {
+      // a diagonal pass: the factor of each of this thread's amplitudes as the
+      // thread's part (tr, ti) times that of i (fr, fi)
+      const QS_CONST RevDiag &g = diags[r.rows];
+      double tr = 1.0, ti = 0.0, fr[PER], fi[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        fr[i] = 1.0;
+        fi[i] = 0.0;
+      }
+      auto turn = [](double &vr, double &vi, double c, double sv) {
+        const double nr = vr * c - vi * sv, ni = vr * sv + vi * c;
+        vr = nr;
+        vi = ni;
+      };
+      const bool zsums = g.nrz + g.noff != 0;
+      uint32_t lane_row = kRevNone;
+      if (zsums) lane_row = reinterpret_cast<const uint8_t *>(tab + g.lane_row)[lane];
+      if (g.sign != ~0u) {
+        const uint32_t *st = tab + g.sign + (tid >> 5);
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+          if (active && ((st[i * (kBlock / 32)] >> (tid & 31u)) & 1u)) fr[i] = -1.0;
+      }
+      const uint32_t noff = g.noff;
+      uint32_t orow = 0;
+      bool oneg = false;
+      if (noff) {
+        // Z rotations off the tile: lane l (and l + 16, ...) takes entry l,
+        // the product over 16 lanes by exchanges
+        double c = 1.0, s = 0.0;
+        const uint32_t l = (uint32_t)lane & 15u;
+        if (l < noff) {
+          const uint32_t en = tab[g.o0 + l];
+          orow = en & 255u;
+          oneg = (base >> (en >> 8)) & 1ull;
+          const T v = cs[orow];
+          c = v.x;
+          s = oneg ? -(double)v.y : (double)v.y;
+        }
+        auto mul = [&](double oc, double os) { turn(c, s, oc, os); };
+        mul(lane_x<0>(c), lane_x<0>(s));
+        mul(lane_x<1>(c), lane_x<1>(s));
+        if (noff > 4) {
+          mul(lane_x<2>(c), lane_x<2>(s));
+          mul(lane_x<3>(c), lane_x<3>(s));
+          tr = c;
+          ti = s;
+        } else {
+          // entries 0..3 lie in the first quad of every 16 lanes
+          tr = __shfl(c, lane & 48);
+          ti = __shfl(s, lane & 48);
+        }
+      }
+      if (g.nrz) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          if (g.rz[k] == kRevNone) continue;
+          const T v = cs[g.rz[k]];
+          turn(tr, ti, v.x, ((tid >> k) & 1u) ? -(double)v.y : (double)v.y);
+        }
+#pragma unroll
+        for (int k = 0; k < PB; ++k) {
+          if (g.rz[8 + k] == kRevNone) continue;
+          const T v = cs[g.rz[8 + k]];
+#pragma unroll
+          for (int i = 0; i < PER; ++i)
+            turn(fr[i], fi[i], v.x, ((i >> k) & 1) ? -(double)v.y : (double)v.y);
+        }
+      }
+      const uint32_t e = g.first + g.count;
+      uint32_t nmore = 0;  // Z rotations among the records
+      for (uint32_t t = g.first; t < e; ++t) {
+        const QS_CONST RevRec &d = recs[t];
+        if (d.kind == REV_RZ) {
+          ++nmore;
+          const T v = cs[d.out];
+          if (d.k >= 8 && d.k != kRevNone) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+              turn(fr[i], fi[i], v.x, ((i >> (d.k - 8)) & 1) ? -(double)v.y : (double)v.y);
+          } else {
+            const bool bit =
+                d.k == kRevNone ? (bool)((base >> d.a0) & 1ull) : (bool)((tid >> d.k) & 1u);
+            turn(tr, ti, v.x, bit ? -(double)v.y : (double)v.y);
+          }
+          continue;
+        }
+        if ((base & d.umask) != d.uval) continue;  // the same for the whole workgroup
+        const bool on = (tid & (d.lmask & 255u)) == (d.lval & 255u);
+        const uint32_t im = d.lmask >> 8, iv = d.lval >> 8;
+        if (d.kind == REV_PHASE) {
+          const double pr = vals[d.moff], pi = vals[d.moff + 1];
+          const double vr = on ? pr : 1.0, vi = on ? pi : 0.0;
+          if (im == 0) {
+            turn(tr, ti, vr, vi);
+          } else {
+#pragma unroll
+            for (int i = 0; i < PER; ++i)
+              if (((uint32_t)i & im) == iv) turn(fr[i], fi[i], vr, vi);
+          }
+        } else {
+#pragma unroll
+          for (int i = 0; i < PER; ++i) {
+            if (((uint32_t)i & im) != iv) continue;
+            const uint32_t j = tid + (uint32_t)i * kBlock;
+            const uint32_t i0 =
+                d.a0 >= 0 ? (j >> d.a0) & 1u : (uint32_t)((base >> (-1 - d.a0)) & 1ull);
+            const uint32_t i1 =
+                d.axis < 2 ? 0u
+                           : (d.a1 >= 0 ? (j >> d.a1) & 1u : (uint32_t)((base >> (-1 - d.a1)) & 1ull));
+            const R *vg = (const R *)(vals + d.moff) + 2u * (i0 + 2u * i1);
+            const double vr = on ? (double)vg[0] : 1.0, vi = on ? (double)vg[1] : 0.0;
+            turn(fr[i], fi[i], vr, vi);
+          }
+        }
+      }
+      double w[PER];
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        w[i] = 0.0;
+        if (active) {
+          const uint32_t j = tpos + (uint32_t)i * kBlock;
+          const T x = ps[j], l = ls[j];
+          w[i] = (double)l.x * x.y - (double)l.y * x.x;
+          turn(fr[i], fi[i], tr, ti);
+          const R vr = (R)fr[i], vi = (R)fi[i];
           T y, k;
           y.x = vr * x.x - vi * x.y;
           y.y = vr * x.y + vi * x.x;
           k.x = vr * l.x - vi * l.y;
           k.y = vr * l.y + vi * l.x;
-          x = y;
-          l = k;
+          ps[j] = y;
+          ls[j] = k;
         }
-        ps[j] = x;
-        ls[j] = l;
       }
-      __syncthreads();
-      o = e - 1;
-    } else if (r.kind == REV_U1) {
-      if ((base & r.umask) != r.uval) continue;  // the same for the whole workgroup
-      const R *v = vals + r.moff;  // row-major 2x2 of the inverse gate
-      const uint32_t bk = 1u << r.k;
+      if (zsums || nmore) {
+        // total and the sums signed by each bit of i over this thread, then
+        // over the wave
+        double tot = 0.0, di[PB > 0 ? PB : 1] = {};
 #pragma unroll
-      for (int pi = 0; pi < (PER + 1) / 2; ++pi) {
-        const uint32_t p = threadIdx.x + (uint32_t)pi * kBlock;
-        if (p >= E / 2) break;
-        const uint32_t j0 = (uint32_t)insert0(p, (int)r.k), j1 = j0 | bk;
-        if ((j0 & (uint32_t)r.lmask) != (uint32_t)r.lval) continue;
-        T z[2][2] = {{ps[j0], ps[j1]}, {ls[j0], ls[j1]}};
-        for (int s = 0; s < 2; ++s) {
-          const T x0 = z[s][0], x1 = z[s][1];
-          T y0, y1;
-          y0.x = v[0] * x0.x - v[1] * x0.y + v[2] * x1.x - v[3] * x1.y;
-          y0.y = v[0] * x0.y + v[1] * x0.x + v[2] * x1.y + v[3] * x1.x;
-          y1.x = v[4] * x0.x - v[5] * x0.y + v[6] * x1.x - v[7] * x1.y;
-          y1.y = v[4] * x0.y + v[5] * x0.x + v[6] * x1.y + v[7] * x1.x;
-          z[s][0] = y0;
-          z[s][1] = y1;
+        for (int i = 0; i < PER; ++i) {
+          tot += w[i];
+#pragma unroll
+          for (int k = 0; k < PB; ++k) di[k] += ((i >> k) & 1) ? -w[i] : w[i];
         }
-        ps[j0] = z[0][0];
-        ps[j1] = z[0][1];
-        ls[j0] = z[1][0];
-        ls[j1] = z[1][1];
+        tot = wave_signed(tot);
+        // the total of di[k] on lane 16 k
+        double z = 0.0;
+        if constexpr (PB > 0) {
+#pragma unroll
+          for (int k = 0; k < PB; ++k)
+            z = __builtin_amdgcn_mfma_f64_4x4x4f64((tid & 3u) == (uint32_t)k ? 1.0 : 0.0, di[k], z,
+                                                   0, 0, 0);
+          z += lane_x<0>(z);
+          z += lane_x<1>(z);
+          z += lane_x<2>(z);
+          z += lane_x<3>(z);
+        }
+        if (lane_row != kRevNone) rows[lane_row][wave] = tot;
+        const double t6 = (wave & 1) ? -tot : tot, t7 = (wave & 2) ? -tot : tot;
+        if (g.nrz) {
+          if (lane == 0) {
+            if (g.rz[6] != kRevNone) rows[g.rz[6]][wave] = t6;
+            if (g.rz[7] != kRevNone) rows[g.rz[7]][wave] = t7;
+          }
+#pragma unroll
+          for (int k = 0; k < PB; ++k)
+            if (lane == 16 * k && g.rz[8 + k] != kRevNone) rows[g.rz[8 + k]][wave] = z;
+        }
+        if (noff) {
+          const double t0 = __shfl(tot, 0);
+          if ((uint32_t)lane < noff) rows[orow][wave] = oneg ? -t0 : t0;
+        }
+        if (nmore) {
+          for (uint32_t t = g.first; t < e; ++t) {
+            const QS_CONST RevRec &d = recs[t];
+            if (d.kind != REV_RZ) continue;
+            if (d.k == kRevNone) {
+              if (lane == 0) rows[d.out][wave] = ((base >> d.a0) & 1ull) ? -tot : tot;
+            } else if (d.k >= 8) {
+              if (lane == 16 * (int)(d.k - 8)) rows[d.out][wave] = z;
+            } else if (d.k >= 6) {
+              if (lane == 0) rows[d.out][wave] = d.k == 6 ? t6 : t7;
+            } else if (lane == (1 << d.k)) {
+              rows[d.out][wave] = tot;
+            }
+          }
+        }
       }
-      __syncthreads();
     }
+    __syncthreads();
   }
+  // row i of an accumulator is on the lanes 16 i .. 16 i + 15
+#pragma unroll
+  for (uint32_t g = 0; g < kRevMaxSlots / 4; ++g) {
+    if (4 * g >= h.nslot) break;
+    double t = sums.d[g];
+    t += lane_x<0>(t);
+    t += lane_x<1>(t);
+    t += lane_x<2>(t);
+    t += lane_x<3>(t);
+    const uint32_t slot = 4 * g + ((uint32_t)lane >> 4);
+    if ((lane & 15) == 0 && slot < h.nslot) rows[h.row_of[slot]][wave] = t;
+  }
+  __syncthreads();
   if (active) {
     V *pso = reinterpret_cast<V *>(psi), *lao = reinterpret_cast<V *>(lam);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      pso[ioff[i]] = psl[threadIdx.x + i * kBlock];
-      lao[ioff[i]] = lsl[threadIdx.x + i * kBlock];
+      pso[ioff[i]] = psl[tpos + i * kBlock] * whole;
+      lao[ioff[i]] = lsl[tpos + i * kBlock] * whole;
     }
   }
+  // one row per thread, the workgroup's rows side by side
+  if (tid < h.nrot)
+    part[tile * h.nrot + tid] =
+        (((rows[tid][0] + rows[tid][1]) + rows[tid][2]) + rows[tid][3]) *
+        (kExact ? 1.0 : scale[tab[2 * h.nrot + tid]]);
 }
 
-// grad[b * P + params[row]] += sum of the tiles of state b in row `row` of
-// part (rows in order, so a parameter shared by two rotations of the block
-// is summed without a race).  grid = Bp.
-__global__ __launch_bounds__(kBlock) void k_rev_accum(const double *__restrict__ part,
-                                                      uint32_t nrot, uint64_t ntiles,
-                                                      uint64_t tiles_per_state,
-                                                      const uint32_t *__restrict__ params,
-                                                      double *__restrict__ grad, size_t P) {
-  __shared__ double sh[kBlock];
+// grad[b * P + params[row]] += sum over the tiles of state b of
+// part[tile * nrot + row], in a fixed order.  16 waves share the tiles, a
+// lane per row, so the rows of a tile are read side by side; rows with the
+// same parameter are added in order by the first of them.  grid = batch.
+constexpr int kAccumWaves = 16;
+
+__global__ __launch_bounds__(64 * kAccumWaves) void k_rev_accum(
+    const double *__restrict__ part, uint32_t nrot, uint64_t tiles_per_state,
+    const uint32_t *__restrict__ params, double *__restrict__ grad, size_t P) {
+  __shared__ double sh[kAccumWaves][kRevMaxRows];
   const uint64_t b = blockIdx.x;
-  for (uint32_t row = 0; row < nrot; ++row) {
-    const double *pr = part + (uint64_t)row * ntiles + b * tiles_per_state;
-    double v = 0.0;
-    for (uint64_t i = threadIdx.x; i < tiles_per_state; i += kBlock) v += pr[i];
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-      __syncthreads();
+  const uint32_t row = threadIdx.x & 63, w = threadIdx.x >> 6;
+  double v = 0.0;
+  if (row < nrot) {
+    const double *pr = part + b * tiles_per_state * nrot + row;
+    uint64_t i = w;
+    for (; i + 7 * kAccumWaves < tiles_per_state; i += 8 * kAccumWaves) {
+      double x[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) x[k] = pr[(i + (uint64_t)k * kAccumWaves) * nrot];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v += x[k];
     }
-    if (threadIdx.x == 0) grad[b * P + params[row]] += sh[0];
-    __syncthreads();
+    for (; i < tiles_per_state; i += kAccumWaves) v += pr[i * nrot];
+  }
+  sh[w][row] = v;
+  __syncthreads();
+  if (threadIdx.x < nrot) {
+    double t = 0.0;
+    for (int k = 0; k < kAccumWaves; ++k) t += sh[k][row];
+    sh[0][row] = t;
+  }
+  __syncthreads();
+  if (threadIdx.x < nrot) {
+    const uint32_t p = params[row];
+    bool first = true;
+    for (uint32_t r = 0; r < row; ++r) first = first && params[r] != p;
+    if (first) {
+      double t = 0.0;
+      for (uint32_t r = row; r < nrot; ++r)
+        if (params[r] == p) t += sh[0][r];
+      grad[b * P + p] += t;
+    }
   }
 }
 
@@ -970,6 +1447,12 @@ bool adjoint_fused_reverse() {
   return on;
 }
 
+// Qubits 0 .. low - 1 are on every tile of the reverse blocks: runs of 128
+// bytes.  One qubit more (256-byte runs) measured the same per block (20
+// qubits, batch 64: 24.2 ms backward either way) and leaves one less for the
+// pair targets.
+int reverse_low_bits(int dtype) { return dtype == QS_C128 ? 3 : 4; }
+
 // Tile qubits of the reverse blocks: QS_ADJOINT_TILE, default 10 for
 // complex128 and 11 for complex64 (32 KiB of LDS for psi and lambda).
 int reverse_tile_bits(int dtype) {
@@ -978,10 +1461,63 @@ int reverse_tile_bits(int dtype) {
   return std::max(1, std::min(t, kRevMaxBits));
 }
 
-// The reverse sweep in tiled blocks (k_reverse_tile): operations are taken
-// in reverse order while their pair targets fit the tile; a checkpoint
-// restore, a gate with no tile form (two or more dense target qubits) or a
-// full record list ends a block.
+// An operation of the reverse pass: the qubits its inverse touches off the
+// diagonal (x) and on it (z); its pair target (-1: none, diagonal); whether
+// it has a tile form, and the records and gradient rows that takes.
+struct RevItem {
+  size_t op = 0;
+  uint64_t x = 0, z = 0;
+  int pq = -1;
+  bool tile_form = true;
+  int records = 1, rows = 0, slots = 0;  // slots: of RowSums, in complex64 Z rotations too
+};
+
+RevItem rev_item(const POp &op, size_t index) {
+  RevItem it;
+  it.op = index;
+  if (op.kind == 1) {
+    it.rows = it.slots = 1;
+    if (op.axis == QS_AXIS_Z) {
+      it.z = 1ull << op.target;
+    } else {
+      it.x = 1ull << op.target;
+      it.pq = op.target;
+    }
+    return it;
+  }
+  const qs::Gate &g = op.inv;
+  uint64_t act = 0;
+  for (int j = 0; j < g.na; ++j) act |= 1ull << g.act[j];
+  if (g.kind == qs::Gate::kSparse) {
+    it.z = g.smask;
+    it.records = (int)g.spat.size();
+  } else if (g.kind == qs::Gate::kDiag) {
+    it.z = act | g.cmask;
+    it.tile_form = g.na >= 1 && g.na <= 2;
+  } else if (g.kind == qs::Gate::kDense && g.na == 1) {
+    it.x = act;
+    it.z = g.cmask;
+    it.pq = g.act[0];
+  } else {
+    it.x = act;
+    it.z = g.cmask;
+    it.tile_form = false;
+  }
+  return it;
+}
+
+// The reverse sweep in tiled blocks (k_reverse_tile).  Between two checkpoint
+// restores the operations are taken in reverse order, and a later one moves
+// ahead of earlier ones left for another block where it commutes with each of
+// them (on every shared qubit both act diagonally): its gradient Im
+// <lambda|sigma|psi> is then the same before and after them.  The tile takes
+// the pair targets first come, first served while there is room; diagonal
+// operations and controls need no tile qubit.  A gate with no tile form (two
+// or more dense target qubits) runs on its own once nothing before it is
+// left.  On the layered ansatz a block so reaches into the next layers as far
+// as its tile's light cone: 20 qubits, 10 layers, checkpoints every two, 15
+// blocks (26 in strict order).  Complex64 keeps the strict order, so that
+// every amplitude is rounded as if the operations ran one by one.
 template <typename R>
 int reverse_blocks(qs_adjoint *c) {
   using T = typename AV2<R>::T;
@@ -989,35 +1525,44 @@ int reverse_blocks(qs_adjoint *c) {
   const int n = c->n;
   const size_t Bp = c->Bp, P = c->P;
   const int Tt = std::min(reverse_tile_bits(c->dtype), n);
-  const int low = std::min(Tt, c->dtype == QS_C128 ? 4 : 5);  // 256-byte runs
+  // at least one tile qubit is left for a pair target above the low ones
+  const int low = Tt == n ? Tt : std::min(Tt - 1, reverse_low_bits(c->dtype));
   const uint64_t tiles_per_state = 1ull << (n - Tt);
   const uint64_t ntiles = tiles_per_state * Bp;
-  // rows of partial sums per block: at most 32, within 64 MiB
-  const uint64_t rmax = std::max<uint64_t>(1, std::min<uint64_t>(32, (64ull << 20) / (8 * ntiles)));
-  if (!c->d_rpart) AJ(hipMalloc((void **)&c->d_rpart, rmax * ntiles * sizeof(double)));
+  // rows of partial sums per block: within 64 MiB
+  const int rmax =
+      (int)std::max<uint64_t>(1, std::min<uint64_t>(kRevMaxRows, (64ull << 20) / (8 * ntiles)));
+  if (!c->d_rpart) AJ(hipMalloc((void **)&c->d_rpart, (uint64_t)rmax * ntiles * sizeof(double)));
   if (!c->d_ring) {
     c->ring_cap = 8u << 20;
     AJ(hipMalloc((void **)&c->d_ring, c->ring_cap));
     AJ(hipHostMalloc((void **)&c->h_ring, c->ring_cap));
   }
   const uint64_t lowset = (1ull << low) - 1ull;
-  // the block under construction; qubit fields hold global qubits until
-  // the tile is fixed
-  struct Pend {
-    RevRec r;
-    uint64_t cmask, cval;  // global pattern
-    int q0, q1;            // global target / act qubits
+  constexpr bool strict = std::is_same<R, float>::value;
+  // Whether an operation may run ahead of those that touch bx off the
+  // diagonal and bz on it: complex64 keeps the strict order.
+  bool ahead = false;  // something was left behind
+  auto free_of = [&](const RevItem &it, uint64_t bx, uint64_t bz) {
+    return !(strict && ahead) && !(it.x & (bx | bz)) && !(it.z & bx);
   };
-  std::vector<Pend> pend;
+  std::vector<RevItem> items;  // left, in reverse order
+  std::vector<RevItem> block;
+  std::vector<RevPass> passes;
+  std::vector<RevDiag> diags;
+  std::vector<RevRec> recs;
   std::vector<R> vals;
-  std::vector<uint32_t> params;
-  uint64_t S = lowset;  // tile qubits taken
-  auto put = [&](const qs::cd &v) {
-    vals.push_back((R)v.re);
-    vals.push_back((R)v.im);
-  };
-  auto flush = [&]() -> int {
-    if (pend.empty()) return QS_OK;
+  std::vector<uint32_t> rows, params, row_scale, offs, lane_rows, signs;
+  std::vector<char> blob;
+  const int sign_words = std::max(1, 1 << std::max(0, Tt - 5));
+  // bit j of in_bit[k]: bit k of j (amplitudes j of the tile)
+  std::vector<std::vector<uint32_t>> in_bit((size_t)Tt, std::vector<uint32_t>(sign_words, 0));
+  for (int k = 0; k < Tt; ++k)
+    for (uint32_t j = 0; j < (1u << Tt); ++j)
+      if ((j >> k) & 1u) in_bit[k][j >> 5] |= 1u << (j & 31u);
+
+  // Launch the block's operations on a tile with pair targets S.
+  auto launch = [&](uint64_t S) -> int {
     RevHeader hd{};
     hd.T = (uint32_t)Tt;
     uint64_t full = S;
@@ -1031,69 +1576,279 @@ int reverse_blocks(qs_adjoint *c) {
         loc[q] = t++;
       }
     }
-    std::vector<RevRec> recs;
-    for (const Pend &pd : pend) {
-      RevRec r = pd.r;
-      const uint64_t off = pd.cmask & ~full;
-      r.umask = off;
-      r.uval = pd.cval & off;
-      r.lmask = r.lval = 0;
-      for (uint64_t bits = pd.cmask & full; bits; bits &= bits - 1) {
+    passes.clear();
+    diags.clear();
+    recs.clear();
+    vals.clear();
+    rows.clear();
+    params.clear();
+    row_scale.clear();
+    offs.clear();
+    lane_rows.clear();
+    signs.clear();
+    auto put = [&](const qs::cd &v) {
+      vals.push_back((R)v.re);
+      vals.push_back((R)v.im);
+    };
+    auto pattern = [&](RevRec &r, uint64_t mask, uint64_t val) {
+      r.umask = mask & ~full;
+      r.uval = val & r.umask;
+      for (uint64_t bits = mask & full; bits; bits &= bits - 1) {
         const int q = __builtin_ctzll(bits);
-        r.lmask |= 1ull << loc[q];
-        if ((pd.cval >> q) & 1ull) r.lval |= 1ull << loc[q];
+        r.lmask |= 1u << loc[q];
+        if ((val >> q) & 1ull) r.lval |= 1u << loc[q];
       }
-      if (r.kind == REV_ROT || r.kind == REV_U1) r.k = (uint32_t)loc[pd.q0];
-      if (r.kind == REV_DIAG) {
-        r.a0 = loc[pd.q0] >= 0 ? loc[pd.q0] : -1 - pd.q0;
-        r.a1 = pd.q1 < 0 ? 0 : (loc[pd.q1] >= 0 ? loc[pd.q1] : -1 - pd.q1);
+    };
+    auto new_row = [&](const POp &op) {
+      rows.push_back((uint32_t)op.rot_slot | ((uint32_t)op.axis << 30));
+      params.push_back((uint32_t)op.param);
+      row_scale.push_back(hd.nslot);  // the slots before it
+      return (uint32_t)rows.size() - 1;
+    };
+    // a diagonal operation, into the diagonal pass d (signs: its sign table)
+    auto emit_diag = [&](const RevItem &it, RevDiag &d, std::vector<uint32_t> &sg) {
+      const POp &op = c->circ.ops[it.op];
+      const qs::Gate &g = op.inv;
+      RevRec r{};
+      if (op.kind == 1) {
+        r.out = new_row(op);
+        const int k = loc[op.target];
+        if (strict) {
+          r.kind = REV_RZ;
+          r.k = k >= 0 ? (uint32_t)k : kRevNone;
+          r.a0 = op.target;
+          r.slot = hd.nslot++;
+          hd.row_of[r.slot] = r.out;
+          recs.push_back(r);
+        } else if (k >= 0 && d.rz[k] == kRevNone) {
+          d.rz[k] = r.out;
+          ++d.nrz;
+        } else if (k < 0 && d.noff < (uint32_t)kRevMaxOff) {
+          offs.push_back(r.out | ((uint32_t)op.target << 8));
+          ++d.noff;
+        } else {
+          r.kind = REV_RZ;
+          r.k = k >= 0 ? (uint32_t)k : kRevNone;
+          r.a0 = op.target;
+          recs.push_back(r);
+        }
+      } else if (g.kind == qs::Gate::kSparse) {
+        for (size_t k = 0; k < g.spat.size(); ++k) {
+          if (g.m[k].re == -1.0 && g.m[k].im == 0.0 && (g.smask & ~full) == 0) {
+            if (sg.empty()) sg.assign((size_t)sign_words, 0);
+            for (int w = 0; w < sign_words; ++w) {
+              uint32_t on = ~0u;
+              for (uint64_t bits = g.smask; bits; bits &= bits - 1) {
+                const int q = __builtin_ctzll(bits);
+                const uint32_t m = in_bit[loc[q]][w];
+                on &= ((g.spat[k] >> q) & 1ull) ? m : ~m;
+              }
+              sg[w] ^= on;
+            }
+            continue;
+          }
+          RevRec x = r;
+          x.kind = REV_PHASE;
+          x.moff = (uint32_t)vals.size();
+          put(g.m[k]);
+          pattern(x, g.smask, g.spat[k]);
+          recs.push_back(x);
+        }
+      } else {
+        r.kind = REV_DIAG;
+        r.axis = (uint32_t)g.na;
+        r.moff = (uint32_t)vals.size();
+        for (const qs::cd &v : g.m) put(v);
+        pattern(r, g.cmask, g.cval);
+        r.a0 = loc[g.act[0]] >= 0 ? loc[g.act[0]] : -1 - g.act[0];
+        r.a1 = g.na < 2 ? 0 : (loc[g.act[1]] >= 0 ? loc[g.act[1]] : -1 - g.act[1]);
+        recs.push_back(r);
       }
-      recs.push_back(r);
+    };
+    // passes: by turns every diagonal operation that may come next, and every
+    // X / Y rotation that may (two on different qubits to a pass)
+    while (!block.empty()) {
+      std::vector<RevItem> left;
+      std::vector<uint32_t> sg;
+      uint64_t bx = 0, bz = 0;
+      ahead = false;
+      RevDiag d{};
+      d.o0 = (uint32_t)offs.size();
+      d.first = (uint32_t)recs.size();
+      for (uint32_t &v : d.rz) v = kRevNone;
+      bool any = false;
+      for (const RevItem &it : block) {
+        const bool movable = free_of(it, bx, bz);
+        if (movable && it.pq < 0) {
+          emit_diag(it, d, sg);
+          any = true;
+        } else {
+          bx |= it.x;
+          bz |= it.z;
+          left.push_back(it);
+          ahead = true;
+        }
+      }
+      if (any) {
+        d.count = (uint32_t)recs.size() - d.first;
+        d.lane_row = (uint32_t)lane_rows.size();
+        uint8_t lr[64];
+        std::memset(lr, kRevNone, sizeof lr);
+        for (int k = 0; k < std::min(Tt, 6); ++k) lr[1 << k] = (uint8_t)d.rz[k];
+        lane_rows.resize(lane_rows.size() + 16);
+        std::memcpy(&lane_rows[d.lane_row], lr, sizeof lr);
+        d.sign = sg.empty() ? ~0u : (uint32_t)signs.size();
+        signs.insert(signs.end(), sg.begin(), sg.end());
+        passes.push_back({REV_DIAGS, 0, (uint32_t)diags.size(), 0});
+        diags.push_back(d);
+      }
+      block.swap(left);
+      left.clear();
+      bx = bz = 0;
+      ahead = false;
+      size_t open = ~(size_t)0;  // a rotation pass with room for a second
+      for (const RevItem &it : block) {
+        const bool movable = free_of(it, bx, bz);
+        if (!(movable && it.pq >= 0)) {
+          bx |= it.x;
+          bz |= it.z;
+          left.push_back(it);
+          ahead = true;
+          continue;
+        }
+        const POp &op = c->circ.ops[it.op];
+        const uint32_t k = (uint32_t)loc[it.pq];
+        if (op.kind == 1) {
+          const uint32_t row = new_row(op), slot = hd.nslot++;
+          hd.row_of[slot] = row;
+          const uint32_t is_x = op.axis == QS_AXIS_X;
+          if (open != ~(size_t)0 && (passes[open].k & 255u) != k) {
+            // slots are given in the order of the passes: the second's is the
+            // next after the first's
+            passes[open].k |= (k << 8) | (is_x << 17) | (1u << 18);
+            passes[open].rows |= row << 8;
+            open = ~(size_t)0;
+          } else {
+            open = passes.size();
+            passes.push_back({REV_ROT, k | (is_x << 16), row | (slot << 16), 0});
+          }
+        } else {
+          RevRec r{};
+          r.kind = REV_U1;
+          r.moff = (uint32_t)vals.size();
+          for (const qs::cd &v : op.inv.m) put(v);
+          pattern(r, op.inv.cmask, op.inv.cval);
+          r.k = k;
+          passes.push_back({REV_U1, 0, (uint32_t)recs.size(), 0});
+          recs.push_back(r);
+          open = ~(size_t)0;
+        }
+      }
+      block.swap(left);
     }
-    hd.nops = (uint32_t)recs.size();
-    hd.nrot = (uint32_t)params.size();
-    hd.nvals = (uint32_t)vals.size();
-    std::vector<char> blob(sizeof(RevHeader) + recs.size() * sizeof(RevRec) +
-                           vals.size() * sizeof(R) + params.size() * sizeof(uint32_t) + 16);
+    hd.npass = (uint32_t)passes.size();
+    hd.nrot = (uint32_t)rows.size();
+    hd.ndiag = (uint32_t)diags.size();
+    hd.nrec = (uint32_t)recs.size();
+    const size_t fixed = sizeof(RevHeader) + passes.size() * sizeof(RevPass) +
+                         diags.size() * sizeof(RevDiag) + recs.size() * sizeof(RevRec) +
+                         vals.size() * sizeof(R);
+    hd.tab = (uint32_t)((fixed + 15) / 16 * 4);
+    hd.params = hd.tab + hd.nrot;
+    const uint32_t off_at = 3 * hd.nrot, lane_at = off_at + (uint32_t)offs.size(),
+                   sign_at = lane_at + (uint32_t)lane_rows.size();
+    for (RevDiag &d : diags) {  // offsets from `tab`
+      d.o0 += off_at;
+      d.lane_row += lane_at;
+      if (d.sign != ~0u) d.sign += sign_at;
+    }
+    blob.assign((size_t)(hd.tab + sign_at) * 4 + signs.size() * 4, 0);
     char *w = blob.data();
-    std::memcpy(w, &hd, sizeof hd);
-    w += sizeof hd;
-    std::memcpy(w, recs.data(), recs.size() * sizeof(RevRec));
-    w += recs.size() * sizeof(RevRec);
-    if (!vals.empty()) std::memcpy(w, vals.data(), vals.size() * sizeof(R));
-    w += vals.size() * sizeof(R);
-    const size_t poff = (size_t)(w - blob.data() + 3) & ~(size_t)3;
-    if (!params.empty()) std::memcpy(blob.data() + poff, params.data(), params.size() * 4);
+    auto add = [&](const void *p, size_t bytes) {
+      if (bytes) std::memcpy(w, p, bytes);
+      w += bytes;
+    };
+    add(&hd, sizeof hd);
+    add(passes.data(), passes.size() * sizeof(RevPass));
+    add(diags.data(), diags.size() * sizeof(RevDiag));
+    add(recs.data(), recs.size() * sizeof(RevRec));
+    add(vals.data(), vals.size() * sizeof(R));
+    w = blob.data() + (size_t)hd.tab * 4;
+    add(rows.data(), rows.size() * 4);
+    add(params.data(), params.size() * 4);
+    add(row_scale.data(), row_scale.size() * 4);
+    add(offs.data(), offs.size() * 4);
+    add(lane_rows.data(), lane_rows.size() * 4);
+    add(signs.data(), signs.size() * 4);
     void *d_blob = nullptr;
     AJ(ring_upload(c, blob.data(), blob.size(), &d_blob));
-    const size_t lds = 2 * ((size_t)1 << Tt) * sizeof(T);
+    const size_t lds = 2 * std::max<size_t>((size_t)1 << Tt, kBlock) * sizeof(T);
     auto kern = Tt <= 8 ? k_reverse_tile<R, 1>
                         : (Tt == 9 ? k_reverse_tile<R, 2>
                                    : (Tt == 10 ? k_reverse_tile<R, 4> : k_reverse_tile<R, 8>));
     hipLaunchKernelGGL(kern, dim3((unsigned)ntiles), dim3(kBlock), lds, c->stream, (T *)c->psi,
                        (T *)c->lam, n, (const char *)d_blob, (const T *)c->d_rot, (uint64_t)Bp,
-                       c->d_rpart, ntiles);
+                       c->d_rpart);
     AJ(hipGetLastError());
     ++c->rev_blocks;
     if (!params.empty()) {
-      hipLaunchKernelGGL(k_rev_accum, dim3((unsigned)Bp), dim3(kBlock), 0, c->stream,
-                         (const double *)c->d_rpart, (uint32_t)params.size(), ntiles,
-                         tiles_per_state, (const uint32_t *)((char *)d_blob + poff), c->d_grad,
-                         P);
+      hipLaunchKernelGGL(k_rev_accum, dim3((unsigned)Bp), dim3(64 * kAccumWaves), 0, c->stream,
+                         (const double *)c->d_rpart, (uint32_t)params.size(), tiles_per_state,
+                         (const uint32_t *)d_blob + hd.params, c->d_grad, P);
       AJ(hipGetLastError());
     }
-    pend.clear();
-    vals.clear();
-    params.clear();
-    S = lowset;
     return QS_OK;
   };
-  // pair targets must be tile qubits
-  auto fits = [&](int q) { return ((S >> q) & 1ull) || __builtin_popcountll(S) < Tt; };
+
+  // Run everything in `items` (the operations since the last restore).
+  auto drain = [&]() -> int {
+    std::vector<RevItem> left;
+    while (!items.empty()) {
+      if (!items[0].tile_form) {
+        const size_t ii = items[0].op;
+        const qs::Gate &g = c->circ.ops[ii].inv;
+        const void *tab = (const char *)c->d_gmat + c->gmat_off[2 * ii + 1];
+        AJ(apply_fixed<R>(c, c->psi, g, tab));
+        AJ(apply_fixed<R>(c, c->lam, g, tab));
+        items.erase(items.begin());
+        continue;
+      }
+      block.clear();
+      left.clear();
+      uint64_t S = lowset, bx = 0, bz = 0;
+      ahead = false;
+      int nrec = 0, nrow = 0, nslot = 0;
+      for (size_t i = 0; i < items.size(); ++i) {
+        const RevItem &it = items[i];
+        const uint64_t bq = it.pq >= 0 ? 1ull << it.pq : 0;
+        const bool movable = free_of(it, bx, bz);
+        if (it.tile_form && movable && nrec + it.records <= kRevMaxOps &&
+            nrow + it.rows <= rmax && nslot + (strict || it.pq >= 0 ? it.slots : 0) <= kRevMaxSlots &&
+            __builtin_popcountll(S | bq) <= Tt) {
+          S |= bq;
+          nrec += it.records;
+          nrow += it.rows;
+          nslot += strict || it.pq >= 0 ? it.slots : 0;
+          block.push_back(it);
+        } else {
+          bx |= it.x;
+          bz |= it.z;
+          if (!it.tile_form) bx |= it.z;
+          left.push_back(it);
+          ahead = true;
+        }
+      }
+      items.swap(left);
+      const int rc = launch(S);
+      if (rc != QS_OK) return rc;
+    }
+    return QS_OK;
+  };
+
   int ck = (int)c->ckpt.size() - 1;
   for (size_t ii = c->circ.ops.size(); ii-- > 0;) {
     if (ck >= 0 && c->ckpt_at[ck] == ii + 1) {
-      int rc = flush();
+      int rc = drain();
       if (rc != QS_OK) return rc;
       AJ(hipMemcpyAsync(c->psi, c->ckpt[ck], c->state_bytes(), hipMemcpyDeviceToDevice,
                         c->stream));
@@ -1101,82 +1856,10 @@ int reverse_blocks(qs_adjoint *c) {
       --ck;
     }
     const POp &op = c->circ.ops[ii];
-    const qs::Gate &g = op.inv;
-    int need = 1;  // records this operation adds
-    bool tile_form = true;
-    int pq = -1;  // its pair target
-    if (op.kind == 1) {
-      pq = op.target;
-    } else if (g.kind == qs::Gate::kIdentity) {
-      continue;
-    } else if (g.kind == qs::Gate::kSparse) {
-      need = (int)g.spat.size();
-    } else if (g.kind == qs::Gate::kDiag) {
-      tile_form = g.na >= 1 && g.na <= 2;
-    } else if (g.kind == qs::Gate::kDense && g.na == 1) {
-      pq = g.act[0];
-    } else {
-      tile_form = false;
-    }
-    if (!tile_form) {
-      int rc = flush();
-      if (rc != QS_OK) return rc;
-      const void *tab = (const char *)c->d_gmat + c->gmat_off[2 * ii + 1];
-      AJ(apply_fixed<R>(c, c->psi, g, tab));
-      AJ(apply_fixed<R>(c, c->lam, g, tab));
-      continue;
-    }
-    if ((int)pend.size() + need > kRevMaxOps || (pq >= 0 && !fits(pq)) ||
-        (op.kind == 1 && params.size() >= rmax)) {
-      int rc = flush();
-      if (rc != QS_OK) return rc;
-    }
-    if (pq >= 0) S |= 1ull << pq;
-    if (op.kind == 1) {
-      Pend pd{};
-      pd.r.kind = REV_ROT;
-      pd.r.axis = (uint32_t)op.axis;
-      pd.r.rslot = (uint32_t)op.rot_slot;
-      pd.r.out = (uint32_t)params.size();
-      pd.q0 = op.target;
-      pd.q1 = -1;
-      params.push_back((uint32_t)op.param);
-      pend.push_back(pd);
-    } else if (g.kind == qs::Gate::kSparse) {
-      for (size_t k = 0; k < g.spat.size(); ++k) {
-        Pend pd{};
-        pd.r.kind = REV_PHASE;
-        pd.r.moff = (uint32_t)vals.size();
-        put(g.m[k]);
-        pd.cmask = g.smask;
-        pd.cval = g.spat[k];
-        pd.q0 = pd.q1 = -1;
-        pend.push_back(pd);
-      }
-    } else if (g.kind == qs::Gate::kDiag) {
-      Pend pd{};
-      pd.r.kind = REV_DIAG;
-      pd.r.axis = (uint32_t)g.na;
-      pd.r.moff = (uint32_t)vals.size();
-      for (const qs::cd &v : g.m) put(v);
-      pd.cmask = g.cmask;
-      pd.cval = g.cval;
-      pd.q0 = g.act[0];
-      pd.q1 = g.na > 1 ? g.act[1] : -1;
-      pend.push_back(pd);
-    } else {
-      Pend pd{};
-      pd.r.kind = REV_U1;
-      pd.r.moff = (uint32_t)vals.size();
-      for (const qs::cd &v : g.m) put(v);
-      pd.cmask = g.cmask;
-      pd.cval = g.cval;
-      pd.q0 = g.act[0];
-      pd.q1 = -1;
-      pend.push_back(pd);
-    }
+    if (op.kind == 0 && op.inv.kind == qs::Gate::kIdentity) continue;
+    items.push_back(rev_item(op, ii));
   }
-  return flush();
+  return drain();
 }
 
 template <typename R>
