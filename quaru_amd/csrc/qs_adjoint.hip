@@ -512,6 +512,8 @@ __device__ __forceinline__ double wave_signed(double v) {
 // spread over the banks.  Linear over XOR: pos(j ^ b) = pos(j) ^ pos(b).
 __device__ __forceinline__ uint32_t rev_pos(uint32_t j) { return j ^ ((j >> 3) & 7u); }
 
+// With `hdiag` lambda is not read but begins as hdiag . psi.
+//
 // One workgroup per tile (grid = ntiles); dynamic LDS 2 x 2^T amplitudes (at
 // least 256); PER = max(1, 2^T / 256).  part[tile * nrot + row] = the tile's
 // share of the gradient of the rotation with that row.
@@ -533,7 +535,8 @@ __attribute__((amdgpu_waves_per_eu(PER < 8 ? 4 : (sizeof(R) == 8 ? 2 : 3)))) voi
                                                          typename AV2<R>::T *__restrict__ lam,
                                                          int n, const char *__restrict__ blob_g,
                                                          const typename AV2<R>::T *__restrict__ rot,
-                                                         uint64_t Bp, double *__restrict__ part) {
+                                                         uint64_t Bp, double *__restrict__ part,
+                                                         const double *__restrict__ hdiag) {
   using T = typename AV2<R>::T;
   constexpr int PB = PER == 1 ? 0 : (PER == 2 ? 1 : (PER == 4 ? 2 : 3));  // bits of i
   constexpr bool kExact = sizeof(R) == 4;  // complex64: see rot_reverse_pair_f
@@ -593,7 +596,16 @@ __attribute__((amdgpu_waves_per_eu(PER < 8 ? 4 : (sizeof(R) == 8 ? 2 : 3)))) voi
 #pragma unroll
       for (int i = 0; i < PER; ++i) {
         xv[i] = psv[ioff[i]];
-        lv[i] = lav[ioff[i]];
+        if (!hdiag) lv[i] = lav[ioff[i]];
+      }
+      if (hdiag) {
+        // the first block: lambda = h psi (k_apply_h)
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+          const double hv = hdiag[ioff[i] & ((1ull << n) - 1ull)];
+          lv[i].x = (R)((double)xv[i].x * hv);
+          lv[i].y = (R)((double)xv[i].y * hv);
+        }
       }
     }
     // a thread per rotation fetches its angle's cosine and sine: m[0] = c (X,
@@ -1546,6 +1558,7 @@ int reverse_blocks(qs_adjoint *c) {
   auto free_of = [&](const RevItem &it, uint64_t bx, uint64_t bz) {
     return !(strict && ahead) && !(it.x & (bx | bz)) && !(it.z & bx);
   };
+  bool made = false;  // whether lambda = h psi is in memory
   std::vector<RevItem> items;  // left, in reverse order
   std::vector<RevItem> block;
   std::vector<RevPass> passes;
@@ -1788,8 +1801,9 @@ int reverse_blocks(qs_adjoint *c) {
                                    : (Tt == 10 ? k_reverse_tile<R, 4> : k_reverse_tile<R, 8>));
     hipLaunchKernelGGL(kern, dim3((unsigned)ntiles), dim3(kBlock), lds, c->stream, (T *)c->psi,
                        (T *)c->lam, n, (const char *)d_blob, (const T *)c->d_rot, (uint64_t)Bp,
-                       c->d_rpart);
+                       c->d_rpart, made ? nullptr : c->d_h);
     AJ(hipGetLastError());
+    made = true;
     ++c->rev_blocks;
     if (!params.empty()) {
       hipLaunchKernelGGL(k_rev_accum, dim3((unsigned)Bp), dim3(64 * kAccumWaves), 0, c->stream,
@@ -1797,6 +1811,17 @@ int reverse_blocks(qs_adjoint *c) {
                          (const uint32_t *)d_blob + hd.params, c->d_grad, P);
       AJ(hipGetLastError());
     }
+    return QS_OK;
+  };
+
+  // lambda = h psi for what is not the first block
+  auto make = [&]() -> int {
+    if (made) return QS_OK;
+    made = true;
+    const uint64_t total = (uint64_t)Bp << n;
+    hipLaunchKernelGGL(k_apply_h<R>, dim3(grid_of(total, kBlock * 4)), dim3(kBlock), 0, c->stream,
+                       (T *)c->lam, (const T *)c->psi, n, c->d_h, total);
+    AJ(hipGetLastError());
     return QS_OK;
   };
 
@@ -1808,6 +1833,8 @@ int reverse_blocks(qs_adjoint *c) {
         const size_t ii = items[0].op;
         const qs::Gate &g = c->circ.ops[ii].inv;
         const void *tab = (const char *)c->d_gmat + c->gmat_off[2 * ii + 1];
+        const int rc = make();
+        if (rc != QS_OK) return rc;
         AJ(apply_fixed<R>(c, c->psi, g, tab));
         AJ(apply_fixed<R>(c, c->lam, g, tab));
         items.erase(items.begin());
@@ -1849,9 +1876,9 @@ int reverse_blocks(qs_adjoint *c) {
   for (size_t ii = c->circ.ops.size(); ii-- > 0;) {
     if (ck >= 0 && c->ckpt_at[ck] == ii + 1) {
       int rc = drain();
+      if (rc == QS_OK) rc = make();
       if (rc != QS_OK) return rc;
-      AJ(hipMemcpyAsync(c->psi, c->ckpt[ck], c->state_bytes(), hipMemcpyDeviceToDevice,
-                        c->stream));
+      std::swap(c->psi, c->ckpt[ck]);  // the uncomputed state is not needed any more
       ++c->rev_restores;
       --ck;
     }
@@ -1873,9 +1900,12 @@ int backward_t(qs_adjoint *c, double *grads) {
   if (!c->d_grad) AJ(hipMalloc((void **)&c->d_grad, Bp * std::max<size_t>(P, 1) * sizeof(double)));
   hipLaunchKernelGGL(k_fill_zero, dim3(grid_of(Bp * P, kBlock)), dim3(kBlock), 0, c->stream,
                      c->d_grad, (uint64_t)(Bp * P));
-  hipLaunchKernelGGL(k_apply_h<R>, dim3(grid_of(total, kBlock * 4)), dim3(kBlock), 0, c->stream,
-                     (T *)c->lam, (const T *)c->psi, n, c->d_h, total);
   AJ(hipGetLastError());
+  if (!adjoint_fused_reverse()) {  // the tiled blocks make lambda themselves
+    hipLaunchKernelGGL(k_apply_h<R>, dim3(grid_of(total, kBlock * 4)), dim3(kBlock), 0, c->stream,
+                       (T *)c->lam, (const T *)c->psi, n, c->d_h, total);
+    AJ(hipGetLastError());
+  }
   const uint64_t pps = 1ull << (n - 1);
   const uint64_t per = std::min<uint64_t>(pps, 1024);
   const int nblk = (int)((pps + per - 1) / per);
@@ -1887,8 +1917,7 @@ int backward_t(qs_adjoint *c, double *grads) {
   }
   for (size_t ii = adjoint_fused_reverse() ? 0 : c->circ.ops.size(); ii-- > 0;) {
     if (ck >= 0 && c->ckpt_at[ck] == ii + 1) {
-      AJ(hipMemcpyAsync(c->psi, c->ckpt[ck], c->state_bytes(), hipMemcpyDeviceToDevice,
-                        c->stream));
+      std::swap(c->psi, c->ckpt[ck]);
       --ck;
     }
     const POp &op = c->circ.ops[ii];

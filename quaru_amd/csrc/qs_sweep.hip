@@ -42,7 +42,13 @@ static_assert(kFirstLaneSlot == (int)kLaneSlot && kFirstWaveSlot == (int)kWaveSl
 
 constexpr int kMaxOps = 512;     // op records per sweep
 constexpr int kWindow = 384;     // look-ahead over unscheduled gates
-constexpr size_t kMaxBlobBytes = 64 * 1024;
+// Descriptor bytes per sweep.  A batched rotation's matrices alone take 4 KiB
+// at complex128 and batch 64, so 64 KiB held a sweep of the adjoint forward
+// pass to 16 rotations (40 sweeps for the 20-qubit, 10-layer ansatz, 15 with
+// 512 KiB: 15.1 ms of sweeps and 6.9 ms).  Complex64 keeps the smaller bound,
+// which fixes which operations merge and so how its results round.
+template <typename R>
+constexpr size_t kMaxBlobBytes = sizeof(R) == 8 ? 512 * 1024 : 64 * 1024;
 
 inline int popc(uint64_t x) { return __builtin_popcountll(x); }
 
@@ -385,7 +391,7 @@ hipError_t execute_t(SweepRunner &run, const std::vector<Gate> &gates, uint64_t 
         const bool movable = !(gx[i] & (bx | bz)) && !(gz[i] & bx);
         const bool room =
             (int)pl.gates.size() < max_gates && nops + op_count(g) <= kMaxOps &&
-            blob_bytes<R>(nops + op_count(g), npool + pool_count(g)) <= kMaxBlobBytes;
+            blob_bytes<R>(nops + op_count(g), npool + pool_count(g)) <= kMaxBlobBytes<R>;
         bool ok = movable && room && sweepable(g, lowb);
         if (ok) ok = fixed ? fits_set(g, S, ts, pl) : try_place(g, ts, pl);
         if (ok) {
