@@ -1110,7 +1110,19 @@ struct qs_adjoint {
   size_t B = 0, Bp = 1, P = 0;
   int dtype = QS_C128;
   size_t checkpoint_every = 0;
+  qs::Workspace *ws = nullptr;  // owns the stream and the descriptor ring
   hipStream_t stream = nullptr;
+  // every buffer below comes from take(), which keeps its size for free_ctx
+  struct Buf {
+    void *p;
+    size_t bytes;
+  };
+  std::vector<Buf> bufs;
+  hipError_t take(void **p, size_t bytes) {
+    const hipError_t e = qs::pool_malloc(p, bytes);
+    if (e == hipSuccess) bufs.push_back({*p, bytes});
+    return e;
+  }
   void *psi = nullptr, *lam = nullptr;
   std::vector<void *> ckpt;
   std::vector<size_t> ckpt_at;  // checkpoint j holds psi after ops [0, ckpt_at[j])
@@ -1137,19 +1149,10 @@ namespace {
 void free_ctx(qs_adjoint *c) {
   if (!c) return;
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  if (c->psi) (void)hipFree(c->psi);
-  if (c->lam) (void)hipFree(c->lam);
-  for (void *p : c->ckpt) (void)hipFree(p);
-  if (c->d_h) (void)hipFree(c->d_h);
-  if (c->d_rot) (void)hipFree(c->d_rot);
-  if (c->d_gmat) (void)hipFree(c->d_gmat);
-  if (c->d_part) (void)hipFree(c->d_part);
-  if (c->d_grad) (void)hipFree(c->d_grad);
-  if (c->d_rpart) (void)hipFree(c->d_rpart);
-  if (c->d_ring) (void)hipFree(c->d_ring);
-  if (c->h_ring) (void)hipHostFree(c->h_ring);
+  for (const auto &b : c->bufs) qs::pool_free(b.p, b.bytes, c->ws->device);
   if (c->engine) qs::sweep_engine_free(c->engine);
-  if (c->stream) (void)hipStreamDestroy(c->stream);
+  qs::workspace_put(c->ws);
+  qs::pool_release();
   delete c;
 }
 
@@ -1169,6 +1172,33 @@ hipError_t ring_upload(qs_adjoint *c, const void *src, size_t bytes, void **dev)
   c->ring_off += need;
   *dev = d;
   return hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, c->stream);
+}
+
+// Copy host bytes to device memory in stream order, through the ring in
+// pieces of at most a quarter of it, so that the host source may go away.
+hipError_t upload_to(qs_adjoint *c, const void *src, size_t bytes, void *dev) {
+  for (size_t off = 0; off < bytes;) {
+    const size_t cnt = std::min(bytes - off, c->ring_cap / 4);
+    if (c->ring_off + ((cnt + 255) & ~(size_t)255) > c->ring_cap) {
+      const hipError_t e = hipStreamSynchronize(c->stream);
+      if (e != hipSuccess) return e;
+      c->ring_off = 0;
+    }
+    char *h = c->h_ring + c->ring_off;
+    std::memcpy(h, (const char *)src + off, cnt);
+    c->ring_off += (cnt + 255) & ~(size_t)255;
+    const hipError_t e =
+        hipMemcpyAsync((char *)dev + off, h, cnt, hipMemcpyHostToDevice, c->stream);
+    if (e != hipSuccess) return e;
+    off += cnt;
+  }
+  return hipSuccess;
+}
+
+// The same into a buffer of the pass's own.
+hipError_t upload(qs_adjoint *c, const void *src, size_t bytes, void **dev) {
+  const hipError_t e = c->take(dev, bytes);
+  return e == hipSuccess ? upload_to(c, src, bytes, *dev) : e;
 }
 
 // Whether the forward pass runs through the fused sweep engine
@@ -1216,11 +1246,6 @@ int forward_sweeps(qs_adjoint *c, const double *thetas) {
   const int n = c->n, ntot = c->n + c->nb;
   const size_t Bp = c->Bp, B = c->B, P = c->P;
   hipError_t e = hipSuccess;
-  if (!c->d_ring) {
-    c->ring_cap = 8u << 20;
-    AJ(hipMalloc((void **)&c->d_ring, c->ring_cap));
-    AJ(hipHostMalloc((void **)&c->h_ring, c->ring_cap));
-  }
   if (!c->engine) c->engine = qs::sweep_engine_new();
   qs::SweepRunner run;
   run.n = ntot;
@@ -1311,7 +1336,7 @@ int forward_sweeps(qs_adjoint *c, const double *thetas) {
         const int rc = flush();
         if (rc != QS_OK) return rc;
         void *cp = nullptr;
-        AJ(hipMalloc(&cp, c->state_bytes()));
+        AJ(c->take(&cp, c->state_bytes()));
         AJ(hipMemcpyAsync(cp, c->psi, c->state_bytes(), hipMemcpyDeviceToDevice, c->stream));
         c->ckpt.push_back(cp);
         c->ckpt_at.push_back(i + 1);
@@ -1329,24 +1354,19 @@ int forward_t(qs_adjoint *c, const double *thetas, const uint64_t *masks, const 
   const size_t Bp = c->Bp, B = c->B, P = c->P;
   const uint64_t total = (uint64_t)Bp << n;
   hipError_t e = hipSuccess;
-  AJ(hipMalloc(&c->psi, c->state_bytes()));
+  AJ(c->take(&c->psi, c->state_bytes()));
   // observable table
   {
-    unsigned long long *d_m = nullptr;
-    double *d_c = nullptr;
-    AJ(hipMalloc((void **)&c->d_h, sizeof(double) << n));
-    AJ(hipMalloc((void **)&d_m, sizeof(unsigned long long) * (nterms ? nterms : 1)));
-    AJ(hipMalloc((void **)&d_c, sizeof(double) * (nterms ? nterms : 1)));
-    if (nterms) {
-      AJ(hipMemcpy(d_m, masks, sizeof(unsigned long long) * nterms, hipMemcpyHostToDevice));
-      AJ(hipMemcpy(d_c, coeffs, sizeof(double) * nterms, hipMemcpyHostToDevice));
-    }
+    AJ(c->take((void **)&c->d_h, sizeof(double) << n));
+    void *d_m = nullptr, *d_c = nullptr;
+    const uint64_t none = 0;
+    AJ(upload(c, nterms ? masks : &none, sizeof(uint64_t) * std::max<size_t>(nterms, 1), &d_m));
+    AJ(upload(c, nterms ? coeffs : (const double *)&none,
+              sizeof(double) * std::max<size_t>(nterms, 1), &d_c));
     hipLaunchKernelGGL(k_htable, dim3(grid_of(1ull << n, kBlock * 4)), dim3(kBlock), 0, c->stream,
-                       c->d_h, n, d_m, d_c, (int)nterms);
+                       c->d_h, n, (const unsigned long long *)d_m, (const double *)d_c,
+                       (int)nterms);
     AJ(hipGetLastError());
-    AJ(hipStreamSynchronize(c->stream));
-    (void)hipFree(d_m);
-    (void)hipFree(d_c);
   }
   // rotation matrices, one per (rotation, batch element)
   const int nrot = c->circ.nrot;
@@ -1371,8 +1391,8 @@ int forward_t(qs_adjoint *c, const double *thetas, const uint64_t *masks, const 
       for (int k = 0; k < 8; ++k) dst[k] = (R)m[k];
     }
   }
-  AJ(hipMalloc(&c->d_rot, rot.size() * sizeof(R)));
-  AJ(hipMemcpy(c->d_rot, rot.data(), rot.size() * sizeof(R), hipMemcpyHostToDevice));
+  AJ(c->take(&c->d_rot, rot.size() * sizeof(R)));
+  AJ(upload_to(c, rot.data(), rot.size() * sizeof(R), c->d_rot));
   // diagonal tables of the fixed gates
   {
     std::vector<R> tab;
@@ -1391,8 +1411,8 @@ int forward_t(qs_adjoint *c, const double *thetas, const uint64_t *masks, const 
       }
     }
     if (tab.empty()) tab.push_back((R)0);
-    AJ(hipMalloc(&c->d_gmat, tab.size() * sizeof(R)));
-    AJ(hipMemcpy(c->d_gmat, tab.data(), tab.size() * sizeof(R), hipMemcpyHostToDevice));
+    AJ(c->take(&c->d_gmat, tab.size() * sizeof(R)));
+    AJ(upload_to(c, tab.data(), tab.size() * sizeof(R), c->d_gmat));
   }
   hipLaunchKernelGGL(k_init_zero_states<R>, dim3(grid_of(total, kBlock * 4)), dim3(kBlock), 0,
                      c->stream, (T *)c->psi, n, total);
@@ -1420,7 +1440,7 @@ int forward_t(qs_adjoint *c, const double *thetas, const uint64_t *masks, const 
       if (c->checkpoint_every > 0 && layer % c->checkpoint_every == 0 &&
           layer < c->circ.layer_ends.size()) {
         void *cp = nullptr;
-        AJ(hipMalloc(&cp, c->state_bytes()));
+        AJ(c->take(&cp, c->state_bytes()));
         AJ(hipMemcpyAsync(cp, c->psi, c->state_bytes(), hipMemcpyDeviceToDevice, c->stream));
         c->ckpt.push_back(cp);
         c->ckpt_at.push_back(i + 1);
@@ -1432,9 +1452,9 @@ int forward_t(qs_adjoint *c, const double *thetas, const uint64_t *masks, const 
   const uint64_t per = std::min<uint64_t>(len, 1ull << 14);
   const int nblk = (int)((len + per - 1) / per);
   c->part_count = std::max<size_t>((size_t)nblk, (size_t)((pps + 1023) / 1024)) * Bp;
-  AJ(hipMalloc((void **)&c->d_part, c->part_count * sizeof(double)));
+  AJ(c->take((void **)&c->d_part, c->part_count * sizeof(double)));
   double *d_e = nullptr;
-  AJ(hipMalloc((void **)&d_e, Bp * sizeof(double)));
+  AJ(c->take((void **)&d_e, Bp * sizeof(double)));
   hipLaunchKernelGGL(k_expect<R>, dim3(nblk, (unsigned)Bp), dim3(kBlock), 0, c->stream,
                      (const T *)c->psi, n, c->d_h, per, c->d_part);
   hipLaunchKernelGGL(k_sum_rows, dim3((unsigned)Bp), dim3(kBlock), 0, c->stream,
@@ -1443,7 +1463,6 @@ int forward_t(qs_adjoint *c, const double *thetas, const uint64_t *masks, const 
   std::vector<double> eh(Bp);
   AJ(hipMemcpyAsync(eh.data(), d_e, Bp * sizeof(double), hipMemcpyDeviceToHost, c->stream));
   AJ(hipStreamSynchronize(c->stream));
-  (void)hipFree(d_e);
   if (energies)
     for (size_t b = 0; b < B; ++b) energies[b] = eh[b];
   return QS_OK;
@@ -1544,12 +1563,7 @@ int reverse_blocks(qs_adjoint *c) {
   // rows of partial sums per block: within 64 MiB
   const int rmax =
       (int)std::max<uint64_t>(1, std::min<uint64_t>(kRevMaxRows, (64ull << 20) / (8 * ntiles)));
-  if (!c->d_rpart) AJ(hipMalloc((void **)&c->d_rpart, (uint64_t)rmax * ntiles * sizeof(double)));
-  if (!c->d_ring) {
-    c->ring_cap = 8u << 20;
-    AJ(hipMalloc((void **)&c->d_ring, c->ring_cap));
-    AJ(hipHostMalloc((void **)&c->h_ring, c->ring_cap));
-  }
+  if (!c->d_rpart) AJ(c->take((void **)&c->d_rpart, (uint64_t)rmax * ntiles * sizeof(double)));
   const uint64_t lowset = (1ull << low) - 1ull;
   constexpr bool strict = std::is_same<R, float>::value;
   // Whether an operation may run ahead of those that touch bx off the
@@ -1896,8 +1910,8 @@ int backward_t(qs_adjoint *c, double *grads) {
   const size_t Bp = c->Bp, P = c->P;
   const uint64_t total = (uint64_t)Bp << n;
   hipError_t e = hipSuccess;
-  if (!c->lam) AJ(hipMalloc(&c->lam, c->state_bytes()));
-  if (!c->d_grad) AJ(hipMalloc((void **)&c->d_grad, Bp * std::max<size_t>(P, 1) * sizeof(double)));
+  if (!c->lam) AJ(c->take(&c->lam, c->state_bytes()));
+  if (!c->d_grad) AJ(c->take((void **)&c->d_grad, Bp * std::max<size_t>(P, 1) * sizeof(double)));
   hipLaunchKernelGGL(k_fill_zero, dim3(grid_of(Bp * P, kBlock)), dim3(kBlock), 0, c->stream,
                      c->d_grad, (uint64_t)(Bp * P));
   AJ(hipGetLastError());
@@ -1952,12 +1966,17 @@ int qs_pcircuit_new(size_t n, qs_pcircuit **out) {
   if (!out) return fail_arg("out is NULL");
   if (n < 1 || n > 30) return qs::set_error(QS_ERR_ARGUMENT, n, 0, "pcircuit needs 1..30 qubits");
   qs_pcircuit *c = new qs_pcircuit();
+  qs::pool_retain();  // buffers of its passes are kept while it lives
   c->n = (int)n;
   *out = c;
   return QS_OK;
 }
 
-void qs_pcircuit_free(qs_pcircuit *c) { delete c; }
+void qs_pcircuit_free(qs_pcircuit *c) {
+  if (!c) return;
+  delete c;
+  qs::pool_release();
+}
 
 int qs_pcircuit_gate(qs_pcircuit *c, const double *matrix, const size_t *targets, size_t k) {
   if (!c || !matrix || !targets) return fail_arg("NULL argument");
@@ -2034,11 +2053,16 @@ int qs_adjoint_forward(const qs_pcircuit *c, const double *thetas, size_t batch,
   a->P = c->nparams;
   a->dtype = dtype;
   a->checkpoint_every = checkpoint_every;
-  hipError_t e = hipStreamCreateWithFlags(&a->stream, hipStreamNonBlocking);
+  hipError_t e = qs::workspace_get(&a->ws);
   if (e != hipSuccess) {
     delete a;
-    return qs::set_hip_error(e, "hipStreamCreate");
+    return qs::set_hip_error(e, "adjoint workspace");
   }
+  qs::pool_retain();
+  a->stream = a->ws->stream;
+  a->d_ring = a->ws->d_ring;
+  a->h_ring = a->ws->h_ring;
+  a->ring_cap = qs::kRingBytes;
   const int rc = dtype == QS_C128 ? forward_t<double>(a, thetas, masks, coeffs, nterms, energies)
                                   : forward_t<float>(a, thetas, masks, coeffs, nterms, energies);
   if (rc != QS_OK || !ctx) {

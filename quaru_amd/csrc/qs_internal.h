@@ -62,6 +62,36 @@ struct Fixed {
 
 Fixed make_fixed(uint64_t mask, uint64_t set);
 
+// ---- kept device memory and workspaces (qs_pool.hip) --------------------------
+
+constexpr int kReduceBlocks = 1024;
+constexpr size_t kRedDoubles = 4 * kReduceBlocks + 64;
+constexpr size_t kRingBytes = 8u << 20;
+
+// hipMalloc and hipFree on the current device through the pool of kept
+// blocks.  pool_free takes the size and device of the allocation; no GPU work
+// may use the block any more.
+hipError_t pool_malloc(void **out, size_t bytes);
+void pool_free(void *p, size_t bytes, int device);
+
+// Registers, circuits and adjoint passes count themselves while they live;
+// when none does, the pool gives most of its memory back.
+void pool_retain();
+void pool_release();
+
+// What every register and adjoint pass needs beside its states: a stream, an
+// upload ring (pinned host buffer mirrored in device memory) and buffers of
+// the reductions.  put: the stream has been drained.
+struct Workspace {
+  int device = 0;
+  hipStream_t stream = nullptr;
+  char *d_ring = nullptr, *h_ring = nullptr;
+  double *d_red = nullptr, *h_red = nullptr;
+};
+
+hipError_t workspace_get(Workspace **out);
+void workspace_put(Workspace *w);
+
 // Classify a dense 2^k x 2^k complex128 matrix on `targets` (qs_register.hip);
 // cmask/cval are controls already known.
 Gate classify_matrix(const double *mat, const size_t *targets, size_t k, uint64_t cmask,
@@ -94,7 +124,6 @@ hipError_t launch_gate_perm(void *psi, int n, const Gate &g, const void *d_tab, 
 
 // Reductions write FP64 results to device memory `d_out` (caller copies).
 // d_part must hold kReduceBlocks * 2 doubles.
-constexpr int kReduceBlocks = 1024;
 template <typename R>
 hipError_t launch_prob_split(const void *psi, int n, int target, double *d_part, double *d_out,
                              hipStream_t s);

@@ -68,11 +68,12 @@ struct qs_register {
   int dtype = QS_C128;
   uint64_t len = 1;
   int device = 0;
+  qs::Workspace *ws = nullptr;  // owns stream, ring, d_red and h_red below
   hipStream_t stream = nullptr;
   void *psi = nullptr;
   void *scratch = nullptr;  // 2^n amplitudes, only for dense ops with > 5 active bits
   double *d_red = nullptr;  // reduction partials + results
-  size_t d_red_bytes = 0;
+  bool slots_used = false;  // a deferred measurement wrote its slot in d_red
   double *d_big = nullptr;  // measurement and readout work buffer, grown on demand
   size_t d_big_bytes = 0;
   void *d_upload = nullptr;  // tables of gates too large for the ring, grown on demand
@@ -112,7 +113,6 @@ struct qs_register {
 
 namespace {
 
-constexpr size_t kRingBytes = 8u << 20;
 // Readouts (state, probabilities, amplitudes) go through the register's work
 // buffer in pieces of at most 2^22 amplitudes (64 MiB widened to complex128),
 // so they allocate nothing after the first call.
@@ -120,7 +120,6 @@ constexpr int kReadoutBits = 22;
 constexpr uint64_t kReadoutAmps = 1ull << kReadoutBits;
 // Shots of qs_sample_cdf scanned per launch (2 MiB of work buffer).
 constexpr size_t kSamplePiece = 1u << 16;
-constexpr size_t kRedDoubles = 4 * qs::kReduceBlocks + 64;
 
 bool valid_dtype(int d) { return d == QS_C128 || d == QS_C64; }
 
@@ -145,18 +144,17 @@ int alloc_register(size_t n, int dtype, qs_register **out) {
   r->dtype = dtype;
   r->len = 1ull << n;
   hipError_t e = hipGetDevice(&r->device);
-  if (e == hipSuccess) e = hipStreamCreateWithFlags(&r->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = hipMalloc(&r->psi, r->state_bytes());
+  qs::pool_retain();
+  if (e == hipSuccess) e = qs::workspace_get(&r->ws);
   if (e == hipSuccess) {
-    r->d_red_bytes = kRedDoubles * sizeof(double);
-    e = hipMalloc((void **)&r->d_red, r->d_red_bytes);
+    r->stream = r->ws->stream;
+    r->d_red = r->ws->d_red;
+    r->h_red = r->ws->h_red;
+    r->d_ring = r->ws->d_ring;
+    r->h_ring = r->ws->h_ring;
+    r->ring_cap = qs::kRingBytes;
+    e = qs::pool_malloc(&r->psi, r->state_bytes());
   }
-  if (e == hipSuccess) e = hipHostMalloc((void **)&r->h_red, 64 * sizeof(double));
-  if (e == hipSuccess) {
-    r->ring_cap = kRingBytes;
-    e = hipMalloc((void **)&r->d_ring, r->ring_cap);
-  }
-  if (e == hipSuccess) e = hipHostMalloc((void **)&r->h_ring, r->ring_cap);
   if (e != hipSuccess) {
     qs_register_free(r);
     return hip_fail(e, "allocating the register");
@@ -172,10 +170,10 @@ hipError_t ensure_big(qs_register *r, size_t bytes, double **out) {
   if (r->d_big_bytes < bytes) {
     hipError_t e = hipStreamSynchronize(r->stream);
     if (e != hipSuccess) return e;
-    if (r->d_big) (void)hipFree(r->d_big);
+    qs::pool_free(r->d_big, r->d_big_bytes, r->device);
     r->d_big = nullptr;
     r->d_big_bytes = 0;
-    e = hipMalloc((void **)&r->d_big, bytes);
+    e = qs::pool_malloc((void **)&r->d_big, bytes);
     if (e != hipSuccess) return e;
     r->d_big_bytes = bytes;
   }
@@ -216,10 +214,10 @@ hipError_t big_upload(qs_register *r, const void *src, size_t bytes, void **dev)
   if (r->d_upload_bytes < bytes) {
     e = hipStreamSynchronize(r->stream);
     if (e != hipSuccess) return e;
-    if (r->d_upload) (void)hipFree(r->d_upload);
+    qs::pool_free(r->d_upload, r->d_upload_bytes, r->device);
     r->d_upload = nullptr;
     r->d_upload_bytes = 0;
-    e = hipMalloc(&r->d_upload, bytes);
+    e = qs::pool_malloc(&r->d_upload, bytes);
     if (e != hipSuccess) return e;
     r->d_upload_bytes = bytes;
   }
@@ -455,7 +453,7 @@ hipError_t launch_one(qs_register *r, const Gate &g) {
                                                      : big_upload(r, buf.data(), buf.size(), &dm);
       if (e != hipSuccess) return e;
       if (!r->scratch) {
-        e = hipMalloc(&r->scratch, r->state_bytes());
+        e = qs::pool_malloc(&r->scratch, r->state_bytes());
         if (e != hipSuccess) return e;
       }
       ++r->st_kernels;
@@ -478,7 +476,7 @@ hipError_t launch_one(qs_register *r, const Gate &g) {
                                        : big_upload(r, buf.data(), bytes, &dm);
         if (e != hipSuccess) return e;
         if (g.na > 5 && !r->scratch) {
-          e = hipMalloc(&r->scratch, r->state_bytes());
+          e = qs::pool_malloc(&r->scratch, r->state_bytes());
           if (e != hipSuccess) return e;
         }
       }
@@ -977,16 +975,15 @@ int qs_register_from_qubits(const double *qubits, const size_t *lens, size_t cou
   int rc = alloc_register(count, dtype, out);
   if (rc) return rc;
   qs_register *r = *out;
-  double *d_q = nullptr;
-  hipError_t e = hipMalloc((void **)&d_q, std::max<size_t>(1, count) * 4 * sizeof(double));
-  if (e == hipSuccess && count)
-    e = hipMemcpy(d_q, qubits, count * 4 * sizeof(double), hipMemcpyHostToDevice);
+  // the qubits' amplitudes through the upload ring (at most 40 of them)
+  void *d_q = nullptr;
+  const double none[4] = {};
+  hipError_t e = ring_upload(r, count ? qubits : none,
+                             std::max<size_t>(1, count) * 4 * sizeof(double), &d_q);
   if (e == hipSuccess)
     e = by_dtype(r, [&](auto z) {
-      return qs::launch_init_product<decltype(z)>(r->psi, r->n, d_q, r->stream);
+      return qs::launch_init_product<decltype(z)>(r->psi, r->n, (const double *)d_q, r->stream);
     });
-  if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
-  if (d_q) (void)hipFree(d_q);
   if (e != hipSuccess) {
     qs_register_free(r);
     *out = nullptr;
@@ -1016,6 +1013,7 @@ int qs_register_clone(qs_register *src, qs_register **out) {
 
 void qs_register_free(qs_register *r) {
   if (!r) return;
+  if (r->slots_used) (void)hipMemsetAsync(slot_base(r), 0, QS_MEASURE_SLOTS, r->stream);
   if (r->stream) (void)hipStreamSynchronize(r->stream);
   for (const auto &m : r->marks) {
     (void)hipEventDestroy(m.a);
@@ -1024,15 +1022,12 @@ void qs_register_free(qs_register *r) {
   for (hipEvent_t e : r->ev_pool) (void)hipEventDestroy(e);
   if (r->open_ev) (void)hipEventDestroy(r->open_ev);
   if (r->engine) qs::sweep_engine_free(r->engine);
-  if (r->psi) (void)hipFree(r->psi);
-  if (r->scratch) (void)hipFree(r->scratch);
-  if (r->d_red) (void)hipFree(r->d_red);
-  if (r->d_big) (void)hipFree(r->d_big);
-  if (r->d_upload) (void)hipFree(r->d_upload);
-  if (r->h_red) (void)hipHostFree(r->h_red);
-  if (r->d_ring) (void)hipFree(r->d_ring);
-  if (r->h_ring) (void)hipHostFree(r->h_ring);
-  if (r->stream) (void)hipStreamDestroy(r->stream);
+  qs::pool_free(r->psi, r->state_bytes(), r->device);
+  qs::pool_free(r->scratch, r->state_bytes(), r->device);
+  qs::pool_free(r->d_big, r->d_big_bytes, r->device);
+  qs::pool_free(r->d_upload, r->d_upload_bytes, r->device);
+  qs::workspace_put(r->ws);
+  qs::pool_release();
   delete r;
 }
 
@@ -1167,6 +1162,7 @@ int qs_measure_deferred(qs_register *r, size_t target, double uniform, size_t sl
   if (slot >= QS_MEASURE_SLOTS) return fail(QS_ERR_ARGUMENT, slot, 0, "slot out of range");
   int rc = flush(r);
   if (rc) return rc;
+  r->slots_used = true;
   double *res_dev = r->d_red + 4 * qs::kReduceBlocks;
   auto go = [&](auto z) {
     using Rt = decltype(z);

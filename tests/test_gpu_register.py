@@ -947,3 +947,40 @@ def test_measure_deferred_equals_measure():
         _check(lib.qs_measure_deferred(r.handle, 0, 0.5, _lib.QS_MEASURE_SLOTS))
     with pytest.raises(EngineError):
         _check(lib.qs_read_slots(r.handle, 60, 5, (ctypes.c_ubyte * 5)()))
+
+
+def test_registers_in_turn_share_no_contents():
+    # a closed register's buffers go to the next one: states and measurement
+    # slots start clean, from several threads at once
+    import ctypes
+    import threading
+
+    from quaru_amd import _lib
+
+    lib = _lib.load()
+    failures = []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        for k in range(12):
+            n = int(rng.integers(1, 12))
+            r = Register.from_int(n, 1, dtype="c128", seed=seed)
+            out = np.full(_lib.QS_MEASURE_SLOTS, 7, dtype=np.uint8)
+            rc = lib.qs_read_slots(r.handle, 0, out.size, out.ctypes.data_as(ctypes.c_void_p))
+            want = np.zeros(1 << n)
+            want[1] = 1
+            if rc or out.any() or not np.array_equal(r.state, want):
+                failures.append((seed, k, n))
+            for q in range(n):
+                r.apply(ops.not_(q))
+            lib.qs_measure_deferred(r.handle, n - 1, 0.5, int(rng.integers(64)))
+            if k % 3 == 0:
+                r.clone().close()
+            r.close()
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures
