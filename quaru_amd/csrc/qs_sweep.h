@@ -33,6 +33,9 @@ struct SweepRunner {
   int n = 0;
   bool dtype_c64 = false;
   void *psi = nullptr;
+  // States of the batch, when batched gates stack 2^nb of them in the high
+  // index bits and only the first `states` matter; 0: all.
+  size_t states = 0;
   hipStream_t stream = nullptr;
   // Copy host bytes to a device buffer that stays valid until the stream
   // reaches the next launch.

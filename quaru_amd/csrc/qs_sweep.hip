@@ -637,7 +637,8 @@ hipError_t execute_t(SweepRunner &run, const std::vector<Gate> &gates, uint64_t 
       std::fprintf(stderr, " ops %u\n", h.nops);
     }
     h.npool = (uint32_t)pool.size();
-    h.ntiles = 1ull << (n - T);
+    // the padding states of a batch are the last tiles: they are left out
+    h.ntiles = run.states && nt < n ? (uint64_t)run.states << (nt - T) : 1ull << (n - T);
     const size_t hbytes = (sizeof(SweepHeader) + 15) & ~(size_t)15;
     const size_t bbytes = blob_bytes<R>((int)h.nops, (int)h.npool);
     blob.assign(bbytes, 0);

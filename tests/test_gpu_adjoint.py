@@ -340,3 +340,58 @@ def test_ansatz20_full_size(dtype):
         ex0 = Expectation(ParamCircuit.from_ansatz(ans), ref["masks"], ref["coeffs"])
         ex0.forward(th[:8])
         assert np.max(np.abs(ex0.backward() - g[:8])) < 1e-10
+
+
+@pytest.mark.parametrize("dtype,tol", [("c128", 1e-12), ("c64", 2e-5)])
+@pytest.mark.parametrize("n,batch", [(1, 3), (5, 5), (9, 3), (10, 33), (11, 5), (13, 9)])
+def test_batches_equal_their_parameter_sets_alone(n, batch, dtype, tol):
+    # padding states of a batch are left out; tiles of every size
+    ans = circuits.hardware_efficient_ansatz(n, 3)
+    masks, coeffs = circuits.zz_chain_observable(n)
+    th = circuits.seeded_thetas(batch, ans.nparams, seed=17)
+    pc = ParamCircuit.from_ansatz(ans)
+    ex = Expectation(pc, masks, coeffs, dtype=dtype, checkpoint_every=2)
+    e = ex.forward(th)
+    g = ex.backward()
+    one = Expectation(pc, masks, coeffs, dtype="c128")
+    for b in sorted({0, batch // 2, batch - 1}):
+        eb = one.forward(th[b])
+        gb = one.backward()
+        assert np.max(np.abs(e[b] - eb[0])) < tol * n
+        assert np.max(np.abs(g[b] - gb[0])) < tol * n
+
+
+@pytest.mark.parametrize("dtype,tol", [("c128", 1e-9), ("c64", 2e-3)])
+@pytest.mark.parametrize("n", [2, 8, 9, 11, 14])
+def test_reverse_blocks_with_every_record(n, dtype, tol):
+    # rotations about all axes in any order, several Z rotations of one qubit
+    # in a row, phases and diagonals on and off the tile, controlled 2x2s:
+    # against central differences of the engine's own FP64 energies
+    rng = np.random.default_rng(n)
+    pc = ParamCircuit(n)
+    p = 0
+    for _ in range(70):
+        k = rng.integers(0, 8)
+        a, b = (int(q) for q in rng.permutation(n)[:2])
+        if k < 4:
+            pc.rotation("xyzz"[k], a, p)
+            p += 1
+        elif k == 4:
+            pc.gate(np.diag(np.exp(1j * rng.random(4) * 6)), [a, b])
+        elif k == 5:
+            pc.gate(ops.cz(a, b).matrix(), [a, b])
+        elif k == 6:
+            pc.gate(np.diag([1, 1, 1, np.exp(0.7j)]), [a, b])
+        else:
+            pc.gate(ops.cnot(a, b).matrix(), ops.cnot(a, b).targets())
+    masks, coeffs = circuits.zz_chain_observable(n)
+    th = rng.random((3, p)) * 6.2
+    ex = Expectation(pc, masks, coeffs, dtype=dtype)
+    ex.forward(th)
+    g = ex.backward()
+    fd = Expectation(pc, masks, coeffs, dtype="c128")
+    for q in sorted({0, p // 3, p // 2, p - 1}):
+        d = np.zeros(p)
+        d[q] = 1e-4
+        want = (fd.energies(th + d) - fd.energies(th - d)) / 2e-4
+        assert np.max(np.abs(g[:, q] - want)) < max(tol, 1e-6)
