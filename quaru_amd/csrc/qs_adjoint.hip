@@ -1156,7 +1156,6 @@ void free_ctx(qs_adjoint *c) {
   for (const auto &b : c->bufs) qs::pool_free(b.p, b.bytes, c->ws->device);
   if (c->engine) qs::sweep_engine_free(c->engine);
   qs::workspace_put(c->ws);
-  qs::pool_release();
   delete c;
 }
 
@@ -1971,17 +1970,12 @@ int qs_pcircuit_new(size_t n, qs_pcircuit **out) {
   if (!out) return fail_arg("out is NULL");
   if (n < 1 || n > 30) return qs::set_error(QS_ERR_ARGUMENT, n, 0, "pcircuit needs 1..30 qubits");
   qs_pcircuit *c = new qs_pcircuit();
-  qs::pool_retain();  // buffers of its passes are kept while it lives
   c->n = (int)n;
   *out = c;
   return QS_OK;
 }
 
-void qs_pcircuit_free(qs_pcircuit *c) {
-  if (!c) return;
-  delete c;
-  qs::pool_release();
-}
+void qs_pcircuit_free(qs_pcircuit *c) { delete c; }
 
 int qs_pcircuit_gate(qs_pcircuit *c, const double *matrix, const size_t *targets, size_t k) {
   if (!c || !matrix || !targets) return fail_arg("NULL argument");
@@ -2063,7 +2057,6 @@ int qs_adjoint_forward(const qs_pcircuit *c, const double *thetas, size_t batch,
     delete a;
     return qs::set_hip_error(e, "adjoint workspace");
   }
-  qs::pool_retain();
   a->stream = a->ws->stream;
   a->d_ring = a->ws->d_ring;
   a->h_ring = a->ws->h_ring;

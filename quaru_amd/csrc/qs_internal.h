@@ -74,11 +74,6 @@ constexpr size_t kRingBytes = 8u << 20;
 hipError_t pool_malloc(void **out, size_t bytes);
 void pool_free(void *p, size_t bytes, int device);
 
-// Registers, circuits and adjoint passes count themselves while they live;
-// when none does, the pool gives most of its memory back.
-void pool_retain();
-void pool_release();
-
 // What every register and adjoint pass needs beside its states: a stream, an
 // upload ring (pinned host buffer mirrored in device memory) and buffers of
 // the reductions.  put: the stream has been drained.

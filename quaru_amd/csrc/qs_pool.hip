@@ -3,24 +3,28 @@
 //
 // A register or an adjoint pass lives for one run of a program that makes
 // the next one at once.  hipMalloc and hipFree of its buffers cost set-up
-// time on every run, and memory handed back and taken again at many GB/s
-// makes the driver clear it each time: an adjoint loop that allocated 6 GiB
-// per 33 ms pass stalled now and then for 0.1 to 2 s.  So freed blocks are
-// kept, by size, and handed to the next caller of the same size.
+// time on every run, and the driver clears memory that is handed back before
+// it gives it out again, at some 50 GB/s: an adjoint loop that allocated 6 GiB
+// per 33 ms pass stalled now and then for 0.1 to 2 s, and a loop over 32 GiB
+// registers took 0.96 s per pass of 0.38 s of work.  So freed blocks are kept,
+// by size, and handed to the next caller of the same size.
 //
-// Bounds: blocks of more than kMaxBlock bytes are never kept, all kept blocks
-// together take at most kMaxKept bytes per device, the oldest leave first;
-// when the last register and circuit is gone, all but kIdleKept bytes are
-// given back; and when an allocation of this library fails, everything kept
-// on the device is given back before it is tried again.  A block is handed
-// in only when no GPU work uses it any more (its owner has drained its
-// stream), so any thread and any stream may take it next.  Contents are
-// whatever was there.
+// Bounds: all kept blocks together take at most an eighth of the device's
+// memory, the oldest leave first; once nothing has been taken or handed in
+// for a second, all but kIdleKept bytes are given back; and when an
+// allocation of this library fails, everything kept on the device is given
+// back before it is tried again.  A block is handed in only when no GPU work
+// uses it any more (its owner has drained its stream), so any thread and any
+// stream may take it next.  Contents are whatever was there.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
+#include <chrono>
+#include <condition_variable>
+#include <cstdlib>
 #include <list>
+#include <map>
 #include <mutex>
+#include <thread>
 #include <vector>
 
 #include "qs_internal.h"
@@ -28,9 +32,8 @@
 namespace qs {
 namespace {
 
-constexpr size_t kMaxBlock = 2ull << 30;
-constexpr size_t kMaxKept = 8ull << 30;
 constexpr size_t kIdleKept = 64ull << 20;
+constexpr auto kIdle = std::chrono::seconds(1);
 constexpr size_t kMaxSpaces = 4;  // kept workspaces per device
 
 struct Block {
@@ -42,8 +45,14 @@ struct Block {
 struct Pool {
   std::mutex mu;
   std::list<Block> blocks;  // oldest first
+  size_t kept = 0;          // bytes in blocks
   std::vector<Workspace *> spaces;
-  size_t live = 0;  // registers and circuits
+  std::map<int, size_t> bound;  // bytes kept per device at most
+  // gives back what is idle
+  std::condition_variable wake;
+  std::mutex freeing;  // held while the idle thread frees
+  std::chrono::steady_clock::time_point used;
+  bool started = false, stopping = false;
 };
 
 // Never destroyed: threads may free their registers while the process exits.
@@ -65,6 +74,7 @@ std::vector<Block> take_out(Pool &p, int device, size_t keep) {
       continue;
     }
     kept -= it->bytes;
+    p.kept -= it->bytes;
     out.push_back(*it);
     it = p.blocks.erase(it);
   }
@@ -79,6 +89,39 @@ bool out_of_memory(hipError_t e) {
   return e == hipErrorOutOfMemory || e == hipErrorMemoryAllocation;
 }
 
+void idle_thread() {
+  Pool &p = pool();
+  std::unique_lock<std::mutex> lk(p.mu);
+  while (!p.stopping) {
+    if (p.kept <= kIdleKept) {
+      p.wake.wait(lk);
+      continue;
+    }
+    const auto due = p.used + kIdle;
+    if (std::chrono::steady_clock::now() < due) {
+      p.wake.wait_until(lk, due);
+      continue;
+    }
+    const std::vector<Block> freed = take_out(p, -1, kIdleKept);
+    std::unique_lock<std::mutex> busy(p.freeing);
+    lk.unlock();
+    give_back(freed);
+    busy.unlock();
+    lk.lock();
+  }
+}
+
+// At exit (before the runtime is torn down): no frees from here on, and none
+// under way.
+void stop_idle_thread() {
+  Pool &p = pool();
+  {
+    std::lock_guard<std::mutex> lk(p.mu);
+    p.stopping = true;
+  }
+  std::lock_guard<std::mutex> busy(p.freeing);
+}
+
 }  // namespace
 
 hipError_t pool_malloc(void **out, size_t bytes) {
@@ -89,10 +132,12 @@ hipError_t pool_malloc(void **out, size_t bytes) {
   Pool &p = pool();
   {
     std::lock_guard<std::mutex> lk(p.mu);
+    p.used = std::chrono::steady_clock::now();
     for (auto it = p.blocks.end(); it != p.blocks.begin();) {
       --it;  // the newest first
       if (it->bytes == bytes && it->device == device) {
         *out = it->p;
+        p.kept -= bytes;
         p.blocks.erase(it);
         return hipSuccess;
       }
@@ -105,7 +150,8 @@ hipError_t pool_malloc(void **out, size_t bytes) {
     std::lock_guard<std::mutex> lk(p.mu);
     freed = take_out(p, device, 0);
   }
-  if (freed.empty()) return e;
+  // (also when nothing was kept: the idle thread may just be freeing)
+  std::lock_guard<std::mutex> busy(p.freeing);
   (void)hipGetLastError();
   give_back(freed);
   return hipMalloc(out, bytes);
@@ -113,33 +159,34 @@ hipError_t pool_malloc(void **out, size_t bytes) {
 
 void pool_free(void *ptr, size_t bytes, int device) {
   if (!ptr) return;
-  if (bytes == 0 || bytes > kMaxBlock) {
-    (void)hipFree(ptr);
-    return;
-  }
   Pool &p = pool();
   std::vector<Block> freed;
+  bool kept = false;
   {
     std::lock_guard<std::mutex> lk(p.mu);
-    p.blocks.push_back({ptr, bytes, device});
-    freed = take_out(p, device, kMaxKept);
+    p.used = std::chrono::steady_clock::now();
+    auto it = p.bound.find(device);
+    if (it == p.bound.end()) {
+      size_t total = 0;
+      hipDevice_t d = 0;
+      if (hipDeviceGet(&d, device) != hipSuccess || hipDeviceTotalMem(&total, d) != hipSuccess)
+        total = 0;
+      it = p.bound.emplace(device, total / 8).first;
+    }
+    kept = bytes > 0 && bytes <= it->second && !p.stopping;
+    if (kept) {
+      p.blocks.push_back({ptr, bytes, device});
+      p.kept += bytes;
+      freed = take_out(p, device, it->second);
+      if (!p.started && p.kept > kIdleKept) {
+        p.started = true;
+        std::atexit(stop_idle_thread);
+        std::thread(idle_thread).detach();
+      }
+      p.wake.notify_one();
+    }
   }
-  give_back(freed);
-}
-
-void pool_retain() {
-  Pool &p = pool();
-  std::lock_guard<std::mutex> lk(p.mu);
-  ++p.live;
-}
-
-void pool_release() {
-  Pool &p = pool();
-  std::vector<Block> freed;
-  {
-    std::lock_guard<std::mutex> lk(p.mu);
-    if (--p.live == 0) freed = take_out(p, -1, kIdleKept);
-  }
+  if (!kept) (void)hipFree(ptr);
   give_back(freed);
 }
 

@@ -144,7 +144,6 @@ int alloc_register(size_t n, int dtype, qs_register **out) {
   r->dtype = dtype;
   r->len = 1ull << n;
   hipError_t e = hipGetDevice(&r->device);
-  qs::pool_retain();
   if (e == hipSuccess) e = qs::workspace_get(&r->ws);
   if (e == hipSuccess) {
     r->stream = r->ws->stream;
@@ -1027,7 +1026,6 @@ void qs_register_free(qs_register *r) {
   qs::pool_free(r->d_big, r->d_big_bytes, r->device);
   qs::pool_free(r->d_upload, r->d_upload_bytes, r->device);
   qs::workspace_put(r->ws);
-  qs::pool_release();
   delete r;
 }
 
