@@ -294,10 +294,114 @@ int validate_dims(size_t rows, size_t cols, size_t k) {
 inline bool is_one(const cd &v) { return v.re == 1.0 && v.im == 0.0; }
 inline bool is_zero(const cd &v) { return v.re == 0.0 && v.im == 0.0; }
 
+// The 2x2 factors of a Kronecker product, lowest matrix bit first.
+using Factors = std::vector<std::array<cd, 4>>;
+
+// A dense gate on several active qubits that is a Kronecker product of
+// 2x2 factors (Hadamard transforms, layers of one-qubit gates that a caller
+// fused into one matrix) is applied as those factors: each is a one-qubit
+// gate that the sweep engine fuses with its neighbours, one pass over the
+// state for many of them, where the dense form costs a pass (and 2^k complex
+// products per amplitude) for each block.  Controls carry over to every
+// factor (C-(A (x) B) = C-A . C-B).  The product must reproduce the matrix
+// to 1e-14 of its largest entry, far inside the engine's 1e-12 bar.
+//
+// `red(r, c)` is the matrix on the active bits.  A matrix that is no such
+// product is told by a few 2x2 minors (of the entries as a 4 x 4^(k-1) matrix
+// of the first bit against the others, of rank one in a product) before its
+// entries are weighed one by one.  A period finding on 15 qubits with 1024 x
+// 1024 Fourier and Hadamard matrices takes 5.4 ms, 85 when every entry of both
+// was copied twice and multiplied out from its ten factors.
+template <typename M>
+bool kron_factors(int k, const M &red, Factors &f) {
+  if (k < 2 || k > 12) return false;
+  const size_t d = (size_t)1 << k;
+  auto cmul = [](const cd &a, const cd &b) {
+    return cd{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
+  };
+  if (k > 5) {
+    double top = 0.0;  // largest component: the largest modulus is below 1.5 times it
+    for (size_t r = 0; r < d; ++r)
+      for (size_t c = 0; c < d; ++c) {
+        const cd &v = red(r, c);
+        const double a = std::fabs(v.re), b = std::fabs(v.im);
+        const double m = a > b ? a : b;
+        if (m > top) top = m;
+      }
+    const double bar = 1e-10 * 2.25 * top * top;
+    for (size_t s = 1; s < 64; ++s) {
+      const size_t r = (s * 0x9E3779B1u) % d & ~(size_t)1, c = (s * 0x85EBCA77u) % d & ~(size_t)1;
+      const size_t r2 = (s * 0xC2B2AE3Du) % d & ~(size_t)1, c2 = (s * 0x27D4EB2Fu) % d & ~(size_t)1;
+      const cd x = cmul(red(r, c), red(r2 | 1, c2 | 1)), y = cmul(red(r | 1, c | 1), red(r2, c2));
+      const cd u = cmul(red(r, c | 1), red(r2, c2)), v = cmul(red(r, c), red(r2, c2 | 1));
+      if (std::hypot(x.re - y.re, x.im - y.im) > bar ||
+          std::hypot(u.re - v.re, u.im - v.im) > bar)
+        return false;
+    }
+  }
+  size_t pr = 0, pc = 0;
+  double amax = -1.0;
+  for (size_t r = 0; r < d; ++r)
+    for (size_t c = 0; c < d; ++c) {
+      const cd &v = red(r, c);
+      const double a = v.im == 0.0 ? std::fabs(v.re) : std::hypot(v.re, v.im);
+      if (a > amax) {
+        amax = a;
+        pr = r;
+        pc = c;
+      }
+    }
+  if (!(amax > 0.0)) return false;
+  const cd p = red(pr, pc);
+  const double pn = p.re * p.re + p.im * p.im;
+  auto cdiv = [&](const cd &v) {  // v / p
+    return cd{(v.re * p.re + v.im * p.im) / pn, (v.im * p.re - v.re * p.im) / pn};
+  };
+  f.assign(k, {});
+  for (int a = 0; a < k; ++a) {
+    const size_t ba = (size_t)1 << a;
+    for (int x = 0; x < 2; ++x)
+      for (int y = 0; y < 2; ++y) {
+        const size_t r = x ? (pr | ba) : (pr & ~ba), c = y ? (pc | ba) : (pc & ~ba);
+        f[a][2 * x + y] = cdiv(red(r, c));
+      }
+  }
+  for (int q = 0; q < 4; ++q) f[0][q] = cmul(f[0][q], p);
+  // the products over the low half of the bits and over the high half, as
+  // tables by row and column
+  const int h = k / 2;
+  auto table = [&](int from, int to) {
+    const size_t n = (size_t)1 << (to - from);
+    std::vector<cd> t(n * n);
+    for (size_t r = 0; r < n; ++r)
+      for (size_t c = 0; c < n; ++c) {
+        cd v{1.0, 0.0};
+        for (int a = from; a < to; ++a)
+          v = cmul(v, f[a][2 * ((r >> (a - from)) & 1) + ((c >> (a - from)) & 1)]);
+        t[r * n + c] = v;
+      }
+    return t;
+  };
+  const std::vector<cd> lo = table(0, h), hi = table(h, k);
+  const size_t nl = (size_t)1 << h, nh = (size_t)1 << (k - h);
+  const double tol = 1e-14 * amax;
+  for (size_t r = 0; r < d; ++r)
+    for (size_t c = 0; c < d; ++c) {
+      const cd v = cmul(lo[(r & (nl - 1)) * nl + (c & (nl - 1))], hi[(r >> h) * nh + (c >> h)]);
+      const cd &w = red(r, c);
+      const double dr = std::fabs(v.re - w.re), di = std::fabs(v.im - w.im);
+      // (NaN fails too)
+      if (!(dr + di <= tol) && !(std::hypot(dr, di) <= tol)) return false;
+    }
+  return true;
+}
+
 // Classify a dense 2^k x 2^k matrix on `targets`; `cmask_in/cval_in` are
-// controls already known (qs_apply_controlled).
+// controls already known (qs_apply_controlled).  With `factors`, a dense
+// matrix that is a Kronecker product leaves its 2x2 factors there and its own
+// entries out.
 Gate classify(const double *mat, const size_t *targets, size_t k, uint64_t cmask_in,
-              uint64_t cval_in) {
+              uint64_t cval_in, Factors *factors = nullptr) {
   const size_t D = (size_t)1 << k;
   const cd *M = reinterpret_cast<const cd *>(mat);
   Gate g;
@@ -332,21 +436,19 @@ Gate classify(const double *mat, const size_t *targets, size_t k, uint64_t cmask
   g.na = (int)actj.size();
   for (int a = 0; a < g.na; ++a) g.act[a] = (int)targets[actj[a]];
   const size_t d = (size_t)1 << g.na;
-  // reduced matrix: rows/cols with every control bit set
-  auto full_index = [&](size_t ri) {
-    size_t x = cbits;
+  // reduced matrix: rows/cols with every control bit set, read in place
+  // through the full index of each reduced index (a copy is made at the end,
+  // of a dense matrix only)
+  std::vector<size_t> full(d, cbits);
+  for (size_t ri = 0; ri < d; ++ri)
     for (int a = 0; a < g.na; ++a)
-      if ((ri >> a) & 1) x |= (size_t)1 << actj[a];
-    return x;
-  };
-  std::vector<cd> red(d * d);
-  for (size_t r = 0; r < d; ++r)
-    for (size_t c = 0; c < d; ++c) red[r * d + c] = M[full_index(r) * D + full_index(c)];
+      if ((ri >> a) & 1) full[ri] |= (size_t)1 << actj[a];
+  auto red = [&](size_t r, size_t c) -> const cd & { return M[full[r] * D + full[c]]; };
   // 2. diagonal?
   bool diag = true;
   for (size_t r = 0; r < d && diag; ++r)
     for (size_t c = 0; c < d; ++c)
-      if (r != c && !is_zero(red[r * d + c])) {
+      if (r != c && !is_zero(red(r, c))) {
         diag = false;
         break;
       }
@@ -361,7 +463,7 @@ Gate classify(const double *mat, const size_t *targets, size_t k, uint64_t cmask
       for (size_t r = 0; r < d && mono; ++r) {
         size_t nz = 0;
         for (size_t c = 0; c < d; ++c)
-          if (!is_zero(red[r * d + c])) {
+          if (!is_zero(red(r, c))) {
             ++nz;
             src[r] = (uint32_t)c;
           }
@@ -372,18 +474,25 @@ Gate classify(const double *mat, const size_t *targets, size_t k, uint64_t cmask
         g.kind = Gate::kPerm;
         g.perm = std::move(src);
         g.m.resize(d);
-        for (size_t r = 0; r < d; ++r) g.m[r] = red[r * d + g.perm[r]];
+        for (size_t r = 0; r < d; ++r) g.m[r] = red(r, g.perm[r]);
         return g;
       }
     }
     g.kind = Gate::kDense;
-    g.m = std::move(red);
+    if (factors && kron_factors(g.na, red, *factors)) return g;
+    g.m.reserve(d * d);
+    for (size_t r = 0; r < d; ++r) {
+      if (g.na == (int)k)  // no controls: rows as they are
+        g.m.insert(g.m.end(), M + r * D, M + (r + 1) * D);
+      else
+        for (size_t c = 0; c < d; ++c) g.m.push_back(red(r, c));
+    }
     return g;
   }
   std::vector<cd> dv(d);
   size_t nonunit = 0;
   for (size_t r = 0; r < d; ++r) {
-    dv[r] = red[r * d + r];
+    dv[r] = red(r, r);
     if (!is_one(dv[r])) ++nonunit;
   }
   if (nonunit == 0) {
@@ -464,15 +573,21 @@ hipError_t launch_one(qs_register *r, const Gate &g) {
       void *dm = nullptr;
       hipError_t e = hipSuccess;
       if (g.na >= 3) {
-        // row-major {re, im} in the register's precision
-        std::vector<T> buf(2 * d * d);
-        for (size_t e = 0; e < d * d; ++e) {
-          buf[2 * e] = (T)g.m[e].re;
-          buf[2 * e + 1] = (T)g.m[e].im;
+        // row-major {re, im} in the register's precision (complex128: the
+        // matrix as it is)
+        std::vector<T> buf;
+        const void *src = g.m.data();
+        if constexpr (std::is_same<T, float>::value) {
+          buf.resize(2 * d * d);
+          for (size_t e = 0; e < d * d; ++e) {
+            buf[2 * e] = (T)g.m[e].re;
+            buf[2 * e + 1] = (T)g.m[e].im;
+          }
+          src = buf.data();
         }
-        const size_t bytes = buf.size() * sizeof(T);
-        e = bytes + 256 <= r->ring_cap ? ring_upload(r, buf.data(), bytes, &dm)
-                                       : big_upload(r, buf.data(), bytes, &dm);
+        const size_t bytes = 2 * d * d * sizeof(T);
+        e = bytes + 256 <= r->ring_cap ? ring_upload(r, src, bytes, &dm)
+                                       : big_upload(r, src, bytes, &dm);
         if (e != hipSuccess) return e;
         if (g.na > 5 && !r->scratch) {
           e = qs::pool_malloc(&r->scratch, r->state_bytes());
@@ -822,63 +937,13 @@ int measure_fast(qs_register *r, const size_t *order, size_t count, const double
   return QS_OK;
 }
 
-// A dense gate on several active qubits that is a Kronecker product of
-// 2x2 factors (Hadamard transforms, layers of one-qubit gates that a caller
-// fused into one matrix) is applied as those factors: each is a one-qubit
-// gate that the sweep engine fuses with its neighbours, one pass over the
-// state for many of them, where the dense form costs a pass (and 2^k complex
-// products per amplitude) for each block.  Controls carry over to every
-// factor (C-(A (x) B) = C-A . C-B).  The product must reproduce the matrix
-// to 1e-14 of its largest entry, far inside the engine's 1e-12 bar.
-bool kron_factors(const Gate &g, std::vector<std::array<cd, 4>> &f) {
-  if (g.kind != Gate::kDense || g.na < 2 || g.na > 12) return false;
-  const int k = g.na;
-  const size_t d = (size_t)1 << k;
-  const cd *M = g.m.data();
-  size_t piv = 0;
-  double amax = -1.0;
-  for (size_t i = 0; i < d * d; ++i) {
-    const double a = std::hypot(M[i].re, M[i].im);
-    if (a > amax) {
-      amax = a;
-      piv = i;
-    }
-  }
-  if (!(amax > 0.0)) return false;
-  const size_t r0 = piv / d, c0 = piv % d;
-  const cd p = M[piv];
-  const double pn = p.re * p.re + p.im * p.im;
-  auto cdiv = [&](const cd &v) {  // v / p
-    return cd{(v.re * p.re + v.im * p.im) / pn, (v.im * p.re - v.re * p.im) / pn};
-  };
-  auto cmul = [](const cd &a, const cd &b) {
-    return cd{a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re};
-  };
-  f.assign(k, {});
-  for (int a = 0; a < k; ++a) {
-    const size_t ba = (size_t)1 << a;
-    for (int x = 0; x < 2; ++x)
-      for (int y = 0; y < 2; ++y) {
-        const size_t r = x ? (r0 | ba) : (r0 & ~ba), c = y ? (c0 | ba) : (c0 & ~ba);
-        f[a][2 * x + y] = cdiv(M[r * d + c]);
-      }
-  }
-  for (int q = 0; q < 4; ++q) f[0][q] = cmul(f[0][q], p);
-  const double tol = 1e-14 * amax;
-  for (size_t r = 0; r < d; ++r)
-    for (size_t c = 0; c < d; ++c) {
-      cd v{1.0, 0.0};
-      for (int a = 0; a < k; ++a) v = cmul(v, f[a][2 * ((r >> a) & 1) + ((c >> a) & 1)]);
-      if (std::hypot(v.re - M[r * d + c].re, v.im - M[r * d + c].im) > tol) return false;
-    }
-  return true;
-}
-
-// Enqueue a classified gate, as its one-qubit factors when it has them and
+// Classify and enqueue a gate, as its one-qubit factors when it has them and
 // fusion is on (with fusion off every factor would be a pass of its own).
-int enqueue_split(qs_register *r, Gate &&g) {
-  std::vector<std::array<cd, 4>> f;
-  if (!r->fusion || !kron_factors(g, f)) return enqueue(r, std::move(g));
+int enqueue_matrix(qs_register *r, const double *matrix, const size_t *targets, size_t k,
+                   uint64_t cmask, uint64_t cval) {
+  Factors f;
+  Gate g = classify(matrix, targets, k, cmask, cval, r->fusion ? &f : nullptr);
+  if (g.kind != Gate::kDense || !g.m.empty()) return enqueue(r, std::move(g));
   int rc = QS_OK;
   for (int a = 0; a < g.na && rc == QS_OK; ++a) {
     const size_t t = (size_t)g.act[a];
@@ -1041,7 +1106,7 @@ int qs_apply(qs_register *r, const double *matrix, size_t rows, size_t cols,
   if (rc) return rc;
   rc = validate_targets((size_t)r->n, targets, k);
   if (rc) return rc;
-  return enqueue_split(r, classify(matrix, targets, k, 0, 0));
+  return enqueue_matrix(r, matrix, targets, k, 0, 0);
 }
 
 int qs_apply_controlled(qs_register *r, const size_t *controls, const unsigned char *cvals,
@@ -1059,7 +1124,7 @@ int qs_apply_controlled(qs_register *r, const size_t *controls, const unsigned c
     cmask |= 1ull << controls[i];
     if (!cvals || cvals[i]) cval |= 1ull << controls[i];
   }
-  return enqueue_split(r, classify(matrix, targets, k, cmask, cval));
+  return enqueue_matrix(r, matrix, targets, k, cmask, cval);
 }
 
 int qs_apply_diagonal(qs_register *r, const double *diag, const size_t *targets, size_t k) {

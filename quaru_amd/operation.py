@@ -19,6 +19,7 @@ Two additions the reference does not need:
 """
 from __future__ import annotations
 
+import copyreg
 import math
 from typing import Callable, Iterable, List, Optional, Sequence
 
@@ -36,7 +37,7 @@ class Operation:
     ``targets + controls`` and ``matrix()`` is the dense equivalent.
     """
 
-    __slots__ = ("_matrix", "_targets", "_controls", "_cvals", "_label")
+    __slots__ = ("_matrix", "_targets", "_controls", "_cvals", "_label", "_call")
 
     def __init__(self, matrix: np.ndarray, targets: Sequence[int],
                  controls: Sequence[int] = (), label: str = "",
@@ -48,6 +49,16 @@ class Operation:
         if self._cvals is not None and len(self._cvals) != len(self._controls):
             raise ValueError("one control value per control")
         self._label = label
+        # the register's C call for this operation: addresses of arrays that
+        # this object owns (made on first use, see Register.try_apply_fast)
+        self._call = None
+
+    def __getstate__(self):
+        # copies and pickles get arrays of their own, so not the addresses
+        slots = {n: getattr(self, n) for n in copyreg._slotnames(type(self))
+                 if n != "_call" and hasattr(self, n)}
+        slots["_call"] = None
+        return getattr(self, "__dict__", None) or None, slots
 
     # -- construction -------------------------------------------------------
     @staticmethod

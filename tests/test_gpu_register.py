@@ -14,6 +14,7 @@ import pytest
 import oracle
 from quaru_amd import OperationError, QuaruPanic, Register, circuits
 from quaru_amd import operation as ops
+from quaru_amd.operation import Operation
 from tests.conftest import random_state, random_unitary
 
 pytestmark = pytest.mark.gpu
@@ -984,3 +985,44 @@ def test_registers_in_turn_share_no_contents():
     for t in threads:
         t.join()
     assert not failures
+
+
+@pytest.mark.parametrize("off", [0.0, 1e-9])
+@pytest.mark.parametrize("k", [2, 5, 6, 7])
+def test_products_of_one_qubit_gates(k, off):
+    # Kronecker products run as their factors, matrices that are 1e-9 off one
+    # as dense gates: both within the bar of the oracle
+    rng = np.random.default_rng(10 * k)
+    n = 9
+    m = np.eye(1)
+    for _ in range(k):
+        m = np.kron(random_unitary(rng, 2), m)
+    m = m + off * rng.standard_normal(m.shape)
+    targets = [int(q) for q in rng.permutation(n)[:k]]
+    psi = random_state(rng, n)
+    r = Register.from_int(n, 0)
+    r.state = psi
+    r.apply(Operation(m, targets))
+    assert maxdiff(r.state, oracle.apply_fast(psi, m, targets)) < TOL
+
+
+def test_copied_operations_use_their_own_arrays():
+    import copy
+    import pickle
+
+    r = Register.from_int(3, 0)
+    op = ops.cnx([0, 2], 1)
+    r.apply(op)  # the call behind it is laid out
+    twins = [copy.copy(op), copy.deepcopy(op), pickle.loads(pickle.dumps(op))]
+    assert all(t._call is None and t == op for t in twins)
+    del op
+    r.apply(ops.not_(0)).apply(ops.not_(2))
+    for t in twins:
+        r.apply(t)
+    assert abs(r.state[0b111] - 1) < TOL
+    # a matrix changed in place is read as it is now
+    op = Operation(np.eye(2), [0])
+    r.apply(op)
+    op.active_matrix[:] = [[0, 1], [1, 0]]
+    r.apply(op)
+    assert abs(r.state[0b110] - 1) < TOL
