@@ -18,7 +18,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libquaru_hip.so")
 SOURCES = ["qs_kernels.hip", "qs_sweep.hip", "qs_register.hip", "qs_adjoint.hip",
-           "qs_sweep_jit.hip", "qs_pool.hip"]
+           "qs_sweep_jit.hip", "qs_pool.hip", "qs_small.hip"]
 # qs_sweep_launch.hip holds the k_sweep instantiations of one (precision,
 # register bits) pair; it is compiled once per pair so that they build in
 # parallel.

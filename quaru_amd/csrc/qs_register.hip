@@ -694,6 +694,7 @@ int flush(qs_register *r) {
     run.n = r->n;
     run.dtype_c64 = r->dtype == QS_C64;
     run.psi = r->psi;
+    run.small = true;
     run.stream = r->stream;
     run.upload = [r](const void *src, size_t bytes, void **dev) {
       return ring_upload(r, src, bytes, dev);

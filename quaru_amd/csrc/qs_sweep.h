@@ -36,6 +36,8 @@ struct SweepRunner {
   // States of the batch, when batched gates stack 2^nb of them in the high
   // index bits and only the first `states` matter; 0: all.
   size_t states = 0;
+  // Whether a state that fits one compute unit may run there (qs_small.hip).
+  bool small = false;
   hipStream_t stream = nullptr;
   // Copy host bytes to a device buffer that stays valid until the stream
   // reaches the next launch.
@@ -59,6 +61,11 @@ struct SweepRunner {
 // per-gate kernels.  Counters are incremented by the launches made.
 hipError_t sweep_execute(SweepEngine *e, SweepRunner &run, const std::vector<Gate> &gates,
                          uint64_t *sweeps, uint64_t *kernels);
+
+// Registers whose state fits one compute unit's LDS run their gates there, in
+// one launch for any run of them (qs_small.hip); whether this one does.
+bool small_fits(int n, bool c64);
+hipError_t execute_small(SweepRunner &run, const std::vector<Gate> &gates, uint64_t *sweeps);
 
 // Register bits per lane used for a dtype (a wave holds 2^(6 + bits)
 // amplitudes of its tile).

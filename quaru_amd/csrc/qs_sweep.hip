@@ -794,6 +794,8 @@ hipError_t sweep_execute(SweepEngine *eng, SweepRunner &run, const std::vector<G
                          uint64_t *sweeps, uint64_t *kernels) {
   (void)eng;
   (void)kernels;
+  if (run.small && !run.host_sweep && small_fits(run.n, run.dtype_c64))
+    return execute_small(run, gates, sweeps);
   if (run.dtype_c64) return execute_t<float>(run, gates, sweeps);
   return execute_t<double>(run, gates, sweeps);
 }

@@ -1026,3 +1026,57 @@ def test_copied_operations_use_their_own_arrays():
     op.active_matrix[:] = [[0, 1], [1, 0]]
     r.apply(op)
     assert abs(r.state[0b110] - 1) < TOL
+
+
+def small_run_ops(rng, n, count):
+    """Every gate form a run in one compute unit's LDS takes, between gates
+    that it leaves to kernels of their own."""
+    opl = []
+    for _ in range(count):
+        q = [int(x) for x in rng.permutation(n)]
+        kind = int(rng.integers(0, 12))
+        if kind < 3:
+            opl.append(Operation(random_unitary(rng, 2), q[:1]))
+        elif kind == 3:
+            opl.append(ops.cnot(q[0], q[1]))
+        elif kind == 4:
+            opl.append(ops.cz(q[0], q[1]))
+        elif kind == 5:
+            opl.append(Operation(random_unitary(rng, 4), q[:2]))
+        elif kind == 6:
+            opl.append(Operation(np.diag(np.exp(1j * rng.random(4) * 6)), q[:2]))
+        elif kind == 7:
+            opl.append(Operation.controlled(q[1:n], random_unitary(rng, 2), q[:1],
+                                            control_values=[bool(v) for v in
+                                                            rng.integers(0, 2, n - 1)]))
+        elif kind == 8:
+            opl.append(ops.rz(float(rng.uniform(0, 6)), q[0]))
+        elif kind == 9 and n > 2:
+            opl.append(ops.to_controlled(Operation(random_unitary(rng, 4), q[:2]), q[2]))
+        elif kind == 10 and n > 2:
+            opl.append(Operation(random_unitary(rng, 8), q[:3]))
+        else:
+            opl.append(ops.to_controlled(ops.phase(q[0]), q[1]))
+    return opl
+
+
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+@pytest.mark.parametrize("n", [2, 3, 5, 6, 8, 10, 12, 13])
+def test_small_registers_in_one_launch(n, dtype):
+    rng = np.random.default_rng(4000 + n)
+    opl = small_run_ops(rng, n, 150)
+    psi = random_state(rng, n)
+    ref = oracle_run(psi.copy(), opl)
+    got = {}
+    for fusion in (True, False):
+        r = Register.from_int(n, 0, dtype=dtype).set_fusion(fusion)
+        r.state = psi
+        for op in opl:
+            r.apply(op)
+        got[fusion] = r.state
+    if dtype == "c128":
+        assert maxdiff(got[True], ref) < TOL
+    else:
+        assert infid(got[True], ref) < 1e-6
+        if n <= 10:  # rounded as by one kernel per gate
+            assert np.array_equal(got[True], got[False])
