@@ -105,6 +105,8 @@ hipError_t launch_init_product(void *psi, int n, const double *d_qubits, hipStre
 template <typename R>
 hipError_t launch_gate_dense(void *psi, int n, const Gate &g, void *d_mat, void *scratch,
                              hipStream_t s);
+// Whether the gate's kernel reads a copy of the state, in `scratch`.
+bool dense_needs_scratch(bool c64, int n, const Gate &g);
 template <typename R>
 hipError_t launch_gate_diag(void *psi, int n, const Gate &g, void *d_mat, hipStream_t s);
 template <typename R>

@@ -729,35 +729,6 @@ static bool stage_map(const Fixed &fx, const Fixed &ax, int n, StageMap &sm) {
   return true;
 }
 
-// Any K: out-of-place from `src` (a copy of the state) into psi, one thread
-// per (group, row).  Used for the dense k = n operations of the examples.
-template <typename R>
-__global__ __launch_bounds__(kBlock) void k_gate_big(typename V2<R>::T *__restrict__ psi,
-                                                     const typename V2<R>::T *__restrict__ src,
-                                                     uint64_t ngroups, int K, Fixed fx, Fixed ax,
-                                                     const typename V2<R>::T *__restrict__ m) {
-  using T = typename V2<R>::T;
-  const uint64_t D = 1ull << K;
-  const uint64_t total = ngroups * D;
-  for (uint64_t w = (uint64_t)blockIdx.x * kBlock + threadIdx.x; w < total;
-       w += (uint64_t)gridDim.x * kBlock) {
-    const uint64_t i = w % D, g = w / D;
-    const uint64_t b = expand(g, fx);
-    uint64_t oi = 0;
-    for (int j = 0; j < K; ++j)
-      if ((i >> j) & 1ull) oi |= 1ull << ax.pos[j];
-    T acc = czero<T>();
-    for (uint64_t j = 0; j < D; ++j) {
-      uint64_t oj = 0;
-      for (int q = 0; q < K; ++q)
-        if ((j >> q) & 1ull) oj |= 1ull << ax.pos[q];
-      const T mv = m[i * D + j];
-      acc = cmla(acc, mv.x, mv.y, src[b | oj]);
-    }
-    psi[b | oi] = acc;
-  }
-}
-
 template <typename R, int D>
 static MatArg<R, D> to_matarg(const Gate &g) {
   MatArg<R, D> m;
@@ -783,6 +754,364 @@ static uint64_t active_mask(const Gate &g) {
   return m;
 }
 
+// ---- dense blocks on the FP64 matrix cores -----------------------------------
+
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// Complex sums of 16 rows x 16 columns.  Four real sums, so that each is one
+// chain over the summed index, as short as the halves of k_gatek's.
+struct CplxAcc {
+  f64x4 rr, ii, ri, ir;
+  __device__ __forceinline__ void clear() { rr = ii = ri = ir = f64x4{0, 0, 0, 0}; }
+  __device__ __forceinline__ double2 at(int v) const {
+    return double2{rr[v] - ii[v], ri[v] + ir[v]};
+  }
+};
+
+// acc += A x B for 4 values of the summed index: lane l holds A[l % 16][l / 16]
+// and B[l / 16][l % 16]; element v of a sum, lane l, is [4 v + l / 16][l % 16].
+template <bool kReal>
+__device__ __forceinline__ void mfma_cplx(CplxAcc &s, double ar, double ai, double2 b) {
+  s.rr = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, b.x, s.rr, 0, 0, 0);
+  s.ri = __builtin_amdgcn_mfma_f64_16x16x4f64(ar, b.y, s.ri, 0, 0, 0);
+  if constexpr (!kReal) {
+    s.ii = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, b.y, s.ii, 0, 0, 0);
+    s.ir = __builtin_amdgcn_mfma_f64_16x16x4f64(ai, b.x, s.ir, 0, 0, 0);
+  }
+}
+
+// Bit layout of one tile of k_dense_tile: 2^LC groups (columns) x 2^K rows =
+// 2^(K+LC) slots.  Slot bit b sits at state index bit pa[b], ascending (the
+// active positions and the lowest LC free ones, so that consecutive lanes of
+// a staging load take the lowest index bits the tile has); col[] and row[]
+// are the slot bits of the column and of the row number.
+struct TileMap {
+  uint8_t pa[16];
+  uint8_t col[8];
+  uint8_t row[8];
+};
+
+// LDS place of slot s: the low four bits (16 complex128 cover the banks once)
+// XORed with the next eight, so that 16 columns spread over the banks on
+// whatever slot bits they are.  Linear over XOR.
+__device__ __forceinline__ int tile_phys(int s) { return s ^ (((s >> 4) ^ (s >> 8)) & 15); }
+
+// K = 4..6 active targets, complex128, in place.  A workgroup stages a tile
+// through LDS and multiplies it by the 2^K x 2^K matrix: each of the 4 waves
+// holds 16 rows of it in registers for all its tiles and computes NCT blocks
+// of 16 columns.  The next tile's loads are in flight meanwhile.  Small tiles
+// (16 or 32 KiB) keep several workgroups per CU and fill the chip from 15
+// qubits on.  Bound by memory for K = 4 and 5, by the matrix cores' FP64 rate
+// for K = 6: 27 qubits, 6 targets 1.2 ms a gate (57 TFLOP/s, 3.6 TB/s), 29.6
+// ms with one thread per output; 5 targets on low qubits 0.80 ms, 1.17 ms in
+// k_gatek_staged; 15 qubits, 5 targets 4.9 us, 36 us in k_gatek.
+template <int K, int LC, bool kReal, bool kNT>
+__global__ __launch_bounds__(256, 2) void k_dense_tile(double2 *__restrict__ psi, uint64_t ntiles,
+                                                       Fixed fx, TileMap tm,
+                                                       const double2 *__restrict__ m) {
+  constexpr int D = 1 << K, S = 1 << (K + LC);
+  constexpr int RB = D / 16, CB = (1 << LC) / 16, NCT = RB * CB / 4;
+  constexpr int KS = D / 4, NL = S / 256;
+  static_assert(RB <= 4 && NCT >= 1, "four waves share the tile's blocks");
+  __shared__ double2 lds[S];
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r0 = 16 * (wave % RB), ct0 = (wave / RB) * NCT;
+  // this thread's slots are tid + 256 r
+  uint64_t lp = 0;
+#pragma unroll
+  for (int b = 0; b < 8; ++b)
+    if ((tid >> b) & 1) lp |= 1ull << tm.pa[b];
+  auto rp = [&](int r) {
+    uint64_t v = 0;
+#pragma unroll
+    for (int b = 0; b < K + LC - 8; ++b)
+      if ((r >> b) & 1) v |= 1ull << tm.pa[8 + b];
+    return v;
+  };
+  int lcol = 0;  // this lane's column and low row bits, as LDS places
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+    if ((c >> b) & 1) lcol |= 1 << tm.col[b];
+  int lrow = 0;
+#pragma unroll
+  for (int b = 0; b < 2; ++b)
+    if ((q >> b) & 1) lrow |= 1 << tm.row[b];
+  const int at = tile_phys(lcol | lrow);
+  auto row_at = [&](int s) {  // row bits from 2 up
+    int v = 0;
+#pragma unroll
+    for (int b = 0; b < K - 2; ++b)
+      if ((s >> b) & 1) v ^= tile_phys(1 << tm.row[2 + b]);
+    return v;
+  };
+  auto col_at = [&](int s) {  // column bits from 4 up
+    int v = 0;
+#pragma unroll
+    for (int b = 0; b < LC - 4; ++b)
+      if ((s >> b) & 1) v ^= tile_phys(1 << tm.col[4 + b]);
+    return v;
+  };
+  double ar[KS], ai[KS];
+#pragma unroll
+  for (int s = 0; s < KS; ++s) {
+    const double2 v = m[(r0 + c) * D + 4 * s + q];
+    ar[s] = v.x;
+    ai[s] = v.y;
+  }
+  double2 next[NL];
+  uint64_t t = blockIdx.x, base = 0;
+  if (t < ntiles) {
+    base = expand(t << LC, fx) | lp;
+#pragma unroll
+    for (int r = 0; r < NL; ++r) next[r] = ld<kNT>(psi + (base | rp(r)));
+  }
+  while (t < ntiles) {
+#pragma unroll
+    for (int r = 0; r < NL; ++r) lds[tile_phys(r * 256 + tid)] = next[r];
+    __syncthreads();
+    const uint64_t here = base;
+    t += gridDim.x;
+    if (t < ntiles) {
+      base = expand(t << LC, fx) | lp;
+#pragma unroll
+      for (int r = 0; r < NL; ++r) next[r] = ld<kNT>(psi + (base | rp(r)));
+    }
+    CplxAcc acc[NCT];
+#pragma unroll
+    for (int j = 0; j < NCT; ++j) acc[j].clear();
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int as = at ^ row_at(s);
+#pragma unroll
+      for (int j = 0; j < NCT; ++j) {
+        const double2 b = lds[as ^ col_at(ct0 + j)];
+        mfma_cplx<kReal>(acc[j], ar[s], ai[s], b);
+      }
+    }
+    __syncthreads();  // every wave has read the inputs
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int as = at ^ row_at(r0 / 4 + v);
+#pragma unroll
+      for (int j = 0; j < NCT; ++j) lds[as ^ col_at(ct0 + j)] = acc[j].at(v);
+    }
+    __syncthreads();
+    // (the next tile goes to the places that this thread reads here)
+#pragma unroll
+    for (int r = 0; r < NL; ++r) st<kNT>(psi + (here | rp(r)), lds[tile_phys(r * 256 + tid)]);
+  }
+}
+
+// Index bits of row or column number k of a matrix on the positions of ax.
+__device__ __forceinline__ uint64_t deposit(uint32_t k, int K, const Fixed &ax) {
+  uint64_t off = 0;
+  for (int b = 0; b < K; ++b)
+    if ((k >> b) & 1u) off |= 1ull << ax.pos[b];
+  return off;
+}
+
+// Any K >= 6, complex128: out of place from `src` (a copy of the state) into
+// psi, the product of the matrix and the 2^K x ngroups matrix of the groups.
+// A workgroup takes 16 rows and CT blocks of 16 columns, its NW waves a share
+// of the summed index each; their sums meet in LDS.  A wave's lanes
+// take the summed index in fours (lane l: 4 (l / 16) .. + 3 of every 16), so
+// that its matrix reads are 256-byte runs.  10 targets of 15 qubits (a 16 MiB
+// matrix): 27 us with 16 waves on 16 columns, 44 with 4, 55 with 4 on 32
+// columns, 904 with one thread per output; 10 targets of 22 qubits 0.7 ms
+// besides the matrix's upload, was 17.6.  Errors against 80-bit products are
+// a fifth to two thirds of those of one thread's chain (6 to 10 targets).
+template <int CT, int NW>
+__global__ __launch_bounds__(64 * NW) void k_dense_mm(double2 *__restrict__ psi,
+                                                  const double2 *__restrict__ src,
+                                                  uint64_t ngroups, int K, Fixed fx, Fixed ax,
+                                                  const double2 *__restrict__ m) {
+  __shared__ double2 part[NW][4][CT][64];
+  const uint32_t D = 1u << K;
+  const int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint64_t nrow = D / 16, ncol = (ngroups + 16 * CT - 1) / (16 * CT);
+  const uint64_t oq = deposit(4u * q, K, ax);
+  const uint64_t o1 = 1ull << ax.pos[0], o2 = 1ull << ax.pos[1];
+  const uint32_t k0 = wave * (D / NW), k1 = k0 + D / NW;
+  for (uint64_t tile = blockIdx.x; tile < nrow * ncol; tile += gridDim.x) {
+    const uint32_t r0 = (uint32_t)(tile % nrow) * 16;
+    const uint64_t g0 = (tile / nrow) * (16 * CT);
+    const double2 *col[CT];
+#pragma unroll
+    for (int j = 0; j < CT; ++j) {
+      const uint64_t g = g0 + 16 * j + c;  // past the last group: group 0, not stored
+      col[j] = src + (expand(g < ngroups ? g : 0, fx) | oq);
+    }
+    const double2 *row = m + (uint64_t)(r0 + c) * D + 4 * q;
+    CplxAcc acc[CT];
+#pragma unroll
+    for (int j = 0; j < CT; ++j) acc[j].clear();
+#pragma unroll 2
+    for (uint32_t k = k0; k < k1; k += 16) {
+      const uint64_t ok = deposit(k, K, ax);
+      double2 a[4], b[4][CT];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) a[s] = row[k + s];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+          b[s][j] = col[j][ok + ((s & 1) ? o1 : 0) + ((s & 2) ? o2 : 0)];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < CT; ++j) mfma_cplx<false>(acc[j], a[s].x, a[s].y, b[s][j]);
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+#pragma unroll
+      for (int j = 0; j < CT; ++j) part[wave][v][j][lane] = acc[j].at(v);
+    __syncthreads();
+    if (wave < 4) {  // rows 4 wave .. 4 wave + 3
+      const uint64_t out = deposit(r0 + 4u * wave + q, K, ax);
+#pragma unroll
+      for (int j = 0; j < CT; ++j) {
+        double2 s = part[0][wave][j][lane];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) {
+          s.x += part[w][wave][j][lane].x;
+          s.y += part[w][wave][j][lane].y;
+        }
+        const uint64_t g = g0 + 16 * j + c;
+        if (g < ngroups) psi[expand(g, fx) | out] = s;
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Any K >= 6, complex64: the same product with one chain of FMAs per output,
+// in the order of the summed index.  A workgroup takes 16 NR rows and 16 NC
+// columns in steps of 64 values of the index, a thread NR x NC outputs 16
+// apart.  In place (src == psi) when the rows are all of the matrix's: they
+// are stored after the only step has been read.  Bound by FP32 issue and LDS
+// reads: 27 qubits, 6 targets 1.4-1.7 ms, 25-28 ms with one thread per output.
+template <int NR, int NC>
+__global__ __launch_bounds__(256) void k_dense_f32(float2 *psi, const float2 *src,
+                                                   uint64_t ngroups, int K, Fixed fx, Fixed ax,
+                                                   const float2 *__restrict__ m) {
+  constexpr int TR = 16 * NR, TC = 16 * NC, KC = 64;
+  __shared__ float2 sa[KC][TR + 1];
+  __shared__ float2 sb[KC][TC];
+  __shared__ uint64_t soff[KC], sbase[TC];
+  const uint32_t D = 1u << K;
+  const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+  const uint64_t nrow = D / TR, ncol = (ngroups + TC - 1) / TC;
+  if (tid < KC) soff[tid] = deposit(tid, 6, ax);
+  for (uint64_t tile = blockIdx.x; tile < nrow * ncol; tile += gridDim.x) {
+    const uint32_t r0 = (uint32_t)(tile % nrow) * TR;
+    const uint64_t g0 = (tile / nrow) * TC;
+    if (tid < TC) sbase[tid] = expand(g0 + tid < ngroups ? g0 + tid : 0, fx);
+    float2 acc[NR][NC];
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+#pragma unroll
+      for (int j = 0; j < NC; ++j) acc[i][j] = czero<float2>();
+    for (uint32_t k0 = 0; k0 < D; k0 += KC) {
+      __syncthreads();
+      const uint64_t ok = deposit(k0, K, ax);
+      for (int e = tid; e < TR * KC; e += 256)
+        sa[e % KC][e / KC] = m[(uint64_t)(r0 + e / KC) * D + k0 + e % KC];
+      for (int e = tid; e < TC * KC; e += 256)
+        sb[e / TC][e % TC] = src[sbase[e % TC] | soff[e / TC] | ok];
+      __syncthreads();
+#pragma unroll 4
+      for (int k = 0; k < KC; ++k) {
+        float2 a[NR], b[NC];
+#pragma unroll
+        for (int i = 0; i < NR; ++i) a[i] = sa[k][ty + 16 * i];
+#pragma unroll
+        for (int j = 0; j < NC; ++j) b[j] = sb[k][tx + 16 * j];
+#pragma unroll
+        for (int i = 0; i < NR; ++i)
+#pragma unroll
+          for (int j = 0; j < NC; ++j) acc[i][j] = cmla(acc[i][j], a[i].x, a[i].y, b[j]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const uint64_t out = deposit(r0 + ty + 16 * i, K, ax);
+#pragma unroll
+      for (int j = 0; j < NC; ++j)
+        if (g0 + tx + 16 * j < ngroups) psi[sbase[tx + 16 * j] | out] = acc[i][j];
+    }
+    __syncthreads();
+  }
+}
+
+// Which kernel a dense gate on na >= 4 qubits takes, nfree index bits being
+// neither its targets nor its controls; low: a fixed bit among the lowest 4;
+// big: a streaming state.  Measured, complex128 (us per gate with its upload):
+//   5 qubits, 15-qubit state: tiles 10-11, k_gatek and its staged form 40;
+//   24 qubits: 80-100 against 114 (free low bits) and 156-184; 27 qubits:
+//   800 against 950-1160 (low bits fixed), but 870-1040 against 780-800 of
+//   k_gatek's long runs (low bits free), which it keeps.
+//   4 qubits: 9.5 against 13-19 up to 18 qubits, 75 against 81-87 at 24; at
+//   28 qubits 1580-1850 against 1460-1600, so streaming states keep theirs.
+//   6 qubits: 32 columns per tile from 20 qubits on (33 against 37 at 20, 67
+//   against 74 at 22, 1200 against 1240 at 27), 16 below (24 against 26).
+// Larger products take 32 columns per workgroup when that still fills the
+// chip.  Complex64: 64 x 64 outputs per workgroup from 20 qubits on.
+enum DenseForm { kDenseDirect, kDenseTile, kDenseTileSmall, kDenseWide, kDenseNarrow };
+
+static DenseForm dense_form(bool c64, int na, int nfree, bool low, bool big) {
+  if (c64) {
+    if (na <= 5) return kDenseDirect;
+    return nfree >= 6 && na + nfree >= 20 ? kDenseWide : kDenseNarrow;
+  }
+  if (na == 4) return nfree >= 6 && !big ? kDenseTile : kDenseDirect;
+  if (na == 5) return nfree >= 5 && (low || !big) ? kDenseTile : kDenseDirect;
+  if (na == 6 && nfree >= 4) return nfree < 14 ? kDenseTileSmall : kDenseTile;
+  return nfree >= 5 && na + nfree >= 17 ? kDenseWide : kDenseNarrow;
+}
+
+bool dense_needs_scratch(bool c64, int n, const Gate &g) {
+  if (g.na <= 5) return false;
+  const Fixed fx = make_fixed(g.cmask | active_mask(g), g.cval);
+  const DenseForm f = dense_form(c64, g.na, n - fx.nf, false, false);
+  if (c64) return !(g.na == 6 && f == kDenseWide);
+  return f != kDenseTile && f != kDenseTileSmall;
+}
+
+static TileMap tile_map(const Fixed &fx, const Fixed &ax, int lc) {
+  const uint64_t fixed = fx_mask(fx);
+  TileMap tm{};
+  int slot = 0, col = 0;
+  for (int q = 0; q < 64; ++q) {
+    int row = -1;
+    for (int j = 0; j < ax.nf; ++j)
+      if (ax.pos[j] == q) row = j;
+    if (row < 0 && (((fixed >> q) & 1ull) || col == lc)) continue;
+    if (row >= 0) tm.row[row] = (uint8_t)slot;
+    else tm.col[col++] = (uint8_t)slot;
+    tm.pa[slot++] = (uint8_t)q;
+  }
+  return tm;
+}
+
+template <int K, int LC>
+static void launch_dense_tile(double2 *psi, int nfree, const Fixed &fx, const Fixed &ax, bool real,
+                              bool big, const double2 *m, hipStream_t s) {
+  const TileMap tm = tile_map(fx, ax, LC);
+  const uint64_t ntiles = 1ull << (nfree - LC);
+  constexpr uint64_t kPerCU = K + LC == 11 ? 4 : 8;
+  const unsigned grid = (unsigned)std::min<uint64_t>(ntiles, 256 * kPerCU);
+  nt_dispatch(big, [&](auto nt) {
+    if (K <= 5 && real)
+      hipLaunchKernelGGL((k_dense_tile<K, LC, K <= 5, decltype(nt)::value>), dim3(grid),
+                         dim3(256), 0, s, psi, ntiles, fx, tm, m);
+    else
+      hipLaunchKernelGGL((k_dense_tile<K, LC, false, decltype(nt)::value>), dim3(grid), dim3(256),
+                         0, s, psi, ntiles, fx, tm, m);
+  });
+}
+
 // Calls f(integral_constant K, integral_constant real) for K = na in 3..5.
 template <typename F>
 static void gatek_dispatch(int na, bool real, F &&f) {
@@ -799,7 +1128,7 @@ static void gatek_dispatch(int na, bool real, F &&f) {
 }
 
 // d_mat layout: row-major D x D {re, im} in precision R.  `scratch` (2^n amplitudes) is needed
-// only when K > 5.
+// where dense_needs_scratch says so.
 template <typename R>
 hipError_t launch_gate_dense(void *psi_v, int n, const Gate &g, void *d_mat, void *scratch,
                              hipStream_t s) {
@@ -892,6 +1221,16 @@ hipError_t launch_gate_dense(void *psi_v, int n, const Gate &g, void *d_mat, voi
     const R *m = (const R *)d_mat;  // row-major {re, im}
     bool real = true;
     for (const cd &v : g.m) real = real && v.im == 0.0;
+    if constexpr (std::is_same<R, double>::value) {
+      if (g.na >= 4 &&
+          dense_form(false, g.na, nfree, (fx_mask(fx) & 0xFull) != 0, big) == kDenseTile) {
+        if (g.na == 4)
+          launch_dense_tile<4, 6>(psi, nfree, fx, ax, real, big, (const double2 *)m, s);
+        else
+          launch_dense_tile<5, 5>(psi, nfree, fx, ax, real, big, (const double2 *)m, s);
+        return hipGetLastError();
+      }
+    }
     StageMap sm{};
     // fixed low bits (active or control on qubits 0..3) break the direct
     // kernel's 64-amplitude runs: stage through LDS instead
@@ -899,9 +1238,11 @@ hipError_t launch_gate_dense(void *psi_v, int n, const Gate &g, void *d_mat, voi
       const unsigned sgrid = (unsigned)(nfreeN / 64);
       auto staged = [&](auto kk, auto rr) {
         nt_dispatch(big, [&](auto nt) {
-          hipLaunchKernelGGL((k_gatek_staged<R, decltype(kk)::value, decltype(rr)::value,
-                                             decltype(nt)::value>),
-                             dim3(sgrid), dim3(64), 0, s, psi, nfreeN, fx, sm, m);
+          // (complex128 blocks of 5 qubits on low bits are tiles)
+          if constexpr (!(std::is_same<R, double>::value && decltype(kk)::value == 5))
+            hipLaunchKernelGGL((k_gatek_staged<R, decltype(kk)::value, decltype(rr)::value,
+                                               decltype(nt)::value>),
+                               dim3(sgrid), dim3(64), 0, s, psi, nfreeN, fx, sm, m);
         });
       };
       gatek_dispatch(g.na, real, staged);
@@ -936,12 +1277,40 @@ hipError_t launch_gate_dense(void *psi_v, int n, const Gate &g, void *d_mat, voi
     gatek_dispatch(g.na, real, direct);
   } else {
     const Fixed ax = active_positions(g);
-    hipError_t e = hipMemcpyAsync(scratch, psi, sizeof(T) << n, hipMemcpyDeviceToDevice, s);
-    if (e != hipSuccess) return e;
-    unsigned grid = grid_for(nfreeN << g.na, kBlock);
-    if (grid > 65536) grid = 65536;
-    hipLaunchKernelGGL(k_gate_big<R>, dim3(grid), dim3(kBlock), 0, s, psi, (const T *)scratch,
-                       nfreeN, g.na, fx, ax, (const T *)d_mat);
+    const T *m = (const T *)d_mat;
+    const DenseForm f = dense_form(std::is_same<R, float>::value, g.na, nfree, false, big);
+    const T *src = psi;
+    if (dense_needs_scratch(std::is_same<R, float>::value, n, g)) {
+      hipError_t e = hipMemcpyAsync(scratch, psi, sizeof(T) << n, hipMemcpyDeviceToDevice, s);
+      if (e != hipSuccess) return e;
+      src = (const T *)scratch;
+    }
+    const auto grid = [&](uint64_t rows, uint64_t cols) {
+      return dim3((unsigned)std::min<uint64_t>(
+          ((1ull << g.na) / rows) * ((nfreeN + cols - 1) / cols), 65536));
+    };
+    if constexpr (std::is_same<R, double>::value) {
+      if (f == kDenseTile)
+        launch_dense_tile<6, 5>(psi, nfree, fx, ax, false, big, m, s);
+      else if (f == kDenseTileSmall)
+        launch_dense_tile<6, 4>(psi, nfree, fx, ax, false, big, m, s);
+      else if (f == kDenseWide)
+        hipLaunchKernelGGL((k_dense_mm<2, 4>), grid(16, 32), dim3(256), 0, s, psi, src, nfreeN,
+                           g.na, fx, ax, m);
+      else if (g.na >= 8)  // a share is at least 16 of the 2^na values
+        hipLaunchKernelGGL((k_dense_mm<1, 16>), grid(16, 16), dim3(1024), 0, s, psi, src, nfreeN,
+                           g.na, fx, ax, m);
+      else
+        hipLaunchKernelGGL((k_dense_mm<1, 4>), grid(16, 16), dim3(256), 0, s, psi, src, nfreeN,
+                           g.na, fx, ax, m);
+    } else {
+      if (f == kDenseWide)
+        hipLaunchKernelGGL((k_dense_f32<4, 4>), grid(64, 64), dim3(256), 0, s, psi, src, nfreeN,
+                           g.na, fx, ax, m);
+      else
+        hipLaunchKernelGGL((k_dense_f32<1, 1>), grid(16, 16), dim3(256), 0, s, psi, src, nfreeN,
+                           g.na, fx, ax, m);
+    }
   }
   return hipGetLastError();
 }

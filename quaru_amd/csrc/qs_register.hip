@@ -589,7 +589,7 @@ hipError_t launch_one(qs_register *r, const Gate &g) {
         e = bytes + 256 <= r->ring_cap ? ring_upload(r, src, bytes, &dm)
                                        : big_upload(r, src, bytes, &dm);
         if (e != hipSuccess) return e;
-        if (g.na > 5 && !r->scratch) {
+        if (!r->scratch && qs::dense_needs_scratch(std::is_same<T, float>::value, r->n, g)) {
           e = qs::pool_malloc(&r->scratch, r->state_bytes());
           if (e != hipSuccess) return e;
         }

@@ -158,6 +158,36 @@ def test_block_gates_low_and_high_targets(dtype, real):
         assert infid(r.state, ref) < 1e-6
 
 
+@pytest.mark.parametrize("dtype, k, n", [
+    ("c128", 5, 9), ("c128", 5, 10), ("c128", 5, 15), ("c128", 5, 21), ("c128", 6, 9),
+    ("c128", 6, 10), ("c128", 6, 12), ("c128", 6, 21), ("c128", 7, 7), ("c128", 7, 13),
+    ("c128", 8, 8), ("c128", 8, 12), ("c128", 8, 17), ("c64", 6, 6), ("c64", 6, 9), ("c64", 6, 14), ("c64", 6, 20),
+    ("c64", 7, 20)])
+def test_dense_blocks_of_every_form(dtype, k, n):
+    """Dense blocks on the matrix cores and in complex64, from one group of
+    amplitudes to several tiles per workgroup: on the lowest qubits, on the
+    highest in reverse, on any, real, and under controls between them."""
+    rng = np.random.default_rng(1000 + 50 * k + n)
+    sets = [list(range(k)), list(range(n - k, n))[::-1], [int(x) for x in rng.permutation(n)[:k]]]
+    opl = [ops.Operation(random_unitary(rng, 1 << k), t) for t in sets]
+    opl.append(ops.Operation(random_orthogonal(rng, 1 << k), sets[2]))
+    for c in (1, 2):
+        if n >= k + c:
+            t = [int(x) for x in rng.permutation(n)[:k + c]]
+            opl.append(ops.Operation.controlled(t[k:], random_unitary(rng, 1 << k), t[:k],
+                                                control_values=[False, True][:c]))
+    psi0 = random_state(rng, n)
+    ref = oracle_run(psi0.copy(), opl)
+    r = Register.new([False] * n, dtype)
+    r.state = psi0
+    for op in opl:
+        r.apply(op)
+    if dtype == "c128":
+        assert maxdiff(r.state, ref) < TOL
+    else:
+        assert infid(r.state, ref) < 1e-6
+
+
 @pytest.mark.parametrize("n", [12, 14])
 def test_c64_complex_5q_blocks_matrix_cores(n):
     """Complex 32 x 32 blocks in complex64 with the 5 lowest index bits free
