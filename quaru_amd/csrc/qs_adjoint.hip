@@ -1287,11 +1287,23 @@ int forward_sweeps(qs_adjoint *c, const double *thetas) {
     }
     return apply_fixed<R>(c, c->psi, g, tab);
   };
+  // every state of the batch starts as |0...0>
+  const uint64_t total = B << n;
+  run.fresh = true;
+  run.known = (1ull << n) - 1ull;
+  run.fill = [c, n, ntot, total, &run]() -> hipError_t {
+    if (!run.fresh) return qs::launch_zero_outside<R>(c->psi, ntot, run.known, 0, c->stream);
+    hipLaunchKernelGGL(k_init_zero_states<R>, dim3(grid_of(total, kBlock * 4)), dim3(kBlock), 0,
+                       c->stream, (T *)c->psi, n, total);
+    return hipGetLastError();
+  };
   std::vector<qs::Gate> gates;
   size_t layer = 0;
   auto flush = [&]() -> int {
-    if (gates.empty()) return QS_OK;
-    hipError_t e2 = qs::sweep_execute(c->engine, run, gates, &c->sweeps, &c->kernels);
+    hipError_t e2 = hipSuccess;
+    if (!gates.empty())
+      e2 = qs::sweep_execute(c->engine, run, gates, &c->sweeps, &c->kernels);
+    if (e2 == hipSuccess) e2 = qs::sweep_settle(run);
     gates.clear();
     if (e2 != hipSuccess) return qs::set_hip_error(e2, "adjoint forward sweeps");
     return QS_OK;
@@ -1418,13 +1430,14 @@ int forward_t(qs_adjoint *c, const double *thetas, const uint64_t *masks, const 
     AJ(c->take(&c->d_gmat, tab.size() * sizeof(R)));
     AJ(upload_to(c, tab.data(), tab.size() * sizeof(R), c->d_gmat));
   }
-  hipLaunchKernelGGL(k_init_zero_states<R>, dim3(grid_of(total, kBlock * 4)), dim3(kBlock), 0,
-                     c->stream, (T *)c->psi, n, total);
-  AJ(hipGetLastError());
   const uint64_t pps = 1ull << (n - 1);
   if (adjoint_sweeps()) {
     const int rc = forward_sweeps<R>(c, thetas);
     if (rc != QS_OK) return rc;
+  } else {
+    hipLaunchKernelGGL(k_init_zero_states<R>, dim3(grid_of(total, kBlock * 4)), dim3(kBlock), 0,
+                       c->stream, (T *)c->psi, n, total);
+    AJ(hipGetLastError());
   }
   size_t layer = 0;
   for (size_t i = 0; i < c->circ.ops.size() && !adjoint_sweeps(); ++i) {

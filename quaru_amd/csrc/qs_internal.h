@@ -100,6 +100,9 @@ int set_hip_error(hipError_t e, const char *where);
 // All launches go to `s`; `psi` is the device state of 2^n amplitudes.
 template <typename R>
 hipError_t launch_init_basis(void *psi, int n, uint64_t k, hipStream_t s);
+// Zero the amplitudes i with (i & mask) != val.
+template <typename R>
+hipError_t launch_zero_outside(void *psi, int n, uint64_t mask, uint64_t val, hipStream_t s);
 template <typename R>
 hipError_t launch_init_product(void *psi, int n, const double *d_qubits, hipStream_t s);
 template <typename R>

@@ -140,6 +140,15 @@ __global__ __launch_bounds__(kBlock) void k_init_basis(typename V2<R>::T *psi, u
   }
 }
 
+template <typename R>
+__global__ __launch_bounds__(kBlock) void k_zero_outside(typename V2<R>::T *psi, uint64_t len,
+                                                         uint64_t mask, uint64_t val) {
+  using T = typename V2<R>::T;
+  for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < len;
+       i += (uint64_t)gridDim.x * kBlock)
+    if ((i & mask) != val) psi[i] = czero<T>();
+}
+
 // Product state in the order of the kron fold of Register::new /
 // try_from_qubits (src/register.rs:47-50, :94-96): amp = b_{n-1} * (... *
 // (b_0 * 1)).
@@ -173,6 +182,16 @@ hipError_t launch_init_basis(void *psi, int n, uint64_t k, hipStream_t s) {
   if (g > 65536) g = 65536;
   hipLaunchKernelGGL(k_init_basis<R>, dim3(g), dim3(kBlock), 0, s,
                      (typename V2<R>::T *)psi, len, k);
+  return hipGetLastError();
+}
+
+template <typename R>
+hipError_t launch_zero_outside(void *psi, int n, uint64_t mask, uint64_t val, hipStream_t s) {
+  const uint64_t len = 1ull << n;
+  unsigned g = grid_for(len, kBlock * 8);
+  if (g > 65536) g = 65536;
+  hipLaunchKernelGGL(k_zero_outside<R>, dim3(g), dim3(kBlock), 0, s, (typename V2<R>::T *)psi,
+                     len, mask, val);
   return hipGetLastError();
 }
 
@@ -2292,6 +2311,7 @@ hipError_t launch_chunk_sums(const void *psi, int n, uint64_t chunk, double *d_o
 #define QS_INSTANTIATE(R)                                                                        \
   template hipError_t launch_init_basis<R>(void *, int, uint64_t, hipStream_t);                 \
   template hipError_t launch_init_product<R>(void *, int, const double *, hipStream_t);         \
+  template hipError_t launch_zero_outside<R>(void *, int, uint64_t, uint64_t, hipStream_t);     \
   template hipError_t launch_gate_dense<R>(void *, int, const Gate &, void *, void *,            \
                                            hipStream_t);                                         \
   template hipError_t launch_gate_diag<R>(void *, int, const Gate &, void *, hipStream_t);      \

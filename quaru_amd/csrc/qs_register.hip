@@ -88,6 +88,9 @@ struct qs_register {
   // the collapse of the last measure, not yet launched: the next measure
   // runs it fused with its own probability split; anything else launches it
   // first (settle)
+  // the state is |basis_k>, not yet written: the first flush starts from it
+  bool basis = false;
+  uint64_t basis_k = 0;
   bool coll_pending = false;
   int coll_target = 0, coll_keep = 0;
   double coll_total = 1.0;
@@ -680,11 +683,24 @@ int settle(qs_register *r) {
   return QS_OK;
 }
 
+// Write the basis state that the register starts from, if it has not been.
+hipError_t write_basis(qs_register *r) {
+  if (!r->basis) return hipSuccess;
+  r->basis = false;
+  return by_dtype(r, [&](auto z) {
+    return qs::launch_init_basis<decltype(z)>(r->psi, r->n, r->basis_k, r->stream);
+  });
+}
+
 // Apply the pending collapse, then every pending gate: through the sweep
 // engine when fusion is on, otherwise one kernel per gate.
 int flush(qs_register *r) {
   int rc = settle(r);
   if (rc) return rc;
+  if (r->pending.empty() || !r->fusion) {
+    const hipError_t e = write_basis(r);
+    if (e != hipSuccess) return hip_fail(e, "writing the basis state");
+  }
   if (r->pending.empty()) return QS_OK;
   std::vector<Gate> gates;
   gates.swap(r->pending);
@@ -703,7 +719,22 @@ int flush(qs_register *r) {
     if (r->timing) run.mark = [r](bool begin) { mark(r, QS_K_SWEEP, begin); };
     run.sweep_ops = &r->st_sweep_ops;
     run.merged = &r->st_merged;
+    if (r->basis) {
+      run.fresh = true;
+      run.known = r->len - 1;
+      run.known_val = r->basis_k;
+      run.fill = [r, &run] {
+        if (run.fresh) return write_basis(r);
+        return by_dtype(r, [&](auto z) {
+          return qs::launch_zero_outside<decltype(z)>(r->psi, r->n, run.known, run.known_val,
+                                                      r->stream);
+        });
+      };
+    }
     e = qs::sweep_execute(r->engine, run, gates, &r->st_sweeps, &r->st_kernels);
+    const hipError_t e2 = qs::sweep_settle(run);
+    r->basis = false;
+    if (e == hipSuccess) e = e2;
   } else {
     for (const Gate &g : gates) {
       e = launch_gate(r, g);
@@ -990,14 +1021,8 @@ int qs_register_new(const unsigned char *bits, size_t n, int dtype, qs_register 
   for (size_t i = 0; i < n; ++i)
     if (bits[i]) k |= 1ull << i;
   qs_register *r = *out;
-  hipError_t e = by_dtype(r, [&](auto z) {
-    return qs::launch_init_basis<decltype(z)>(r->psi, r->n, k, r->stream);
-  });
-  if (e != hipSuccess) {
-    qs_register_free(r);
-    *out = nullptr;
-    return hip_fail(e, "qs_register_new");
-  }
+  r->basis = true;
+  r->basis_k = k;
   return QS_OK;
 }
 
@@ -1007,14 +1032,8 @@ int qs_register_from_int(size_t n, size_t k, int dtype, qs_register **out) {
   int rc = alloc_register(n, dtype, out);
   if (rc) return rc;
   qs_register *r = *out;
-  hipError_t e = by_dtype(r, [&](auto z) {
-    return qs::launch_init_basis<decltype(z)>(r->psi, r->n, k, r->stream);
-  });
-  if (e != hipSuccess) {
-    qs_register_free(r);
-    *out = nullptr;
-    return hip_fail(e, "qs_register_from_int");
-  }
+  r->basis = true;
+  r->basis_k = k;
   return QS_OK;
 }
 
@@ -1213,7 +1232,7 @@ int qs_measure(qs_register *r, size_t target, double uniform, int *result) {
   if (target >= (size_t)r->n) return fail(QS_INVALID_TARGET, target, 0, "target out of range");
   // a collapse left by the previous measure stays pending (the split fuses
   // it) unless gates were applied since: then it goes first, then the gates
-  if (!r->pending.empty()) {
+  if (!r->pending.empty() || r->basis) {
     int rc = flush(r);
     if (rc) return rc;
   }
@@ -1372,9 +1391,17 @@ int qs_get_state(qs_register *r, double *out) {
 
 int qs_set_state(qs_register *r, const double *in) {
   if (!r || !in) return fail(QS_ERR_ARGUMENT, 0, 0, "NULL argument");
-  int rc = sync(r);
-  if (rc) return rc;
+  // (a basis state that nothing has been applied to is not written first)
+  const bool over = r->basis && r->pending.empty();
+  const auto whole = [&] {
+    if (over) r->basis = false;
+  };
+  if (!over) {
+    int rc = sync(r);
+    if (rc) return rc;
+  }
   if (r->dtype == QS_C128) {
+    whole();
     QS_HIP(hipMemcpyAsync(r->psi, in, r->state_bytes(), hipMemcpyHostToDevice, r->stream));
     QS_HIP(hipStreamSynchronize(r->stream));
     return QS_OK;
@@ -1382,6 +1409,7 @@ int qs_set_state(qs_register *r, const double *in) {
   const uint64_t step = std::min<uint64_t>(r->len, kReadoutAmps);
   double *d = nullptr;
   QS_HIP(ensure_big(r, step * 2 * sizeof(double), &d));
+  whole();
   for (uint64_t off = 0; off < r->len; off += step) {
     const uint64_t cnt = std::min<uint64_t>(step, r->len - off);
     hipError_t e = hipMemcpyAsync(d, in + 2 * off, cnt * 2 * sizeof(double),

@@ -98,14 +98,18 @@ __device__ __forceinline__ void small_2x2(const SmallPass<R> &p, int j, uint32_t
 template <typename R>
 __global__ __launch_bounds__(kSmallThreads) void k_small(typename sweep::SV2<R>::T *__restrict__ psi,
                                                          int n, const SmallPass<R> *__restrict__ prog,
-                                                         int npass) {
+                                                         int npass, uint32_t basis) {
   using T = typename sweep::SV2<R>::T;
   extern __shared__ unsigned char small_smem[];
   T *s = (T *)small_smem;
   const uint32_t N = 1u << n;
   SmallPass<R> *chunk = (SmallPass<R> *)(small_smem + (size_t)N * sizeof(T));
   const uint32_t tid = threadIdx.x, nt = blockDim.x;
-  for (uint32_t i = tid; i < N; i += nt) s[small_pos(i)] = psi[i];
+  // (basis < 2^n: the state is that basis state and not in memory yet)
+  if (basis < N)
+    for (uint32_t i = tid; i < N; i += nt) s[small_pos(i)] = T{(R)(i == basis), 0};
+  else
+    for (uint32_t i = tid; i < N; i += nt) s[small_pos(i)] = psi[i];
   constexpr int CP = kChunkPasses<R>;
   constexpr uint32_t kWords = CP * sizeof(SmallPass<R>) / 16;
   const uint4 *src = reinterpret_cast<const uint4 *>(prog);
@@ -296,10 +300,15 @@ hipError_t execute_small_t(SweepRunner &run, const std::vector<Gate> &gates, uin
     const unsigned threads = (unsigned)std::min(kSmallThreads, std::max(64, 1 << (n - 2)));
     if (run.mark) run.mark(true);
     hipLaunchKernelGGL(k_small<R>, dim3(1), dim3(threads), lds, run.stream, (T *)run.psi, n,
-                       (const SmallPass<R> *)d, (int)b.prog.size());
+                       (const SmallPass<R> *)d, (int)b.prog.size(),
+                       run.fresh ? (uint32_t)run.known_val : ~0u);
     if (run.mark) run.mark(false);
     e = hipGetLastError();
-    if (e == hipSuccess) ++*sweeps;
+    if (e == hipSuccess) {
+      ++*sweeps;
+      run.known = run.known_val = 0;
+      run.fresh = false;
+    }
     b.prog.clear();
     b.open = false;
     return e;
@@ -312,6 +321,7 @@ hipError_t execute_small_t(SweepRunner &run, const std::vector<Gate> &gates, uin
   for (size_t at = 0; at < gates.size();) {
     if (!Builder<R>::takes(gates[at])) {
       hipError_t e = launch();
+      if (e == hipSuccess) e = sweep_settle(run);
       if (e == hipSuccess) e = run.single(gates[at]);
       if (e != hipSuccess) return e;
       ++at;

@@ -38,6 +38,15 @@ struct SweepRunner {
   size_t states = 0;
   // Whether a state that fits one compute unit may run there (qs_small.hip).
   bool small = false;
+  // A state that starts as one basis state: only amplitudes i with (i &
+  // known) == known_val can be nonzero and are in memory (fresh: not even
+  // those yet, they are 1); sweeps pass over these only, and read and write
+  // what they make of them.  fill writes the rest (fresh: everything), before
+  // whatever else uses the state; sweep_execute leaves that of the end to
+  // sweep_settle.
+  uint64_t known = 0, known_val = 0;
+  bool fresh = false;
+  std::function<hipError_t()> fill;
   hipStream_t stream = nullptr;
   // Copy host bytes to a device buffer that stays valid until the stream
   // reaches the next launch.
@@ -61,6 +70,9 @@ struct SweepRunner {
 // per-gate kernels.  Counters are incremented by the launches made.
 hipError_t sweep_execute(SweepEngine *e, SweepRunner &run, const std::vector<Gate> &gates,
                          uint64_t *sweeps, uint64_t *kernels);
+
+// Write the amplitudes that run.known leaves out, if any.
+hipError_t sweep_settle(SweepRunner &run);
 
 // Registers whose state fits one compute unit's LDS run their gates there, in
 // one launch for any run of them (qs_small.hip); whether this one does.

@@ -336,6 +336,13 @@ hipError_t launch_sweep_a(int A, int W, SweepRunner &run, const void *d_blob, ui
   }
 }
 
+bool all_finite(const std::vector<Gate> &gates, const std::vector<int> &which) {
+  for (int gi : which)
+    for (const cd &v : gates[gi].m)
+      if (!std::isfinite(v.re) || !std::isfinite(v.im)) return false;
+  return true;
+}
+
 template <typename R>
 hipError_t execute_t(SweepRunner &run, const std::vector<Gate> &gates, uint64_t *sweeps) {
   const int n = run.n;
@@ -352,7 +359,8 @@ hipError_t execute_t(SweepRunner &run, const std::vector<Gate> &gates, uint64_t 
     if (g.bmask) nt = std::min(nt, g.bshift);
   if (nt < T) {
     for (const Gate &g : gates) {
-      hipError_t e = run.single(g);
+      hipError_t e = sweep_settle(run);
+      if (e == hipSuccess) e = run.single(g);
       if (e != hipSuccess) return e;
     }
     return hipSuccess;
@@ -386,7 +394,8 @@ hipError_t execute_t(SweepRunner &run, const std::vector<Gate> &gates, uint64_t 
     while (first < G && done[first]) ++first;
     if (first == G) break;
     if (!sweepable(gates[first], lowb)) {
-      hipError_t e = run.single(gates[first]);
+      hipError_t e = sweep_settle(run);
+      if (e == hipSuccess) e = run.single(gates[first]);
       if (e != hipSuccess) return e;
       done[first] = 1;
       continue;
@@ -586,7 +595,8 @@ hipError_t execute_t(SweepRunner &run, const std::vector<Gate> &gates, uint64_t 
     for (int gi : pl.gates) single_cost += single_amps(gates[gi], n);
     if (single_cost <= std::ldexp(1.0, n)) {
       for (int gi : pl.gates) {
-        hipError_t e = run.single(gates[gi]);
+        hipError_t e = sweep_settle(run);
+        if (e == hipSuccess) e = run.single(gates[gi]);
         if (e != hipSuccess) return e;
       }
       continue;
@@ -695,8 +705,32 @@ hipError_t execute_t(SweepRunner &run, const std::vector<Gate> &gates, uint64_t 
       std::fprintf(stderr, " ops %u\n", h.nops);
     }
     h.npool = (uint32_t)pool.size();
+    if ((run.known || run.fresh) && !all_finite(gates, pl.gates)) {
+      // (an infinity or NaN makes more of the zeros than zeros)
+      hipError_t e = sweep_settle(run);
+      if (e != hipSuccess) return e;
+    }
+    int kept = 0;  // index bits outside the tile that keep their value
+    if (run.known || run.fresh) {
+      for (int q = 0, rank = 0; q < n; ++q) {
+        if ((P >> q) & 1ull) continue;
+        if ((run.known >> q) & 1ull) {
+          h.kmask |= 1ull << rank;
+          ++kept;
+        }
+        ++rank;
+      }
+      h.kset = run.known & run.known_val & ~P;
+      h.pmask = run.known & P;
+      h.pval = h.pmask & run.known_val;
+      h.start = run.fresh ? START_BASIS : (h.pmask ? START_PART : START_FULL);
+      run.fresh = false;
+      for (int gi : pl.gates) run.known &= ~gx[gi];
+      run.known_val &= run.known;
+    }
     // the padding states of a batch are the last tiles: they are left out
-    h.ntiles = run.states && nt < n ? (uint64_t)run.states << (nt - T) : 1ull << (n - T);
+    h.ntiles = run.states && nt < n ? (uint64_t)run.states << (nt - T - kept)
+                                    : 1ull << (n - T - kept);
     const size_t hbytes = (sizeof(SweepHeader) + 15) & ~(size_t)15;
     const size_t bbytes = blob_bytes<R>((int)h.nops, (int)h.npool);
     blob.assign(bbytes, 0);
@@ -788,6 +822,14 @@ bool sweep_xcd_chunks() {
 int sweep_reg_bits(bool c64) {
   const int a = env_int(c64 ? "QS_SWEEP_A_C64" : "QS_SWEEP_A_C128", c64 ? 5 : 4);
   return std::min(5, std::max(3, a));
+}
+
+hipError_t sweep_settle(SweepRunner &run) {
+  if (!run.known && !run.fresh) return hipSuccess;
+  const hipError_t e = run.fill();
+  run.known = run.known_val = 0;
+  run.fresh = false;
+  return e;
 }
 
 hipError_t sweep_execute(SweepEngine *eng, SweepRunner &run, const std::vector<Gate> &gates,

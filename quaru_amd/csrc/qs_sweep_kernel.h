@@ -168,8 +168,22 @@ struct SweepHeader {
   uint64_t gb[8];     // global bit of register slot j
   uint64_t lg[8];     // global bit of lane bit i (i < 6)
   uint64_t wb[2];     // global bit of wave bit k (k < nwave)
-  uint32_t nwave, pad;
+  uint32_t nwave;
+  // A state that starts as one basis state: qubits that no op has changed
+  // yet keep their value, and every other amplitude is zero and not in
+  // memory.  Tile ids enumerate the free bits outside the tile only: kmask
+  // marks the kept ones among the bits outside the tile (bit i: the i-th
+  // lowest), kset their values (index bits).  start = START_PART: of the tile
+  // itself, only amplitudes whose kept bits (pmask) are pval are read, the
+  // others are zero; START_BASIS: those are one instead of read.
+  // The first sweeps of a program then cost 2^12 and about 2^21 amplitudes,
+  // the third one's reads are of what those left, and the state is not
+  // zeroed first: 30 qubits 408 ms, 428 with all of them in full (complex64
+  // 211, 219), 27 qubits with three sweeps of Hadamards 7.9 ms, 9.9.
+  uint32_t start;
+  uint64_t kmask, kset, pmask, pval;
 };
+enum : uint32_t { START_FULL = 0, START_PART = 1, START_BASIS = 2 };
 
 template <typename R>
 __host__ __device__ inline size_t blob_bytes(int nops, int npool) {
@@ -1162,7 +1176,12 @@ __device__ __forceinline__ void sweep_tile(typename SV2<R>::T *__restrict__ psi,
   if (tile >= h.ntiles) return;  // whole waves (W = 0) or whole workgroups
   const Regs<A, I> g = reg_bits<A, I>(h);
   Ctx<I> c;
-  c.tbase = (I)tile_base<T>(tile, h);
+  uint64_t id = tile;
+  for (uint64_t m = h.kmask; m; m &= m - 1) {
+    const uint64_t lo = id & ((m & (0 - m)) - 1ull);
+    id = ((id ^ lo) << 1) | lo;
+  }
+  c.tbase = (I)(tile_base<T>(id, h) | h.kset);
   c.gbase = c.tbase | lane_offset<I>(h, lane) | wave_offset<W, I>(h, wave);
   c.wave = wave;
   c.lane = lane;
@@ -1170,8 +1189,24 @@ __device__ __forceinline__ void sweep_tile(typename SV2<R>::T *__restrict__ psi,
   {
     typename SNT<R>::T v[NA];
     const typename SNT<R>::T *src = reinterpret_cast<const typename SNT<R>::T *>(psi);
+    if (h.start == START_FULL) {
 #pragma unroll
-    for (int r = 0; r < NA; ++r) v[r] = __builtin_nontemporal_load(src + (c.gbase | goff<A>(g, r)));
+      for (int r = 0; r < NA; ++r)
+        v[r] = __builtin_nontemporal_load(src + (c.gbase | goff<A>(g, r)));
+    } else {
+      const I pm = (I)h.pmask, pv = (I)h.pval;
+      const bool on = (c.gbase & pm & ~g.mask) == (pv & ~g.mask);
+#pragma unroll
+      for (int r = 0; r < NA; ++r) {
+        v[r] = typename SNT<R>::T{0, 0};
+        if (on && (goff<A>(g, r) & pm) == (pv & g.mask)) {
+          if (h.start == START_BASIS)
+            v[r].x = 1;
+          else
+            v[r] = __builtin_nontemporal_load(src + (c.gbase | goff<A>(g, r)));
+        }
+      }
+    }
 #pragma unroll
     for (int r = 0; r < NA; ++r) {
       a.re[r] = v[r].x;

@@ -158,6 +158,44 @@ def test_block_gates_low_and_high_targets(dtype, real):
         assert infid(r.state, ref) < 1e-6
 
 
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+@pytest.mark.parametrize("n", [2, 6, 11, 12, 13, 14, 17, 22])
+def test_gates_from_a_basis_state(n, dtype):
+    """A new register's gates run on the part of the state that they reach;
+    one given the same basis state amplitude by amplitude runs on all of it:
+    equal states after gates on some of the qubits, controls and phases on
+    untouched ones, a random circuit, and before any gate."""
+    rng = np.random.default_rng(300 + n)
+    k = int(rng.integers(0, 1 << n))
+    e = np.zeros(1 << n, dtype=np.complex128)
+    e[k] = 1
+    q = [int(x) for x in rng.permutation(n)]
+    some = [ops.Operation(random_unitary(rng, 2), [t]) for t in q[: max(1, n // 3)]]
+    ties = [ops.cnot(a, b) for a, b in zip(q, q[1:])] + [ops.phase(t) for t in q]
+    few = [ops.cnot(q[-1], q[0]), ops.Operation(random_unitary(rng, 4), [q[0], q[1]])]
+    lists = [[], some, some + ties[: n // 2], few, some + few + ties + some,
+             list(circuits.random_circuit(n, 2, seed=n, measure=False).ops)]
+    if n >= 6:
+        lists.append(some + [ops.Operation(random_unitary(rng, 8), q[:3])] + few)
+    for opl in lists:
+        got = []
+        for given in (False, True):
+            r = Register.from_int(n, k, dtype)
+            if given:
+                r.state = e
+            for op in opl:
+                r.apply(op)
+            got.append(r.state)
+            r.close()
+        assert np.array_equal(got[0], got[1]), len(opl)
+    r = Register.from_int(n, k, dtype)
+    c = r.clone()
+    assert r.measure(0) == bool(k & 1)
+    c.apply(ops.hadamard(n - 1))
+    c.apply(ops.hadamard(n - 1))
+    assert abs(abs(c.amplitudes([k])[0]) - 1) < (1e-14 if dtype == "c128" else 1e-6)
+
+
 @pytest.mark.parametrize("dtype, k, n", [
     ("c128", 5, 9), ("c128", 5, 10), ("c128", 5, 15), ("c128", 5, 21), ("c128", 6, 9),
     ("c128", 6, 10), ("c128", 6, 12), ("c128", 6, 21), ("c128", 7, 7), ("c128", 7, 13),
