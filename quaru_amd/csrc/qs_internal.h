@@ -65,7 +65,10 @@ Fixed make_fixed(uint64_t mask, uint64_t set);
 // ---- kept device memory and workspaces (qs_pool.hip) --------------------------
 
 constexpr int kReduceBlocks = 1024;
-constexpr size_t kRedDoubles = 4 * kReduceBlocks + 64;
+// d_red: partials, then 64 doubles of results, collapse parameters and
+// measurement slots, then the counter of split_end (0 between launches).
+constexpr size_t kRedCount = 4 * kReduceBlocks + 64;
+constexpr size_t kRedDoubles = kRedCount + 8;
 constexpr size_t kRingBytes = 8u << 20;
 
 // hipMalloc and hipFree on the current device through the pool of kept
@@ -103,8 +106,12 @@ hipError_t launch_init_basis(void *psi, int n, uint64_t k, hipStream_t s);
 // Zero the amplitudes i with (i & mask) != val.
 template <typename R>
 hipError_t launch_zero_outside(void *psi, int n, uint64_t mask, uint64_t val, hipStream_t s);
+// The n qubits of a product state, amplitudes {re, im} of 0 and of 1 each.
+struct ProductState {
+  double q[4 * kMaxQubits];
+};
 template <typename R>
-hipError_t launch_init_product(void *psi, int n, const double *d_qubits, hipStream_t s);
+hipError_t launch_init_product(void *psi, int n, const ProductState &q, hipStream_t s);
 template <typename R>
 hipError_t launch_gate_dense(void *psi, int n, const Gate &g, void *d_mat, void *scratch,
                              hipStream_t s);
@@ -124,8 +131,20 @@ hipError_t launch_gate_perm(void *psi, int n, const Gate &g, const void *d_tab, 
 
 // Reductions write FP64 results to device memory `d_out` (caller copies).
 // d_part must hold kReduceBlocks * 2 doubles.
+
+// Where a probability split leaves its result: {prob_0, prob_1} in `host`
+// (pinned memory), or the outcome x > prob_0 in *slot and {outcome,
+// sqrt(its probability)} in coll (device memory).  `count` is a counter in
+// device memory that is 0 between launches.
+struct SplitEnd {
+  unsigned *count = nullptr;
+  double *host = nullptr;
+  double x = 0.0;
+  double *coll = nullptr;
+  unsigned char *slot = nullptr;
+};
 template <typename R>
-hipError_t launch_prob_split(const void *psi, int n, int target, double *d_part, double *d_out,
+hipError_t launch_prob_split(void *psi, int n, int target, double *d_part, const SplitEnd &end,
                              hipStream_t s);
 template <typename R>
 hipError_t launch_collapse(void *psi, int n, int target, int keep, double total, hipStream_t s);
@@ -139,13 +158,13 @@ hipError_t launch_collapse_pattern(void *psi, int n, uint64_t mask, uint64_t pat
 // pass, with the same {prob_0, prob_1} bits as the two in sequence.
 template <typename R>
 hipError_t launch_collapse_split(void *psi, int n, int ctarget, int keep, double total,
-                                 int target, double *d_part, double *d_out, hipStream_t s);
+                                 int target, double *d_part, const SplitEnd &end, hipStream_t s);
 // Measure and collapse with the outcome decided on the device (no host
-// round trip): d_probs (2 doubles) and d_coll (2 doubles) are work space, the
-// outcome (0 or 1) goes to *d_slot.
+// round trip): d_coll (2 doubles) is work space, the outcome (0 or 1) goes to
+// *d_slot.
 template <typename R>
 hipError_t launch_measure_deferred(void *psi, int n, int target, double x, double *d_part,
-                                   double *d_probs, double *d_coll, unsigned char *d_slot,
+                                   double *d_coll, unsigned *d_count, unsigned char *d_slot,
                                    hipStream_t s);
 template <typename R>
 hipError_t launch_norm(const void *psi, int n, double *d_part, double *d_out, hipStream_t s);

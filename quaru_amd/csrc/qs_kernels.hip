@@ -154,7 +154,8 @@ __global__ __launch_bounds__(kBlock) void k_zero_outside(typename V2<R>::T *psi,
 // (b_0 * 1)).
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_init_product(typename V2<R>::T *psi, int n,
-                                                         const double *__restrict__ q) {
+                                                         ProductState p) {
+  const double *q = p.q;
   using T = typename V2<R>::T;
   const uint64_t len = 1ull << n;
   for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < len;
@@ -196,12 +197,12 @@ hipError_t launch_zero_outside(void *psi, int n, uint64_t mask, uint64_t val, hi
 }
 
 template <typename R>
-hipError_t launch_init_product(void *psi, int n, const double *d_qubits, hipStream_t s) {
+hipError_t launch_init_product(void *psi, int n, const ProductState &q, hipStream_t s) {
   const uint64_t len = 1ull << n;
   unsigned g = grid_for(len, kBlock * 8);
   if (g > 65536) g = 65536;
   hipLaunchKernelGGL(k_init_product<R>, dim3(g), dim3(kBlock), 0, s,
-                     (typename V2<R>::T *)psi, n, d_qubits);
+                     (typename V2<R>::T *)psi, n, q);
   return hipGetLastError();
 }
 
@@ -1527,10 +1528,65 @@ static inline bool reduce_blocked(uint64_t len) {
   return len >= (uint64_t)kReduceBlocks * kRedTrip;
 }
 
+// The end of a split over all blocks: the partials go to `part`, and the
+// block that comes last (it counts them, and leaves the counter at 0) adds
+// them up in the order of k_finish.  {prob_0, prob_1} go to `host`, or, with a
+// slot, the outcome is decided here (src/register.rs:317-321: x > prob_0),
+// stored there and left with its scale in `coll` for the collapse.  Against a
+// kernel of its own for the sums, a copy to the host and a kernel for the
+// decision: a measurement of 12 qubits is one launch of 5.0 us, was three of
+// 6.5; a deferred one of up to 8 qubits one launch of 2.4 us with its
+// collapse, was four of 6.6 (teleportation of one qubit 101 us, 147).
+// Returns whether this block was the last; v holds the sums on its threads.
+__device__ __forceinline__ bool split_end(double (&v)[2], double (*sh)[kBlock],
+                                          double *__restrict__ part, const SplitEnd &end) {
+  __shared__ bool last;
+  if (gridDim.x > 1) {
+    if (threadIdx.x == 0) {
+      for (int c = 0; c < 2; ++c)
+        __hip_atomic_store(part + 2 * blockIdx.x + c, v[c], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      last = __hip_atomic_fetch_add(end.count, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) ==
+             gridDim.x - 1;
+    }
+    __syncthreads();
+    if (!last) return false;
+    v[0] = v[1] = 0.0;
+    for (unsigned b = threadIdx.x; b < gridDim.x; b += kBlock)
+      for (int c = 0; c < 2; ++c)
+        v[c] += __hip_atomic_load(part + 2 * b + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    block_sum<2>(v, sh);
+    if (threadIdx.x == 0)
+      __hip_atomic_store(end.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (threadIdx.x == 0) {
+    if (end.host) {
+      end.host[0] = v[0];
+      end.host[1] = v[1];
+    }
+    if (end.slot) {
+      const int res = end.x > v[0];
+      end.coll[0] = (double)res;
+      end.coll[1] = sqrt(res ? v[1] : v[0]);
+      *end.slot = (unsigned char)res;
+    }
+  }
+  return true;
+}
+
+// Amplitude a of index i after a collapse on bit `target` of outcome `keep`.
+template <typename R, typename T>
+__device__ __forceinline__ T collapsed(T a, uint64_t i, int target, int keep, double sq) {
+  if ((int)((i >> target) & 1ull) != keep) return czero<T>();
+  a.x = (R)((double)a.x / sq);
+  a.y = (R)((double)a.y / sq);
+  return a;
+}
+
 template <typename R, bool kBlocked>
-__global__ __launch_bounds__(kBlock) void k_prob_split(const typename V2<R>::T *__restrict__ psi,
+__global__ __launch_bounds__(kBlock) void k_prob_split(typename V2<R>::T *__restrict__ psi,
                                                        uint64_t len, int target,
-                                                       double *__restrict__ part) {
+                                                       double *__restrict__ part, SplitEnd end) {
   __shared__ double sh[2][kBlock];
   double v[2] = {0.0, 0.0};
   // each thread adds its amplitudes in index order (k_collapse_split relies
@@ -1553,10 +1609,7 @@ __global__ __launch_bounds__(kBlock) void k_prob_split(const typename V2<R>::T *
       }
     }
     block_sum<2>(v, sh);
-    if (threadIdx.x == 0) {
-      part[2 * blockIdx.x] = v[0];
-      part[2 * blockIdx.x + 1] = v[1];
-    }
+    split_end(v, sh, part, end);
     return;
   }
   // four loads in flight per trip
@@ -1586,24 +1639,26 @@ __global__ __launch_bounds__(kBlock) void k_prob_split(const typename V2<R>::T *
       v[0] += p;
   }
   block_sum<2>(v, sh);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = v[0];
-    part[2 * blockIdx.x + 1] = v[1];
+  split_end(v, sh, part, end);
+  if (end.slot && gridDim.x == 1) {  // one block: the collapse as well
+    const int keep = end.x > v[0];
+    const double sq = sqrt(keep ? v[1] : v[0]);
+    for (i = threadIdx.x; i < len; i += kBlock)
+      psi[i] = collapsed<R>(psi[i], i, target, keep, sq);
   }
 }
 
 template <typename R>
-hipError_t launch_prob_split(const void *psi, int n, int target, double *d_part, double *d_out,
+hipError_t launch_prob_split(void *psi, int n, int target, double *d_part, const SplitEnd &end,
                              hipStream_t s) {
   const uint64_t len = 1ull << n;
   const int g = reduce_grid(len);
   if (reduce_blocked(len))
     hipLaunchKernelGGL((k_prob_split<R, true>), dim3(g), dim3(kBlock), 0, s,
-                       (const typename V2<R>::T *)psi, len, target, d_part);
+                       (typename V2<R>::T *)psi, len, target, d_part, end);
   else
     hipLaunchKernelGGL((k_prob_split<R, false>), dim3(g), dim3(kBlock), 0, s,
-                       (const typename V2<R>::T *)psi, len, target, d_part);
-  hipLaunchKernelGGL(k_finish<2>, dim3(1), dim3(kBlock), 0, s, (const double *)d_part, g, d_out);
+                       (typename V2<R>::T *)psi, len, target, d_part, end);
   return hipGetLastError();
 }
 
@@ -1614,17 +1669,9 @@ template <typename R>
 __global__ __launch_bounds__(kBlock) void k_collapse(typename V2<R>::T *__restrict__ psi,
                                                      uint64_t len, int target, int keep,
                                                      double sq) {
-  using T = typename V2<R>::T;
   for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < len;
        i += (uint64_t)gridDim.x * kBlock) {
-    T a = psi[i];
-    if ((int)((i >> target) & 1ull) != keep) {
-      a = czero<T>();
-    } else {
-      a.x = (R)((double)a.x / sq);
-      a.y = (R)((double)a.y / sq);
-    }
-    psi[i] = a;
+    psi[i] = collapsed<R>(psi[i], i, target, keep, sq);
   }
 }
 
@@ -1640,17 +1687,13 @@ template <typename R, bool kBlocked>
 __global__ __launch_bounds__(kBlock) void k_collapse_split(typename V2<R>::T *__restrict__ psi,
                                                            uint64_t len, int ctarget, int keep,
                                                            double sq, int target,
-                                                           double *__restrict__ part) {
+                                                           double *__restrict__ part,
+                                                           SplitEnd end) {
   using T = typename V2<R>::T;
   __shared__ double sh[2][kBlock];
   double v[2] = {0.0, 0.0};
   auto one = [&](uint64_t i, T a) {
-    if ((int)((i >> ctarget) & 1ull) != keep) {
-      a = czero<T>();
-    } else {
-      a.x = (R)((double)a.x / sq);
-      a.y = (R)((double)a.y / sq);
-    }
+    a = collapsed<R>(a, i, ctarget, keep, sq);
     st<kBlocked>(psi + i, a);
     const double re = (double)a.x, im = (double)a.y;
     const double p = re * re + im * im;
@@ -1675,10 +1718,7 @@ __global__ __launch_bounds__(kBlock) void k_collapse_split(typename V2<R>::T *__
       for (int k = 0; k < kRedLoads; ++k) one(w + (uint64_t)k * kBlock, a[k]);
     }
     block_sum<2>(v, sh);
-    if (threadIdx.x == 0) {
-      part[2 * blockIdx.x] = v[0];
-      part[2 * blockIdx.x + 1] = v[1];
-    }
+    split_end(v, sh, part, end);
     return;
   }
   const uint64_t S = (uint64_t)gridDim.x * kBlock;
@@ -1693,39 +1733,23 @@ __global__ __launch_bounds__(kBlock) void k_collapse_split(typename V2<R>::T *__
   }
   for (; i < len; i += S) one(i, (int)((i >> ctarget) & 1ull) == keep ? psi[i] : czero<T>());
   block_sum<2>(v, sh);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = v[0];
-    part[2 * blockIdx.x + 1] = v[1];
-  }
+  split_end(v, sh, part, end);
 }
 
 template <typename R>
 hipError_t launch_collapse_split(void *psi, int n, int ctarget, int keep, double total,
-                                 int target, double *d_part, double *d_out, hipStream_t s) {
+                                 int target, double *d_part, const SplitEnd &end, hipStream_t s) {
   const uint64_t len = 1ull << n;
   const int g = reduce_grid(len);
   if (reduce_blocked(len))
     hipLaunchKernelGGL((k_collapse_split<R, true>), dim3(g), dim3(kBlock), 0, s,
-                       (typename V2<R>::T *)psi, len, ctarget, keep, sqrt(total), target, d_part);
+                       (typename V2<R>::T *)psi, len, ctarget, keep, sqrt(total), target, d_part,
+                       end);
   else
     hipLaunchKernelGGL((k_collapse_split<R, false>), dim3(g), dim3(kBlock), 0, s,
-                       (typename V2<R>::T *)psi, len, ctarget, keep, sqrt(total), target, d_part);
-  hipLaunchKernelGGL(k_finish<2>, dim3(1), dim3(kBlock), 0, s, (const double *)d_part, g, d_out);
+                       (typename V2<R>::T *)psi, len, ctarget, keep, sqrt(total), target, d_part,
+                       end);
   return hipGetLastError();
-}
-
-// Deferred measurement, decided on the device: probs = {prob_0, prob_1} from
-// k_prob_split, the rule of src/register.rs:317-321 (result = x > prob_0),
-// the outcome into *slot and {keep, sqrt(total)} into coll for
-// k_collapse_dev.
-__global__ void k_measure_decide(const double *__restrict__ probs, double x,
-                                 unsigned char *__restrict__ slot, double *__restrict__ coll) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  const double p0 = probs[0], p1 = probs[1];
-  const int res = x > p0;
-  coll[0] = (double)res;
-  coll[1] = sqrt(res ? p1 : p0);
-  *slot = (unsigned char)res;
 }
 
 // k_collapse with its outcome and scale read from device memory.
@@ -1733,31 +1757,26 @@ template <typename R>
 __global__ __launch_bounds__(kBlock) void k_collapse_dev(typename V2<R>::T *__restrict__ psi,
                                                          uint64_t len, int target,
                                                          const double *__restrict__ coll) {
-  using T = typename V2<R>::T;
   const int keep = (int)coll[0];
   const double sq = coll[1];
   for (uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x; i < len;
        i += (uint64_t)gridDim.x * kBlock) {
-    T a = psi[i];
-    if ((int)((i >> target) & 1ull) != keep) {
-      a = czero<T>();
-    } else {
-      a.x = (R)((double)a.x / sq);
-      a.y = (R)((double)a.y / sq);
-    }
-    psi[i] = a;
+    psi[i] = collapsed<R>(psi[i], i, target, keep, sq);
   }
 }
 
 template <typename R>
 hipError_t launch_measure_deferred(void *psi, int n, int target, double x, double *d_part,
-                                   double *d_probs, double *d_coll, unsigned char *d_slot,
+                                   double *d_coll, unsigned *d_count, unsigned char *d_slot,
                                    hipStream_t s) {
-  hipError_t e = launch_prob_split<R>(psi, n, target, d_part, d_probs, s);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_measure_decide, dim3(1), dim3(64), 0, s, (const double *)d_probs, x,
-                     d_slot, d_coll);
   const uint64_t len = 1ull << n;
+  SplitEnd end;
+  end.count = d_count;
+  end.x = x;
+  end.coll = d_coll;
+  end.slot = d_slot;
+  hipError_t e = launch_prob_split<R>(psi, n, target, d_part, end, s);
+  if (e != hipSuccess || reduce_grid(len) == 1) return e;
   unsigned grid = grid_for(len, kBlock * 4);
   if (grid > 262144) grid = 262144;
   hipLaunchKernelGGL(k_collapse_dev<R>, dim3(grid), dim3(kBlock), 0, s, (typename V2<R>::T *)psi,
@@ -2310,7 +2329,7 @@ hipError_t launch_chunk_sums(const void *psi, int n, uint64_t chunk, double *d_o
 
 #define QS_INSTANTIATE(R)                                                                        \
   template hipError_t launch_init_basis<R>(void *, int, uint64_t, hipStream_t);                 \
-  template hipError_t launch_init_product<R>(void *, int, const double *, hipStream_t);         \
+  template hipError_t launch_init_product<R>(void *, int, const ProductState &, hipStream_t);   \
   template hipError_t launch_zero_outside<R>(void *, int, uint64_t, uint64_t, hipStream_t);     \
   template hipError_t launch_gate_dense<R>(void *, int, const Gate &, void *, void *,            \
                                            hipStream_t);                                         \
@@ -2318,15 +2337,15 @@ hipError_t launch_chunk_sums(const void *psi, int n, uint64_t chunk, double *d_o
   template hipError_t launch_gate_sparse<R>(void *, int, const Gate &, hipStream_t);            \
   template hipError_t launch_gate_perm<R>(void *, int, const Gate &, const void *, void *,       \
                                           hipStream_t);                                          \
-  template hipError_t launch_prob_split<R>(const void *, int, int, double *, double *,          \
+  template hipError_t launch_prob_split<R>(void *, int, int, double *, const SplitEnd &,        \
                                            hipStream_t);                                         \
   template hipError_t launch_collapse<R>(void *, int, int, int, double, hipStream_t);           \
   template hipError_t launch_collapse_pattern<R>(void *, int, uint64_t, uint64_t, double,        \
                                                  hipStream_t);                                   \
   template hipError_t launch_collapse_split<R>(void *, int, int, int, double, int, double *,     \
-                                               double *, hipStream_t);                           \
+                                               const SplitEnd &, hipStream_t);                   \
   template hipError_t launch_measure_deferred<R>(void *, int, int, double, double *, double *,  \
-                                                 double *, unsigned char *, hipStream_t);       \
+                                                 unsigned *, unsigned char *, hipStream_t);     \
   template hipError_t launch_norm<R>(const void *, int, double *, double *, hipStream_t);       \
   template hipError_t launch_neq_count<R>(const void *, const void *, int, double, double *,    \
                                           double *, hipStream_t);                                \

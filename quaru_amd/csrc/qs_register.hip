@@ -775,6 +775,10 @@ hipError_t reduce_norm(qs_register *r, double *out) {
   return e;
 }
 
+unsigned *red_count(qs_register *r) {
+  return reinterpret_cast<unsigned *>(r->d_red + qs::kRedCount);
+}
+
 // One measure (src/register.rs:297-342) on the device state.  The split
 // reads the state (fused with the previous measure's collapse when that is
 // still pending); the collapse itself is left pending, for the next measure
@@ -782,17 +786,16 @@ hipError_t reduce_norm(qs_register *r, double *out) {
 // have been flushed.
 template <typename R>
 int measure_one(qs_register *r, size_t target, double x, int *result) {
-  double *res_dev = r->d_red + 4 * qs::kReduceBlocks;
+  qs::SplitEnd end;
+  end.count = red_count(r);
+  end.host = r->h_red;
   if (r->coll_pending) {
     r->coll_pending = false;
     QS_HIP(qs::launch_collapse_split<R>(r->psi, r->n, r->coll_target, r->coll_keep,
-                                        r->coll_total, (int)target, r->d_red, res_dev,
-                                        r->stream));
+                                        r->coll_total, (int)target, r->d_red, end, r->stream));
   } else {
-    QS_HIP(qs::launch_prob_split<R>(r->psi, r->n, (int)target, r->d_red, res_dev, r->stream));
+    QS_HIP(qs::launch_prob_split<R>(r->psi, r->n, (int)target, r->d_red, end, r->stream));
   }
-  QS_HIP(hipMemcpyAsync(r->h_red, res_dev, 2 * sizeof(double), hipMemcpyDeviceToHost,
-                        r->stream));
   QS_HIP(hipStreamSynchronize(r->stream));
   const double p0 = r->h_red[0], p1 = r->h_red[1];
   const int res = x > p0;
@@ -1059,15 +1062,12 @@ int qs_register_from_qubits(const double *qubits, const size_t *lens, size_t cou
   int rc = alloc_register(count, dtype, out);
   if (rc) return rc;
   qs_register *r = *out;
-  // the qubits' amplitudes through the upload ring (at most 40 of them)
-  void *d_q = nullptr;
-  const double none[4] = {};
-  hipError_t e = ring_upload(r, count ? qubits : none,
-                             std::max<size_t>(1, count) * 4 * sizeof(double), &d_q);
-  if (e == hipSuccess)
-    e = by_dtype(r, [&](auto z) {
-      return qs::launch_init_product<decltype(z)>(r->psi, r->n, (const double *)d_q, r->stream);
-    });
+  // the qubits' amplitudes as kernel arguments (at most 40 of them)
+  qs::ProductState q{};
+  if (count) std::memcpy(q.q, qubits, count * 4 * sizeof(double));
+  hipError_t e = by_dtype(r, [&](auto z) {
+    return qs::launch_init_product<decltype(z)>(r->psi, r->n, q, r->stream);
+  });
   if (e != hipSuccess) {
     qs_register_free(r);
     *out = nullptr;
@@ -1246,11 +1246,11 @@ int qs_measure_deferred(qs_register *r, size_t target, double uniform, size_t sl
   int rc = flush(r);
   if (rc) return rc;
   r->slots_used = true;
-  double *res_dev = r->d_red + 4 * qs::kReduceBlocks;
+  double *coll = r->d_red + 4 * qs::kReduceBlocks;
   auto go = [&](auto z) {
     using Rt = decltype(z);
-    return qs::launch_measure_deferred<Rt>(r->psi, r->n, (int)target, uniform, r->d_red, res_dev,
-                                           res_dev + 2, slot_base(r) + slot, r->stream);
+    return qs::launch_measure_deferred<Rt>(r->psi, r->n, (int)target, uniform, r->d_red, coll,
+                                           red_count(r), slot_base(r) + slot, r->stream);
   };
   QS_HIP(r->dtype == QS_C128 ? go(0.0) : go(0.0f));
   return QS_OK;

@@ -94,11 +94,23 @@ __device__ __forceinline__ void small_2x2(const SmallPass<R> &p, int j, uint32_t
   y = w;
 }
 
-// One workgroup; 2^n amplitudes (n >= 2) in dynamic LDS, then the chunk.
+// A list short enough for the kernel's arguments (at most 4 KiB): no copy of
+// its own to the device, 3 us of the stream and 4 of the host.
 template <typename R>
+constexpr int kArgPasses = sizeof(R) == 8 ? 8 : 14;
+
+template <typename R, int N>
+struct SmallArgs {
+  SmallPass<R> p[N > 0 ? N : 1];
+};
+
+// One workgroup; 2^n amplitudes (n >= 2) in dynamic LDS, then the chunk.  The
+// passes are in `args` (NA > 0) or at prog.
+template <typename R, int NA>
 __global__ __launch_bounds__(kSmallThreads) void k_small(typename sweep::SV2<R>::T *__restrict__ psi,
                                                          int n, const SmallPass<R> *__restrict__ prog,
-                                                         int npass, uint32_t basis) {
+                                                         int npass, uint32_t basis,
+                                                         SmallArgs<R, NA> args) {
   using T = typename sweep::SV2<R>::T;
   extern __shared__ unsigned char small_smem[];
   T *s = (T *)small_smem;
@@ -112,7 +124,7 @@ __global__ __launch_bounds__(kSmallThreads) void k_small(typename sweep::SV2<R>:
     for (uint32_t i = tid; i < N; i += nt) s[small_pos(i)] = psi[i];
   constexpr int CP = kChunkPasses<R>;
   constexpr uint32_t kWords = CP * sizeof(SmallPass<R>) / 16;
-  const uint4 *src = reinterpret_cast<const uint4 *>(prog);
+  const uint4 *src = reinterpret_cast<const uint4 *>(NA > 0 ? args.p : prog);
   uint4 *dst = reinterpret_cast<uint4 *>(chunk);
   const uint32_t total = (uint32_t)npass * (uint32_t)(sizeof(SmallPass<R>) / 16);
   for (int c0 = 0; c0 < npass; c0 += CP) {
@@ -290,18 +302,34 @@ hipError_t execute_small_t(SweepRunner &run, const std::vector<Gate> &gates, uin
   b.n = n;
   auto launch = [&]() -> hipError_t {
     if (b.prog.empty()) return hipSuccess;
+    constexpr int NA = kArgPasses<R>;
+    const bool in_args = b.prog.size() <= (size_t)NA;
     void *d = nullptr;
-    hipError_t e = run.upload(b.prog.data(), b.prog.size() * sizeof(SmallPass<R>), &d);
+    hipError_t e = hipSuccess;
+    if (!in_args) e = run.upload(b.prog.data(), b.prog.size() * sizeof(SmallPass<R>), &d);
     if (e != hipSuccess) return e;
     const size_t lds = (sizeof(T) << n) + kChunkPasses<R> * sizeof(SmallPass<R>);
-    static const hipError_t set = hipFuncSetAttribute(
-        (const void *)k_small<R>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    static const hipError_t set = [] {
+      const hipError_t e1 = hipFuncSetAttribute(
+          (const void *)k_small<R, 0>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+      const hipError_t e2 = hipFuncSetAttribute(
+          (const void *)k_small<R, NA>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+      return e1 != hipSuccess ? e1 : e2;
+    }();
     if (set != hipSuccess) return set;
     const unsigned threads = (unsigned)std::min(kSmallThreads, std::max(64, 1 << (n - 2)));
     if (run.mark) run.mark(true);
-    hipLaunchKernelGGL(k_small<R>, dim3(1), dim3(threads), lds, run.stream, (T *)run.psi, n,
-                       (const SmallPass<R> *)d, (int)b.prog.size(),
-                       run.fresh ? (uint32_t)run.known_val : ~0u);
+    const uint32_t basis = run.fresh ? (uint32_t)run.known_val : ~0u;
+    if (in_args) {
+      SmallArgs<R, NA> args{};
+      std::memcpy(args.p, b.prog.data(), b.prog.size() * sizeof(SmallPass<R>));
+      hipLaunchKernelGGL((k_small<R, NA>), dim3(1), dim3(threads), lds, run.stream, (T *)run.psi,
+                         n, nullptr, (int)b.prog.size(), basis, args);
+    } else {
+      hipLaunchKernelGGL((k_small<R, 0>), dim3(1), dim3(threads), lds, run.stream, (T *)run.psi,
+                         n, (const SmallPass<R> *)d, (int)b.prog.size(), basis,
+                         SmallArgs<R, 0>{});
+    }
     if (run.mark) run.mark(false);
     e = hipGetLastError();
     if (e == hipSuccess) {

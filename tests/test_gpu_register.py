@@ -988,6 +988,43 @@ def test_apply_circuit_condition_on_a_later_measured_target(dtype):
     assert len(seen) == 4
 
 
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+@pytest.mark.parametrize("n", [1, 2, 8, 9, 13, 18, 19, 22])
+def test_measures_of_one_and_many_blocks(n, dtype):
+    """Measures in turn, at once and deferred, from states of one workgroup
+    to those read in 64 KiB trips: outcomes by the oracle's rule from FP64
+    sums of the stored amplitudes (every uniform is 1e-3 away from them), and
+    the collapsed amplitudes."""
+    import ctypes
+    from quaru_amd import _lib
+    rng = np.random.default_rng(4000 + n)
+    psi = random_state(rng, n)
+    a = Register.new([False] * n, dtype)
+    b = Register.new([False] * n, dtype)
+    a.state = psi
+    b.state = psi
+    lib = _lib.load()
+    ref = a.state
+    bits = []
+    for slot, t in enumerate(int(x) for x in rng.permutation(n)[:4]):
+        on = ((np.arange(1 << n) >> t) & 1).astype(bool)
+        p = np.abs(ref) ** 2
+        p0, p1 = p[~on].sum(), p[on].sum()
+        u = p0 + (1e-3 if rng.integers(2) else -1e-3)
+        res = u > p0
+        ref = np.where(on == res, ref / np.sqrt(p1 if res else p0), 0)
+        bits.append(int(res))
+        assert a.measure(t, u) == res
+        assert lib.qs_measure_deferred(b.handle, t, float(u), slot) == 0
+    out = (ctypes.c_ubyte * len(bits))()
+    assert lib.qs_read_slots(b.handle, 0, len(bits), out) == 0
+    assert list(out) == bits
+    assert np.array_equal(a.state, b.state)
+    assert maxdiff(a.state, ref) < (TOL if dtype == "c128" else 2e-6)
+    a.close()
+    b.close()
+
+
 def test_measure_deferred_equals_measure():
     import ctypes
     from quaru_amd import EngineError, _lib
