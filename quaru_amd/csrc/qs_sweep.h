@@ -47,6 +47,10 @@ struct SweepRunner {
   uint64_t known = 0, known_val = 0;
   bool fresh = false;
   std::function<hipError_t()> fill;
+  // Where the state is, if not in psi yet: the next sweep reads it there, and
+  // anything else copies it first.
+  const void *src = nullptr;
+  std::function<hipError_t()> copy;
   hipStream_t stream = nullptr;
   // Copy host bytes to a device buffer that stays valid until the stream
   // reaches the next launch.
@@ -71,7 +75,8 @@ struct SweepRunner {
 hipError_t sweep_execute(SweepEngine *e, SweepRunner &run, const std::vector<Gate> &gates,
                          uint64_t *sweeps, uint64_t *kernels);
 
-// Write the amplitudes that run.known leaves out, if any.
+// Write the amplitudes that run.known leaves out, if any; bring the state to
+// psi.
 hipError_t sweep_settle(SweepRunner &run);
 
 // Registers whose state fits one compute unit's LDS run their gates there, in

@@ -731,6 +731,8 @@ hipError_t execute_t(SweepRunner &run, const std::vector<Gate> &gates, uint64_t 
     // the padding states of a batch are the last tiles: they are left out
     h.ntiles = run.states && nt < n ? (uint64_t)run.states << (nt - T - kept)
                                     : 1ull << (n - T - kept);
+    h.src = (uint64_t)(uintptr_t)run.src;  // (with run.known and run.fresh clear)
+    run.src = nullptr;
     const size_t hbytes = (sizeof(SweepHeader) + 15) & ~(size_t)15;
     const size_t bbytes = blob_bytes<R>((int)h.nops, (int)h.npool);
     blob.assign(bbytes, 0);
@@ -825,6 +827,11 @@ int sweep_reg_bits(bool c64) {
 }
 
 hipError_t sweep_settle(SweepRunner &run) {
+  if (run.src) {
+    const hipError_t e = run.copy();
+    run.src = nullptr;
+    return e;
+  }
   if (!run.known && !run.fresh) return hipSuccess;
   const hipError_t e = run.fill();
   run.known = run.known_val = 0;

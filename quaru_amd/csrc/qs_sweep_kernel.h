@@ -182,6 +182,9 @@ struct SweepHeader {
   // 211, 219), 27 qubits with three sweeps of Hadamards 7.9 ms, 9.9.
   uint32_t start;
   uint64_t kmask, kset, pmask, pval;
+  // Device address that the amplitudes are read from, 0: where they go.  A
+  // state that is kept and carried on (an adjoint checkpoint) costs no copy.
+  uint64_t src;
 };
 enum : uint32_t { START_FULL = 0, START_PART = 1, START_BASIS = 2 };
 
@@ -1188,7 +1191,8 @@ __device__ __forceinline__ void sweep_tile(typename SV2<R>::T *__restrict__ psi,
   Amp<R, NA> a;
   {
     typename SNT<R>::T v[NA];
-    const typename SNT<R>::T *src = reinterpret_cast<const typename SNT<R>::T *>(psi);
+    const typename SNT<R>::T *src = reinterpret_cast<const typename SNT<R>::T *>(
+        h.src ? (const void *)h.src : (const void *)psi);
     if (h.start == START_FULL) {
 #pragma unroll
       for (int r = 0; r < NA; ++r)
