@@ -2108,12 +2108,31 @@ __global__ __launch_bounds__(kBlock) void k_set_hist(const typename V2<R>::T *__
   }
 }
 
+// Column sums of rows x H partials: a workgroup takes bw = min(H, 32) columns
+// (256-byte runs) and splits the rows over 256 / bw slices, added in order in
+// LDS.  Bound by the read.  1024 rows of 4096: 10 us, 256 with one thread per
+// column and 16 workgroups.
 __global__ __launch_bounds__(kBlock) void k_hist_finish(const double *__restrict__ part,
-                                                        int blocks, int H,
+                                                        int rows, int H, int bw,
                                                         double *__restrict__ out) {
-  for (int h = blockIdx.x * kBlock + threadIdx.x; h < H; h += gridDim.x * kBlock) {
-    double v = 0.0;
-    for (int b = 0; b < blocks; ++b) v += part[(size_t)b * H + h];
+  __shared__ double sh[kBlock];
+  const int c = (int)threadIdx.x % bw, sl = (int)threadIdx.x / bw, ns = kBlock / bw;
+  const int h = (int)blockIdx.x * bw + c;
+  int r = (int)((long long)rows * sl / ns);
+  const int end = (int)((long long)rows * (sl + 1) / ns);
+  double v = 0.0;
+  for (; r + 7 < end; r += 8) {
+    double x[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) x[k] = part[(size_t)(r + k) * H + h];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v += x[k];
+  }
+  for (; r < end; ++r) v += part[(size_t)r * H + h];
+  sh[threadIdx.x] = v;
+  __syncthreads();
+  if (sl == 0) {
+    for (int k = 1; k < ns; ++k) v += sh[k * bw + c];
     out[h] = v;
   }
 }
@@ -2139,8 +2158,9 @@ hipError_t launch_set_histogram(const void *psi, int n, const Fixed &fx, const u
                          : k_set_hist<R, 16>;
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(kBlock), 0, s, (const T *)psi, fx, po, m, nfree,
                      per_block, d_part);
-  hipLaunchKernelGGL(k_hist_finish, dim3((H + kBlock - 1) / kBlock), dim3(kBlock), 0, s,
-                     (const double *)d_part, rows, H, d_hist);
+  const int bw = std::min(H, 32);
+  hipLaunchKernelGGL(k_hist_finish, dim3(H / bw), dim3(kBlock), 0, s, (const double *)d_part, rows,
+                     H, bw, d_hist);
   return hipGetLastError();
 }
 

@@ -988,6 +988,37 @@ def test_apply_circuit_condition_on_a_later_measured_target(dtype):
     assert len(seen) == 4
 
 
+@pytest.mark.parametrize("n, m", [(1, 1), (5, 5), (14, 1), (14, 2), (16, 5), (16, 8), (18, 12),
+                                  (20, 3)])
+def test_sequences_of_some_qubits(n, m):
+    """A sequence of m measures at once (from one histogram): outcomes by the
+    oracle's rule from FP64 sums (every uniform 1e-3 away from them) and the
+    collapsed amplitudes."""
+    import ctypes
+    from quaru_amd import _lib
+    rng = np.random.default_rng(5000 + 20 * n + m)
+    psi = random_state(rng, n)
+    order = [int(x) for x in rng.permutation(n)[:m]]
+    ref, us, want = psi, [], 0
+    for t in order:
+        on = ((np.arange(1 << n) >> t) & 1).astype(bool)
+        p = np.abs(ref) ** 2
+        p0, p1 = p[~on].sum(), p[on].sum()
+        us.append(p0 + (1e-3 if rng.integers(2) else -1e-3))
+        res = us[-1] > p0
+        ref = np.where(on == res, ref / np.sqrt(p1 if res else p0), 0)
+        want |= int(res) << t
+    r = Register.new([False] * n)
+    r.state = psi
+    o = (ctypes.c_size_t * m)(*order)
+    u = (ctypes.c_double * m)(*us)
+    out = ctypes.c_uint64()
+    assert _lib.load().qs_measure_sequence(r.handle, o, m, u, ctypes.byref(out)) == 0
+    assert out.value == want
+    assert maxdiff(r.state, ref) < TOL
+    r.close()
+
+
 @pytest.mark.parametrize("dtype", ["c128", "c64"])
 @pytest.mark.parametrize("n", [1, 2, 8, 9, 13, 18, 19, 22])
 def test_measures_of_one_and_many_blocks(n, dtype):
