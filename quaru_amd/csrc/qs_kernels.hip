@@ -15,6 +15,7 @@
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
+#include <utility>
 
 #include "qs_internal.h"
 
@@ -2252,21 +2253,36 @@ __global__ __launch_bounds__(kBlock) void k_chunk_sums(const typename V2<R>::T *
 // (its last amplitude if there is none).
 //
 // The chain of dependent FP64 additions bounds a shot (65536 of them for a
-// whole chunk, about 0.2 ms), so the shots run side by side, and the next
-// kSampleTrip amplitudes load while the current ones are added.  Every lane
-// runs the same chain on broadcast LDS reads.  Measured with the readouts
-// beside it, 1000 shots of 26 qubits, complex128: 1.5 ms, against 110 ms with
-// the ~640 hit chunks' probabilities copied to and scanned on the host.
+// whole chunk), so the shots run side by side, and the next kSampleTrip
+// amplitudes load while the current ones are added.  Every lane runs the same
+// chain; each row of 16 lanes holds the next 16 values and hands them round
+// by DPP.  1000 shots of 26 qubits, complex128: 543 us, 620 with every value
+// read from LDS by all lanes (four waves of a CU share its LDS); with the
+// readouts beside it 1.39 ms, against 110 ms with the ~640 hit chunks'
+// probabilities copied to and scanned on the host.
 constexpr int kSampleLoads = 16;
 constexpr int kSampleTrip = 64 * kSampleLoads;
+constexpr int kSampleGroup = 64;  // additions between two looks at the sum
+
+// Value of lane K of each row of 16 lanes, on all lanes of the row.
+template <int K>
+__device__ __forceinline__ double row_bcast(double v) {
+  return __builtin_amdgcn_mov_dpp(v, 0x150 + K, 0xF, 0xF, false);  // row_newbcast
+}
+
+// sum + v of lane 0 + v of lane 1 + ... of the row, one after the other.
+template <int... K>
+__device__ __forceinline__ double add_row(double sum, double v, std::integer_sequence<int, K...>) {
+  ((sum += row_bcast<K>(v)), ...);
+  return sum;
+}
 
 template <typename R>
 __global__ __launch_bounds__(64) void k_sample(const typename V2<R>::T *__restrict__ psi,
                                                uint64_t chunk, const SampleShot *__restrict__ shots,
                                                uint64_t count, uint64_t *__restrict__ out) {
   using T = typename V2<R>::T;
-  __shared__ double2 p2[kSampleTrip / 2];
-  double *p = reinterpret_cast<double *>(p2);
+  __shared__ double p[kSampleTrip];
   if (blockIdx.x >= count) return;
   const SampleShot s = shots[blockIdx.x];
   const T *src = psi + s.chunk * chunk;
@@ -2295,20 +2311,23 @@ __global__ __launch_bounds__(64) void k_sample(const typename V2<R>::T *__restri
     }
     // amplitudes past the chunk's end add 0; they cannot be the first above
     // tau, which an addition of 0 does not reach
-    for (int g = 0; g < kSampleTrip; g += 16) {
-      double2 v[8];
+    double v[4];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) v[k] = p2[g / 2 + k];
+    for (int k = 0; k < 4; ++k) v[k] = p[16 * k + (lane & 15)];
+    for (int g = 0; g < kSampleTrip; g += kSampleGroup) {
+      // the next group's reads are in flight while this one is added (the
+      // last group reads itself again)
+      double ahead[4];
+      const int ag = g + kSampleGroup < kSampleTrip ? g + kSampleGroup : g;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) ahead[k] = p[ag + 16 * k + (lane & 15)];
       double next = run;
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        next += v[k].x;
-        next += v[k].y;
-      }
+      for (int k = 0; k < 4; ++k) next = add_row(next, v[k], std::make_integer_sequence<int, 16>{});
       // not `next > tau`: a NaN behind the first sum above tau must not hide it
       if (!(next <= tau)) {
         double t = run;
-        for (int k = 0; k < 16; ++k) {
+        for (int k = 0; k < kSampleGroup; ++k) {
           t += p[g + k];
           if (t > tau) {
             if (lane == 0) out[blockIdx.x] = s.chunk * chunk + w + (uint64_t)(g + k);
@@ -2317,6 +2336,8 @@ __global__ __launch_bounds__(64) void k_sample(const typename V2<R>::T *__restri
         }
       }
       run = next;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = ahead[k];
     }
     __syncthreads();
   }
