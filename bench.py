@@ -243,13 +243,12 @@ def adjoint_bench(n: int, layers: int, batch: int, fd_params: int, dtype: str):
     device_sync()
     t2 = time.perf_counter()
     t_adj, t_fwd, t_bwd = t2 - t0, t1 - t0, t2 - t1
-    # algorithmic HBM bytes of the reverse pass (S = the batch of states):
-    # lambda = h psi (2S), each tiled block reads and writes psi and lambda
-    # (4S), each checkpoint restore copies psi (2S)
-    bp = 1 << max(0, (batch - 1).bit_length())
-    S = float(bp << n) * (16 if dtype == "c128" else 8)
+    # algorithmic HBM bytes of the reverse pass (S = the batch of states): each
+    # tiled block reads and writes psi and lambda (4S), the first makes lambda
+    # = h psi instead of reading it; a checkpoint is restored without a copy
+    S = float(batch << n) * (16 if dtype == "c128" else 8)
     rstats = run.reverse_stats
-    bwd_bytes = 2 * S + rstats["blocks"] * 4 * S + rstats["restores"] * 2 * S
+    bwd_bytes = rstats["blocks"] * 4 * S - S
     fwd_bytes = fstats["sweeps"] * 2 * S
     # central finite differences (h = 1e-4, FP64) on the same GPU for a sample
     # of parameters: each needs two forward passes of the whole batch.

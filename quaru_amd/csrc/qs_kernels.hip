@@ -627,9 +627,9 @@ struct StageMap {
 // compute pattern (lanes = groups) over the banks.
 __device__ __forceinline__ int stage_phys(int s) { return s ^ ((s >> 5) & 31); }
 
-// K = 3..5 active targets when low index bits are fixed (active or
-// controls): the direct kernel's loads would then stride by 2^(lowest free
-// bit) amplitudes per lane.  One wave stages 64 groups through LDS with
+// K = 3..5 active targets (complex128: those that k_dense_tile does not take)
+// when low index bits are fixed (active or controls): the direct kernel's
+// loads would then stride by 2^(lowest free bit) amplitudes per lane.  One wave stages 64 groups through LDS with
 // loads over the block's lowest index bits, each lane computes its own group
 // from registers (matrix on scalar loads, as in k_gatek), writes its outputs
 // back to its own slots, and the wave stores the block the way it loaded it.

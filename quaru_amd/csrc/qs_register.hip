@@ -71,7 +71,7 @@ struct qs_register {
   qs::Workspace *ws = nullptr;  // owns stream, ring, d_red and h_red below
   hipStream_t stream = nullptr;
   void *psi = nullptr;
-  void *scratch = nullptr;  // 2^n amplitudes, only for dense ops with > 5 active bits
+  void *scratch = nullptr;  // 2^n amplitudes, for gates whose kernel reads a copy of the state
   double *d_red = nullptr;  // reduction partials + results
   bool slots_used = false;  // a deferred measurement wrote its slot in d_red
   double *d_big = nullptr;  // measurement and readout work buffer, grown on demand
