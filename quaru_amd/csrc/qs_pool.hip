@@ -10,10 +10,10 @@
 // by size, and handed to the next caller of the same size.
 //
 // Bounds: all kept blocks together take at most an eighth of the device's
-// memory, the oldest leave first; once nothing has been taken or handed in
-// for a second, all but kIdleKept bytes are given back; and when an
-// allocation of this library fails, everything kept on the device is given
-// back before it is tried again.  A block is handed in only when no GPU work
+// memory, the oldest leave first; a block that has lain here for a second is
+// given back, whatever goes on with the others, as long as more than
+// kIdleKept bytes are kept; and when an allocation of this library fails,
+// everything kept on the device is given back before it is tried again.  A block is handed in only when no GPU work
 // uses it any more (its owner has drained its stream), so any thread and any
 // stream may take it next.  Contents are whatever was there.
 #include <hip/hip_runtime.h>
@@ -36,10 +36,13 @@ constexpr size_t kIdleKept = 64ull << 20;
 constexpr auto kIdle = std::chrono::seconds(1);
 constexpr size_t kMaxSpaces = 4;  // kept workspaces per device
 
+using Clock = std::chrono::steady_clock;
+
 struct Block {
   void *p;
   size_t bytes;
   int device;
+  Clock::time_point since;  // when it was handed in
 };
 
 struct Pool {
@@ -51,7 +54,6 @@ struct Pool {
   // gives back what is idle
   std::condition_variable wake;
   std::mutex freeing;  // held while the idle thread frees
-  std::chrono::steady_clock::time_point used;
   bool started = false, stopping = false;
 };
 
@@ -61,14 +63,16 @@ Pool &pool() {
   return *p;
 }
 
-// Take kept blocks of `device` (all devices: -1) out, oldest first, until at
-// most `keep` bytes are left there.  The caller frees them without the lock.
-std::vector<Block> take_out(Pool &p, int device, size_t keep) {
+// Take kept blocks of `device` (all devices: -1) that were handed in by
+// `until` out, oldest first, until at most `keep` bytes are left there.  The
+// caller frees them without the lock.
+std::vector<Block> take_out(Pool &p, int device, size_t keep,
+                            Clock::time_point until = Clock::time_point::max()) {
   size_t kept = 0;
   for (const Block &b : p.blocks)
     if (device < 0 || b.device == device) kept += b.bytes;
   std::vector<Block> out;
-  for (auto it = p.blocks.begin(); it != p.blocks.end() && kept > keep;) {
+  for (auto it = p.blocks.begin(); it != p.blocks.end() && kept > keep && it->since <= until;) {
     if (device >= 0 && it->device != device) {
       ++it;
       continue;
@@ -97,12 +101,13 @@ void idle_thread() {
       p.wake.wait(lk);
       continue;
     }
-    const auto due = p.used + kIdle;
-    if (std::chrono::steady_clock::now() < due) {
+    const auto now = Clock::now();
+    const auto due = p.blocks.front().since + kIdle;
+    if (now < due) {
       p.wake.wait_until(lk, due);
       continue;
     }
-    const std::vector<Block> freed = take_out(p, -1, kIdleKept);
+    const std::vector<Block> freed = take_out(p, -1, kIdleKept, now - kIdle);
     std::unique_lock<std::mutex> busy(p.freeing);
     lk.unlock();
     give_back(freed);
@@ -132,7 +137,6 @@ hipError_t pool_malloc(void **out, size_t bytes) {
   Pool &p = pool();
   {
     std::lock_guard<std::mutex> lk(p.mu);
-    p.used = std::chrono::steady_clock::now();
     for (auto it = p.blocks.end(); it != p.blocks.begin();) {
       --it;  // the newest first
       if (it->bytes == bytes && it->device == device) {
@@ -164,7 +168,6 @@ void pool_free(void *ptr, size_t bytes, int device) {
   bool kept = false;
   {
     std::lock_guard<std::mutex> lk(p.mu);
-    p.used = std::chrono::steady_clock::now();
     auto it = p.bound.find(device);
     if (it == p.bound.end()) {
       size_t total = 0;
@@ -175,7 +178,7 @@ void pool_free(void *ptr, size_t bytes, int device) {
     }
     kept = bytes > 0 && bytes <= it->second && !p.stopping;
     if (kept) {
-      p.blocks.push_back({ptr, bytes, device});
+      p.blocks.push_back({ptr, bytes, device, Clock::now()});
       p.kept += bytes;
       freed = take_out(p, device, it->second);
       if (!p.started && p.kept > kIdleKept) {

@@ -1,0 +1,93 @@
+// CPU check of the pool of kept device memory: qs_pool.hip itself, compiled
+// against a stand-in for the HIP runtime (fake_hip).  The first argument
+// names the check; prints "ok" or what failed.
+#include <hip/hip_runtime.h>
+
+#include <chrono>
+#include <cstdio>
+#include <cstring>
+#include <thread>
+
+#include "qs_pool.hip"
+
+using namespace qs;
+
+namespace {
+
+constexpr size_t MiB = 1ull << 20, GiB = 1ull << 30;
+
+#define CHECK(cond)                                                \
+  do {                                                             \
+    if (!(cond)) {                                                 \
+      std::printf("line %d: %s\n", __LINE__, #cond);               \
+      return 1;                                                    \
+    }                                                              \
+  } while (0)
+
+void *take(size_t bytes) {
+  void *p = nullptr;
+  return pool_malloc(&p, bytes) == hipSuccess ? p : nullptr;
+}
+
+void wait_ms(int ms) { std::this_thread::sleep_for(std::chrono::milliseconds(ms)); }
+
+// Until `cond`, at most `ms`.
+template <typename F>
+bool within(int ms, F &&cond) {
+  for (; ms > 0 && !cond(); ms -= 10) wait_ms(10);
+  return cond();
+}
+
+// A block goes to the next caller of its size; all kept ones together stay
+// within an eighth of the device, the oldest leave first; a failed allocation
+// gets what is kept.
+int bounds() {
+  void *a = take(GiB), *b = take(2 * GiB);
+  CHECK(a && b);
+  pool_free(a, GiB, 0);
+  CHECK(fake::used(0) == 3 * GiB);
+  CHECK(take(GiB) == a);
+  void *c = take(GiB);
+  CHECK(c && c != a);
+  pool_free(a, GiB, 0);
+  pool_free(b, 2 * GiB, 0);
+  pool_free(c, GiB, 0);
+  void *d = take(5 * GiB);
+  pool_free(d, 5 * GiB, 0);  // 9 GiB would be kept: the oldest one leaves
+  CHECK(fake::device_of(a) == -1 && fake::device_of(b) == 0 && fake::used(0) == 8 * GiB);
+  void *e = take(9 * GiB);  // more than an eighth is not kept
+  pool_free(e, 9 * GiB, 0);
+  CHECK(fake::used(0) == 8 * GiB);
+  void *f = take(60 * GiB);
+  CHECK(f && fake::used(0) == 60 * GiB);
+  CHECK(!take(60 * GiB));
+  pool_free(f, 60 * GiB, 0);
+  CHECK(fake::used(0) == 0);
+  return 0;
+}
+
+// A block that nothing has taken for a second goes back, also while others
+// come and go.
+int idle() {
+  void *big = take(4 * GiB);
+  pool_free(big, 4 * GiB, 0);
+  for (int k = 0; k < 200; ++k) {
+    void *s = take(MiB);
+    pool_free(s, MiB, 0);
+    wait_ms(10);
+  }
+  CHECK(fake::device_of(big) == -1);
+  CHECK(fake::used(0) == MiB);
+  return 0;
+}
+
+}  // namespace
+
+int main(int argc, char **argv) {
+  const char *what = argc > 1 ? argv[1] : "";
+  int rc = 1;
+  if (!std::strcmp(what, "bounds")) rc = bounds();
+  if (!std::strcmp(what, "idle")) rc = idle();
+  if (rc == 0) std::printf("ok\n");
+  return rc;
+}
