@@ -85,8 +85,15 @@ std::vector<Block> take_out(Pool &p, int device, size_t keep,
   return out;
 }
 
+// Another thread may be recording a stream into a graph, in the mode that
+// refuses every thread's frees (and breaks the recording off); these are none
+// of the recorded work's.
 void give_back(const std::vector<Block> &v) {
+  if (v.empty()) return;
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
   for (const Block &b : v) (void)hipFree(b.p);
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
 }
 
 bool out_of_memory(hipError_t e) {
@@ -189,7 +196,7 @@ void pool_free(void *ptr, size_t bytes, int device) {
       p.wake.notify_one();
     }
   }
-  if (!kept) (void)hipFree(ptr);
+  if (!kept) freed.push_back({ptr, bytes, device, {}});
   give_back(freed);
 }
 

@@ -81,6 +81,19 @@ int idle() {
   return 0;
 }
 
+// The idle thread frees while another thread records a stream: the recording
+// (global mode) refuses every thread's allocations and frees that have not
+// said otherwise.
+int capture() {
+  void *big = take(4 * GiB);
+  fake::rt().capturing = true;
+  pool_free(big, 4 * GiB, 0);
+  CHECK(within(3000, [&] { return fake::device_of(big) == -1; }));
+  CHECK(fake::rt().refused_frees == 0);
+  CHECK(fake::mode == hipStreamCaptureModeGlobal);  // this thread's is as it was
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -88,6 +101,7 @@ int main(int argc, char **argv) {
   int rc = 1;
   if (!std::strcmp(what, "bounds")) rc = bounds();
   if (!std::strcmp(what, "idle")) rc = idle();
+  if (!std::strcmp(what, "capture")) rc = capture();
   if (rc == 0) std::printf("ok\n");
   return rc;
 }
