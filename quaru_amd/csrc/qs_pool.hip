@@ -21,9 +21,11 @@
 #include <chrono>
 #include <condition_variable>
 #include <cstdlib>
+#include <iterator>
 #include <list>
-#include <map>
 #include <mutex>
+#include <new>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -35,6 +37,7 @@ namespace {
 constexpr size_t kIdleKept = 64ull << 20;
 constexpr auto kIdle = std::chrono::seconds(1);
 constexpr size_t kMaxSpaces = 4;  // kept workspaces per device
+constexpr int kMaxDevices = 64;   // memory of further ones is not kept
 
 using Clock = std::chrono::steady_clock;
 
@@ -50,11 +53,11 @@ struct Pool {
   std::list<Block> blocks;  // oldest first
   size_t kept = 0;          // bytes in blocks
   std::vector<Workspace *> spaces;
-  std::map<int, size_t> bound;  // bytes kept per device at most
+  size_t bound[kMaxDevices] = {};  // bytes kept per device at most, 0: not asked yet
   // gives back what is idle
   std::condition_variable wake;
   std::mutex freeing;  // held while the idle thread frees
-  bool started = false, stopping = false;
+  bool started = false, exits = false, stopping = false;
 };
 
 // Never destroyed: threads may free their registers while the process exits.
@@ -66,21 +69,22 @@ Pool &pool() {
 // Take kept blocks of `device` (all devices: -1) that were handed in by
 // `until` out, oldest first, until at most `keep` bytes are left there.  The
 // caller frees them without the lock.
-std::vector<Block> take_out(Pool &p, int device, size_t keep,
-                            Clock::time_point until = Clock::time_point::max()) {
+std::list<Block> take_out(Pool &p, int device, size_t keep,
+                          Clock::time_point until = Clock::time_point::max()) {
   size_t kept = 0;
   for (const Block &b : p.blocks)
     if (device < 0 || b.device == device) kept += b.bytes;
-  std::vector<Block> out;
+  std::list<Block> out;
   for (auto it = p.blocks.begin(); it != p.blocks.end() && kept > keep && it->since <= until;) {
     if (device >= 0 && it->device != device) {
       ++it;
       continue;
     }
+    const auto next = std::next(it);
     kept -= it->bytes;
     p.kept -= it->bytes;
-    out.push_back(*it);
-    it = p.blocks.erase(it);
+    out.splice(out.end(), p.blocks, it);
+    it = next;
   }
   return out;
 }
@@ -88,7 +92,7 @@ std::vector<Block> take_out(Pool &p, int device, size_t keep,
 // Another thread may be recording a stream into a graph, in the mode that
 // refuses every thread's frees (and breaks the recording off); these are none
 // of the recorded work's.
-void give_back(const std::vector<Block> &v) {
+void give_back(const std::list<Block> &v) {
   if (v.empty()) return;
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   (void)hipThreadExchangeStreamCaptureMode(&mode);
@@ -114,7 +118,7 @@ void idle_thread() {
       p.wake.wait_until(lk, due);
       continue;
     }
-    const std::vector<Block> freed = take_out(p, -1, kIdleKept, now - kIdle);
+    const std::list<Block> freed = take_out(p, -1, kIdleKept, now - kIdle);
     std::unique_lock<std::mutex> busy(p.freeing);
     lk.unlock();
     give_back(freed);
@@ -132,6 +136,21 @@ void stop_idle_thread() {
     p.stopping = true;
   }
   std::lock_guard<std::mutex> busy(p.freeing);
+}
+
+// Whether the idle thread runs (it is started on demand): without it nothing
+// would be given back, so nothing above kIdleKept is kept.
+bool idle_thread_runs(Pool &p) {
+  if (p.started) return true;
+  if (p.exits || std::atexit(stop_idle_thread) == 0) {
+    p.exits = true;
+    try {
+      std::thread(idle_thread).detach();
+      p.started = true;
+    } catch (const std::system_error &) {
+    }
+  }
+  return p.started;
 }
 
 }  // namespace
@@ -156,7 +175,7 @@ hipError_t pool_malloc(void **out, size_t bytes) {
   }
   e = hipMalloc(out, bytes);
   if (!out_of_memory(e)) return e;
-  std::vector<Block> freed;
+  std::list<Block> freed;
   {
     std::lock_guard<std::mutex> lk(p.mu);
     freed = take_out(p, device, 0);
@@ -168,35 +187,35 @@ hipError_t pool_malloc(void **out, size_t bytes) {
   return hipMalloc(out, bytes);
 }
 
+// No exception leaves it: closing a register ends here, at a C entry.
 void pool_free(void *ptr, size_t bytes, int device) {
   if (!ptr) return;
   Pool &p = pool();
-  std::vector<Block> freed;
-  bool kept = false;
-  {
+  std::list<Block> freed;
+  try {
+    freed.push_back({ptr, bytes, device, Clock::now()});
+  } catch (const std::bad_alloc &) {
+    (void)hipFree(ptr);
+    return;
+  }
+  if (bytes > 0 && device >= 0 && device < kMaxDevices) {
     std::lock_guard<std::mutex> lk(p.mu);
-    auto it = p.bound.find(device);
-    if (it == p.bound.end()) {
+    size_t &bound = p.bound[device];  // bytes kept there at most
+    if (bound == 0) {
       size_t total = 0;
       hipDevice_t d = 0;
-      if (hipDeviceGet(&d, device) != hipSuccess || hipDeviceTotalMem(&total, d) != hipSuccess)
-        total = 0;
-      it = p.bound.emplace(device, total / 8).first;
+      if (hipDeviceGet(&d, device) == hipSuccess && hipDeviceTotalMem(&total, d) == hipSuccess)
+        bound = total / 8;
     }
-    kept = bytes > 0 && bytes <= it->second && !p.stopping;
-    if (kept) {
-      p.blocks.push_back({ptr, bytes, device, Clock::now()});
+    if (bytes <= bound && !p.stopping) {
       p.kept += bytes;
-      freed = take_out(p, device, it->second);
-      if (!p.started && p.kept > kIdleKept) {
-        p.started = true;
-        std::atexit(stop_idle_thread);
-        std::thread(idle_thread).detach();
-      }
+      p.blocks.splice(p.blocks.end(), freed);
+      freed = take_out(p, device, bound);
+      if (p.kept > kIdleKept && !idle_thread_runs(p))
+        freed.splice(freed.end(), take_out(p, -1, kIdleKept));
       p.wake.notify_one();
     }
   }
-  if (!kept) freed.push_back({ptr, bytes, device, {}});
   give_back(freed);
 }
 

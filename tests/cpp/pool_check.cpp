@@ -1,8 +1,11 @@
 // CPU check of the pool of kept device memory: qs_pool.hip itself, compiled
 // against a stand-in for the HIP runtime (fake_hip).  The first argument
 // names the check; prints "ok" or what failed.
+#include <dlfcn.h>
 #include <hip/hip_runtime.h>
+#include <pthread.h>
 
+#include <cerrno>
 #include <chrono>
 #include <cstdio>
 #include <cstring>
@@ -11,6 +14,15 @@
 #include "qs_pool.hip"
 
 using namespace qs;
+
+// Thread creation, refused on demand.
+static bool no_threads = false;
+extern "C" int pthread_create(pthread_t *t, const pthread_attr_t *a, void *(*f)(void *), void *x) {
+  if (no_threads) return EAGAIN;
+  using Fn = int (*)(pthread_t *, const pthread_attr_t *, void *(*)(void *), void *);
+  static const Fn next = reinterpret_cast<Fn>(dlsym(RTLD_NEXT, "pthread_create"));
+  return next(t, a, f, x);
+}
 
 namespace {
 
@@ -94,6 +106,22 @@ int capture() {
   return 0;
 }
 
+// No thread to be had: nothing may throw out of pool_free (a C entry calls
+// it), and what would never be given back is not kept.
+int no_thread() {
+  void *big = take(4 * GiB), *s = take(MiB);
+  no_threads = true;
+  pool_free(s, MiB, 0);
+  pool_free(big, 4 * GiB, 0);
+  CHECK(fake::used(0) <= 64 * MiB);
+  no_threads = false;
+  big = take(4 * GiB);
+  pool_free(big, 4 * GiB, 0);  // the next one may start it
+  CHECK(fake::device_of(big) == 0);
+  CHECK(within(3000, [&] { return fake::device_of(big) == -1; }));
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -102,6 +130,7 @@ int main(int argc, char **argv) {
   if (!std::strcmp(what, "bounds")) rc = bounds();
   if (!std::strcmp(what, "idle")) rc = idle();
   if (!std::strcmp(what, "capture")) rc = capture();
+  if (!std::strcmp(what, "no_thread")) rc = no_thread();
   if (rc == 0) std::printf("ok\n");
   return rc;
 }

@@ -16,12 +16,12 @@ def exe(tmp_path_factory):
     subprocess.run(["g++", "-x", "c++", "-std=c++17", "-O1", "-pthread",
                     "-I", os.path.join(CPP, "fake_hip"),
                     "-I", os.path.join(ROOT, "quaru_amd", "csrc"),
-                    os.path.join(CPP, "pool_check.cpp"), "-o", out],
+                    os.path.join(CPP, "pool_check.cpp"), "-ldl", "-o", out],
                    check=True, capture_output=True, timeout=300)
     return out
 
 
-@pytest.mark.parametrize("rule", ["bounds", "idle", "capture"])
+@pytest.mark.parametrize("rule", ["bounds", "idle", "capture", "no_thread"])
 def test_kept_memory(exe, rule):
     res = subprocess.run([exe, rule], capture_output=True, text=True, timeout=60)
     assert res.returncode == 0 and res.stdout == "ok\n", res.stdout + res.stderr
