@@ -54,9 +54,9 @@ struct Pool {
   size_t kept = 0;          // bytes in blocks
   std::vector<Workspace *> spaces;
   size_t bound[kMaxDevices] = {};  // bytes kept per device at most, 0: not asked yet
-  // gives back what is idle
-  std::condition_variable wake;
-  std::mutex freeing;  // held while the idle thread frees
+  std::condition_variable wake;  // of the thread that gives back what is idle
+  int freeing = 0;               // threads that are giving blocks back
+  std::condition_variable freed;
   bool started = false, exits = false, stopping = false;
 };
 
@@ -89,15 +89,23 @@ std::list<Block> take_out(Pool &p, int device, size_t keep,
   return out;
 }
 
+// Free blocks that were taken out, without the lock; `freeing` counts the
+// threads that do, so that a failed allocation can wait for them.
+//
 // Another thread may be recording a stream into a graph, in the mode that
 // refuses every thread's frees (and breaks the recording off); these are none
 // of the recorded work's.
-void give_back(const std::list<Block> &v) {
+void give_back(Pool &p, std::unique_lock<std::mutex> &lk, const std::list<Block> &v) {
   if (v.empty()) return;
+  ++p.freeing;
+  lk.unlock();
   hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
   (void)hipThreadExchangeStreamCaptureMode(&mode);
   for (const Block &b : v) (void)hipFree(b.p);
   (void)hipThreadExchangeStreamCaptureMode(&mode);
+  lk.lock();
+  --p.freeing;
+  p.freed.notify_all();
 }
 
 bool out_of_memory(hipError_t e) {
@@ -118,12 +126,7 @@ void idle_thread() {
       p.wake.wait_until(lk, due);
       continue;
     }
-    const std::list<Block> freed = take_out(p, -1, kIdleKept, now - kIdle);
-    std::unique_lock<std::mutex> busy(p.freeing);
-    lk.unlock();
-    give_back(freed);
-    busy.unlock();
-    lk.lock();
+    give_back(p, lk, take_out(p, -1, kIdleKept, now - kIdle));
   }
 }
 
@@ -131,11 +134,9 @@ void idle_thread() {
 // under way.
 void stop_idle_thread() {
   Pool &p = pool();
-  {
-    std::lock_guard<std::mutex> lk(p.mu);
-    p.stopping = true;
-  }
-  std::lock_guard<std::mutex> busy(p.freeing);
+  std::unique_lock<std::mutex> lk(p.mu);
+  p.stopping = true;
+  p.freed.wait(lk, [&] { return p.freeing == 0; });
 }
 
 // Whether the idle thread runs (it is started on demand): without it nothing
@@ -175,15 +176,12 @@ hipError_t pool_malloc(void **out, size_t bytes) {
   }
   e = hipMalloc(out, bytes);
   if (!out_of_memory(e)) return e;
-  std::list<Block> freed;
-  {
-    std::lock_guard<std::mutex> lk(p.mu);
-    freed = take_out(p, device, 0);
-  }
-  // (also when nothing was kept: the idle thread may just be freeing)
-  std::lock_guard<std::mutex> busy(p.freeing);
   (void)hipGetLastError();
-  give_back(freed);
+  std::unique_lock<std::mutex> lk(p.mu);
+  give_back(p, lk, take_out(p, device, 0));
+  // (also when nothing was kept: another thread may just be giving it back)
+  p.freed.wait(lk, [&] { return p.freeing == 0; });
+  lk.unlock();
   return hipMalloc(out, bytes);
 }
 
@@ -198,8 +196,8 @@ void pool_free(void *ptr, size_t bytes, int device) {
     (void)hipFree(ptr);
     return;
   }
+  std::unique_lock<std::mutex> lk(p.mu);
   if (bytes > 0 && device >= 0 && device < kMaxDevices) {
-    std::lock_guard<std::mutex> lk(p.mu);
     size_t &bound = p.bound[device];  // bytes kept there at most
     if (bound == 0) {
       size_t total = 0;
@@ -216,7 +214,7 @@ void pool_free(void *ptr, size_t bytes, int device) {
       p.wake.notify_one();
     }
   }
-  give_back(freed);
+  give_back(p, lk, freed);
 }
 
 namespace {

@@ -3,11 +3,13 @@
 // calls, so that pool_check.cpp runs that file itself without a GPU.
 #pragma once
 
+#include <atomic>
+#include <chrono>
 #include <cstddef>
 #include <cstdint>
 #include <map>
 #include <mutex>
-#include <set>
+#include <thread>
 
 enum hipError_t {
   hipSuccess = 0,
@@ -46,8 +48,7 @@ inline Runtime &rt() {
 
 inline thread_local int current = 0;
 inline thread_local hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;
-// how long a free waits for the device
-inline thread_local bool slow_free = false;
+inline std::atomic<int> free_ms{0};  // how long a free waits for the device
 
 // Device of a live block, -1: none there.
 inline int device_of(void *p) {
@@ -104,6 +105,7 @@ inline hipError_t hipMalloc(void **out, size_t bytes) {
 }
 inline hipError_t hipFree(void *p) {
   auto &r = fake::rt();
+  std::this_thread::sleep_for(std::chrono::milliseconds(fake::free_ms.load()));
   std::lock_guard<std::mutex> lk(r.mu);
   if (r.capturing && fake::mode != hipStreamCaptureModeRelaxed) {
     ++r.refused_frees;

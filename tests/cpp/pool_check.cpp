@@ -122,6 +122,31 @@ int no_thread() {
   return 0;
 }
 
+// An allocation that fails while another thread (first the one that hands a
+// block in, then the idle one) is giving memory back waits for that.
+int freeing() {
+  void *a = take(5 * GiB), *b = take(6 * GiB), *rest = take(50 * GiB);
+  pool_free(a, 5 * GiB, 0);
+  fake::free_ms = 300;
+  std::thread other([&] { pool_free(b, 6 * GiB, 0); });  // the 5 GiB leave
+  wait_ms(100);
+  fake::free_ms = 0;
+  void *c = take(14 * GiB);  // needs both blocks' memory
+  CHECK(c);
+  other.join();
+  CHECK(fake::device_of(a) == -1 && fake::device_of(b) == -1);
+  pool_free(c, 14 * GiB, 0);
+  a = take(5 * GiB);
+  c = take(9 * GiB);
+  CHECK(a && c);
+  fake::free_ms = 600;
+  pool_free(a, 5 * GiB, 0);
+  wait_ms(1200);  // the idle thread frees it now
+  CHECK(take(5 * GiB));
+  CHECK(rest);
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -130,6 +155,7 @@ int main(int argc, char **argv) {
   if (!std::strcmp(what, "bounds")) rc = bounds();
   if (!std::strcmp(what, "idle")) rc = idle();
   if (!std::strcmp(what, "capture")) rc = capture();
+  if (!std::strcmp(what, "freeing")) rc = freeing();
   if (!std::strcmp(what, "no_thread")) rc = no_thread();
   if (rc == 0) std::printf("ok\n");
   return rc;
