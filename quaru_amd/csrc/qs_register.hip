@@ -972,6 +972,32 @@ int measure_fast(qs_register *r, const size_t *order, size_t count, const double
   return QS_OK;
 }
 
+// Whether the first `cnt` shots are scanned on the host, chunk by chunk in
+// `order`, instead of by k_sample: `longest` additions for the shot furthest
+// into its chunk, `all` of them together.  The kernel takes one chain of 8.3
+// ns additions at a time per shot, all shots side by side; the host adds at
+// 0.55 ns, one shot after the other, and needs the chunks copied.
+constexpr double kSampleAddUs = 8.3e-3, kSampleShotUs = 0.015, kSampleLaunchUs = 4.0;
+constexpr double kScanAddUs = 0.55e-3, kScanChunkUs = 12.0, kScanCopyUs = 0.2e-3;
+
+bool sample_on_host(const std::vector<qs::SampleShot> &shots, size_t cnt, uint64_t chunk,
+                    double longest, double all, std::vector<uint32_t> &order) {
+  const double device =
+      kSampleLaunchUs + kSampleShotUs * (double)cnt + kSampleAddUs * longest;
+  auto host = [&](size_t chunks) {
+    return kScanChunkUs * (double)(chunks - 1) +
+           kScanCopyUs * (double)chunks * (double)chunk + kScanAddUs * all;
+  };
+  if (!(host(1) < device)) return false;
+  order.resize(cnt);
+  for (size_t j = 0; j < cnt; ++j) order[j] = (uint32_t)j;
+  std::sort(order.begin(), order.end(),
+            [&](uint32_t a, uint32_t b) { return shots[a].chunk < shots[b].chunk; });
+  size_t chunks = 1;
+  for (size_t k = 1; k < cnt; ++k) chunks += shots[order[k]].chunk != shots[order[k - 1]].chunk;
+  return host(chunks) < device;
+}
+
 // Classify and enqueue a gate, as its one-qubit factors when it has them and
 // fusion is on (with fusion off every factor would be a pass of its own).
 int enqueue_matrix(qs_register *r, const double *matrix, const size_t *targets, size_t k,
@@ -1321,10 +1347,11 @@ int qs_sample_cdf(qs_register *r, const double *uniforms, size_t count, uint64_t
   const size_t piece = std::min<size_t>(count, kSamplePiece);
   std::vector<double> sums(nchunks);
   double *d_sums = nullptr;
-  QS_HIP(ensure_big(r, nchunks * sizeof(double) +
+  QS_HIP(ensure_big(r, (nchunks + chunk) * sizeof(double) +
                            piece * (sizeof(qs::SampleShot) + sizeof(uint64_t)),
                     &d_sums));
-  qs::SampleShot *d_shots = reinterpret_cast<qs::SampleShot *>(d_sums + nchunks);
+  double *d_probs = d_sums + nchunks;
+  qs::SampleShot *d_shots = reinterpret_cast<qs::SampleShot *>(d_probs + chunk);
   uint64_t *d_idx = reinterpret_cast<uint64_t *>(d_shots + piece);
   hipError_t e = by_dtype(r, [&](auto z) {
     return qs::launch_chunk_sums<decltype(z)>(r->psi, r->n, chunk, d_sums, r->stream);
@@ -1338,8 +1365,10 @@ int qs_sample_cdf(qs_register *r, const double *uniforms, size_t count, uint64_t
   for (uint64_t c = 0; c < nchunks; ++c) prefix[c + 1] = prefix[c] + sums[c];
   const double total = prefix[nchunks];
   std::vector<qs::SampleShot> shots(piece);
+  std::vector<uint32_t> order;
   for (size_t off = 0; off < count; off += piece) {
     const size_t cnt = std::min(piece, count - off);
+    double longest = 0.0, all = 0.0;  // additions, by where tau lies in its chunk
     for (size_t j = 0; j < cnt; ++j) {
       const double tau = uniforms[off + j] * total;
       // first chunk whose running sum exceeds tau
@@ -1347,6 +1376,42 @@ int qs_sample_cdf(qs_register *r, const double *uniforms, size_t count, uint64_t
                               (prefix.begin() + 1));
       if (c >= nchunks) c = nchunks - 1;
       shots[j] = {c, prefix[c], tau};
+      const double part = (tau - prefix[c]) / sums[c];
+      const double adds = part >= 0.0 && part <= 1.0 ? part * (double)chunk : (double)chunk;
+      longest = std::max(longest, adds);
+      all += adds;
+    }
+    if (sample_on_host(shots, cnt, chunk, longest, all, order)) {
+      // one chunk after the other through the pinned ring (the stream is
+      // drained); as k_sample: the same additions in the same order
+      const double *pr = reinterpret_cast<const double *>(r->h_ring);
+      for (size_t k = 0; k < cnt; ++k) {
+        const qs::SampleShot &s = shots[order[k]];
+        if (k == 0 || s.chunk != shots[order[k - 1]].chunk) {
+          e = by_dtype(r, [&](auto z) {
+            return qs::launch_probabilities<decltype(z)>(
+                (const char *)r->psi + s.chunk * chunk * r->amp_bytes(),
+                (int)(63 - __builtin_clzll(chunk)), d_probs, r->stream);
+          });
+          if (e == hipSuccess)
+            e = hipMemcpyAsync(r->h_ring, d_probs, chunk * sizeof(double), hipMemcpyDeviceToHost,
+                               r->stream);
+          if (e == hipSuccess) e = hipStreamSynchronize(r->stream);
+          if (e != hipSuccess) return hip_fail(e, "qs_sample_cdf");
+        }
+        double run = s.run;
+        uint64_t i = 0;
+        for (; i < chunk; ++i) {
+          run += pr[i];
+          if (run > s.tau) break;
+        }
+        if (i == chunk) {  // the last amplitude with a probability above 0
+          for (i = chunk - 1; i > 0 && !(pr[i] > 0.0);) --i;
+          if (!(pr[i] > 0.0)) i = chunk - 1;
+        }
+        indices[off + order[k]] = s.chunk * chunk + i;
+      }
+      continue;
     }
     e = hipMemcpyAsync(d_shots, shots.data(), cnt * sizeof(qs::SampleShot),
                        hipMemcpyHostToDevice, r->stream);

@@ -646,6 +646,34 @@ def test_sample_cdf_many_shots():
     assert np.array_equal(r.sample(u), np.arange(70001) % 16)
 
 
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+@pytest.mark.parametrize("n", [0, 3, 10, 13, 16, 17, 20])
+def test_samples_alone_and_among_many(n, dtype):
+    """A few shots are scanned on the host, many by the kernel: the same
+    index for the same uniform, also at and past the ends of the range and
+    where the sums are not numbers."""
+    rng = np.random.default_rng(90 + n)
+    r = Register.from_int(n, 0, dtype=dtype, seed=1)
+    u = np.concatenate([rng.random(6), [0.0, 1 - 2**-53, 1.0, 2.0, -1.0]])
+    many = np.concatenate([u, rng.random(20000)])
+    for bad in (None, 0.0, np.nan, np.inf):
+        psi = random_state(rng, n)
+        if bad is not None:
+            psi[-1 - (1 << n) // 3:] = 0
+            psi[(1 << n) // 2] = bad
+        r.state = psi
+        got = r.sample(many)
+        assert np.array_equal([int(r.sample([x])[0]) for x in u], got[:u.size])
+        if bad is not None and not np.isfinite(bad):
+            # every comparison with a sum fails: the last amplitude above 0
+            tail = np.abs(psi[-min(1 << n, 1 << 16):]) ** 2
+            on = np.nonzero(tail > 0)[0]
+            last = on[-1] if on.size else tail.size - 1
+            if np.isnan(bad):
+                assert np.all(got == (1 << n) - tail.size + last)
+    r.close()
+
+
 # ---- reductions and equality ---------------------------------------------------------
 
 @pytest.mark.parametrize("dtype", ["c128", "c64"])
