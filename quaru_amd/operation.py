@@ -57,8 +57,13 @@ class Operation:
         # copies and pickles get arrays of their own, so not the addresses
         slots = {n: getattr(self, n) for n in copyreg._slotnames(type(self))
                  if n != "_call" and hasattr(self, n)}
-        slots["_call"] = None
         return getattr(self, "__dict__", None) or None, slots
+
+    def __setstate__(self, state):
+        self._call = None
+        for part in state:
+            for name, value in (part or {}).items():
+                setattr(self, name, value)
 
     # -- construction -------------------------------------------------------
     @staticmethod
