@@ -336,10 +336,10 @@ hipError_t launch_sweep_a(int A, int W, SweepRunner &run, const void *d_blob, ui
   }
 }
 
-bool all_finite(const std::vector<Gate> &gates, const std::vector<int> &which) {
-  for (int gi : which)
-    for (const cd &v : gates[gi].m)
-      if (!std::isfinite(v.re) || !std::isfinite(v.im)) return false;
+template <typename R>
+bool all_finite(const std::vector<R> &v) {
+  for (const R &x : v)
+    if (!std::isfinite(x)) return false;
   return true;
 }
 
@@ -705,8 +705,9 @@ hipError_t execute_t(SweepRunner &run, const std::vector<Gate> &gates, uint64_t 
       std::fprintf(stderr, " ops %u\n", h.nops);
     }
     h.npool = (uint32_t)pool.size();
-    if ((run.known || run.fresh) && !all_finite(gates, pl.gates)) {
-      // (an infinity or NaN makes more of the zeros than zeros)
+    if ((run.known || run.fresh) && !all_finite(pool)) {
+      // An infinity or NaN makes more of the zeros than zeros.  (Told from
+      // the values that the kernel takes: merged, in the state's precision.)
       hipError_t e = sweep_settle(run);
       if (e != hipSuccess) return e;
     }

@@ -196,6 +196,39 @@ def test_gates_from_a_basis_state(n, dtype):
     assert abs(abs(c.amplitudes([k])[0]) - 1) < (1e-14 if dtype == "c128" else 1e-6)
 
 
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+@pytest.mark.parametrize("n", [5, 12, 14, 16])
+@pytest.mark.parametrize("what", ["inf", "nan", "large"])
+def test_entries_that_are_not_finite_from_a_basis_state(n, dtype, what):
+    """An infinity or NaN makes NaN of a zero: a gate with one runs on the
+    whole state, as on a state given amplitude by amplitude.  So do entries
+    that are finite in the matrix and not in the kernels: beyond complex64's
+    range, or in the product of two gates merged into one."""
+    big = {"inf": np.inf, "nan": np.nan, "large": 1e200}[what]
+    lists = [[Operation(np.array([[1, big], [0, 1]]), [q])] for q in (0, n - 1)]
+    lists.append([Operation(np.diag([1, big]), [n // 2])])
+    lists.append([Operation(np.array([[1, big], [0, 1]]), [n - 1])] * 2)
+    lists.append([Operation(np.diag([big, 1]), [n - 1]),
+                  Operation(np.array([[big, 0], [big, 1]]), [n - 1])])
+    lists.append([Operation(np.array([[0, 1], [1, 0]]), [n - 2]),
+                  Operation.controlled([n - 2], np.array([[1, 2], [big, 1]]), [1])])
+    e = np.zeros(1 << n, dtype=np.complex128)
+    e[0] = 1
+    hs = [ops.hadamard(q) for q in range(n)]
+    for opl in lists:
+        for more in ([], hs[: n // 2], hs):
+            got = []
+            for given in (False, True):
+                r = Register.from_int(n, 0, dtype)
+                if given:
+                    r.state = e
+                for op in more + opl + more:
+                    r.apply(op)
+                got.append(r.state)
+                r.close()
+            assert np.array_equal(got[0], got[1], equal_nan=True), (len(opl), len(more))
+
+
 @pytest.mark.parametrize("dtype, k, n", [
     ("c128", 5, 9), ("c128", 5, 10), ("c128", 5, 15), ("c128", 5, 21), ("c128", 6, 9),
     ("c128", 6, 10), ("c128", 6, 12), ("c128", 6, 21), ("c128", 7, 7), ("c128", 7, 13),
