@@ -61,6 +61,7 @@ struct POp {
   int target = 0;
   size_t param = 0;
   qs::Gate fwd, inv;
+  bool unitary = true;  // to 1e-13 (inv undoes fwd)
   int rot_slot = -1;
 };
 
@@ -1524,10 +1525,16 @@ struct RevItem {
   uint64_t x = 0, z = 0;
   int pq = -1;
   bool tile_form = true;
+  bool barrier = false;
   int records = 1, rows = 0, slots = 0;  // slots: of RowSums, in complex64 Z rotations too
 };
 
-RevItem rev_item(const POp &op, size_t index) {
+//
+// A fixed gate that is not unitary keeps its place among all operations, as
+// if it touched every qubit: the gradient before it and after it differ.
+// (A program may put one in front of the rotations, to prepare a state; what
+// the reverse pass does behind it is of no use then.)
+RevItem rev_item(const POp &op, size_t index, int n) {
   RevItem it;
   it.op = index;
   if (op.kind == 1) {
@@ -1558,6 +1565,8 @@ RevItem rev_item(const POp &op, size_t index) {
     it.z = g.cmask;
     it.tile_form = false;
   }
+  it.barrier = !op.unitary;
+  if (it.barrier) it.x = (1ull << n) - 1ull;
   return it;
 }
 
@@ -1730,9 +1739,10 @@ int reverse_blocks(qs_adjoint *c) {
       bool any = false;
       for (const RevItem &it : block) {
         const bool movable = free_of(it, bx, bz);
-        if (movable && it.pq < 0) {
+        if (movable && it.pq < 0 && !(it.barrier && any)) {
           emit_diag(it, d, sg);
           any = true;
+          if (it.barrier) bx = it.x;  // alone in its pass
         } else {
           bx |= it.x;
           bz |= it.z;
@@ -1922,7 +1932,7 @@ int reverse_blocks(qs_adjoint *c) {
     }
     const POp &op = c->circ.ops[ii];
     if (op.kind == 0 && op.inv.kind == qs::Gate::kIdentity) continue;
-    items.push_back(rev_item(op, ii));
+    items.push_back(rev_item(op, ii, n));
   }
   return drain();
 }
@@ -2013,6 +2023,16 @@ int qs_pcircuit_gate(qs_pcircuit *c, const double *matrix, const size_t *targets
     }
   POp op;
   op.kind = 0;
+  for (size_t i = 0; i < D; ++i)
+    for (size_t j = 0; j < D; ++j) {
+      double re = i == j ? -1.0 : 0.0, im = 0.0;  // of row i times row j's conjugate
+      for (size_t e = 0; e < D; ++e) {
+        const double *a = matrix + 2 * (i * D + e), *b = matrix + 2 * (j * D + e);
+        re += a[0] * b[0] + a[1] * b[1];
+        im += a[1] * b[0] - a[0] * b[1];
+      }
+      op.unitary = op.unitary && std::fabs(re) < 1e-13 && std::fabs(im) < 1e-13;
+    }
   op.fwd = qs::classify_matrix(matrix, t.data(), k, 0, 0);
   op.inv = qs::classify_matrix(inv.data(), t.data(), k, 0, 0);
   if ((op.fwd.kind == qs::Gate::kDense && op.fwd.na > 2) ||

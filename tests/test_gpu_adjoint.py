@@ -395,3 +395,44 @@ def test_reverse_blocks_with_every_record(n, dtype, tol):
         d[q] = 1e-4
         want = (fd.energies(th + d) - fd.energies(th - d)) / 2e-4
         assert np.max(np.abs(g[:, q] - want)) < max(tol, 1e-6)
+
+
+def shift_gradients(ex, th):
+    """dE/dtheta by the shift rule, exact for rotations exp(-i t sigma / 2)
+    with a parameter each, in batches of shifted sets."""
+    p = th.shape[1]
+    out = np.empty_like(th)
+    for b, t in enumerate(th):
+        e = ex.energies(np.concatenate([t + np.eye(p) * np.pi / 2, t - np.eye(p) * np.pi / 2]))
+        out[b] = (e[:p] - e[p:]) / 2
+    return out
+
+
+@pytest.mark.parametrize("dtype,tol", [("c128", 1e-11), ("c64", 1e-4)])
+@pytest.mark.parametrize("n", [3, 6, 9, 12, 14])
+def test_gates_that_are_not_unitary_before_the_rotations(n, dtype, tol):
+    """A preparation that is no unitary (columns of zeros, weights on the
+    diagonal) in front of the rotations: nothing that commutes with it may be
+    taken after it in the reverse pass."""
+    rng = np.random.default_rng(600 + n)
+    pc = ParamCircuit(n)
+    for q in range(n):
+        pc.gate(np.array([[0.8, 0.1], [0.5j, -0.3]]), [q])
+    pc.gate(np.diag([1.0, 0.7]), [n - 1])
+    pc.gate(np.diag([1.0, 1.0, 1.0, 0.4j]), [0, n - 1])
+    pc.gate(np.diag([1.0, 0.9, 0.8, 0.6]), [1, 0])
+    for layer in range(3):
+        for q in range(n):
+            pc.rotation("yxz"[(q + layer) % 3], q, pc.nparams)
+            pc.rotation("z", q, pc.nparams)
+        for q in range(n - 1):
+            g = ops.cnot(q, q + 1) if q % 2 else ops.cz(q, q + 1)
+            pc.gate(g.matrix(), g.targets())
+    masks, coeffs = circuits.zz_chain_observable(n)
+    th = rng.random((2, pc.nparams)) * 6.2
+    ex = Expectation(pc, masks, coeffs, dtype=dtype)
+    ex.forward(th)
+    g = ex.backward()
+    want = shift_gradients(Expectation(pc, masks, coeffs, dtype="c128"), th)
+    assert np.max(np.abs(want)) > 1e-4
+    assert np.max(np.abs(g - want)) < tol * n
