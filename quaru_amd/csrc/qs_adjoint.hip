@@ -1184,7 +1184,7 @@ struct qs_adjoint {
   };
   std::vector<Buf> bufs;
   hipError_t take(void **p, size_t bytes) {
-    const hipError_t e = qs::pool_malloc(p, bytes);
+    const hipError_t e = qs::pool_malloc(p, bytes, ws->device);
     if (e == hipSuccess) bufs.push_back({*p, bytes});
     return e;
   }
@@ -2153,7 +2153,9 @@ int qs_adjoint_forward(const qs_pcircuit *c, const double *thetas, size_t batch,
   a->P = c->nparams;
   a->dtype = dtype;
   a->checkpoint_every = checkpoint_every;
-  hipError_t e = qs::workspace_get(&a->ws);
+  int device = 0;
+  hipError_t e = hipGetDevice(&device);
+  if (e == hipSuccess) e = qs::workspace_get(&a->ws, device);
   if (e != hipSuccess) {
     delete a;
     return qs::set_hip_error(e, "adjoint workspace");

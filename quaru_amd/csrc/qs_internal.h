@@ -71,10 +71,10 @@ constexpr size_t kRedCount = 4 * kReduceBlocks + 64;
 constexpr size_t kRedDoubles = kRedCount + 8;
 constexpr size_t kRingBytes = 8u << 20;
 
-// hipMalloc and hipFree on the current device through the pool of kept
-// blocks.  pool_free takes the size and device of the allocation; no GPU work
-// may use the block any more.
-hipError_t pool_malloc(void **out, size_t bytes);
+// hipMalloc and hipFree on `device` (whichever is current) through the pool of
+// kept blocks.  pool_free takes the size and device of the allocation; no GPU
+// work may use the block any more.
+hipError_t pool_malloc(void **out, size_t bytes, int device);
 void pool_free(void *p, size_t bytes, int device);
 
 // What every register and adjoint pass needs beside its states: a stream, an
@@ -87,7 +87,7 @@ struct Workspace {
   double *d_red = nullptr, *h_red = nullptr;
 };
 
-hipError_t workspace_get(Workspace **out);
+hipError_t workspace_get(Workspace **out, int device);
 void workspace_put(Workspace *w);
 
 // Classify a dense 2^k x 2^k complex128 matrix on `targets` (qs_register.hip);

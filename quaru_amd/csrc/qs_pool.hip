@@ -108,6 +108,24 @@ void give_back(Pool &p, std::unique_lock<std::mutex> &lk, const std::list<Block>
   p.freed.notify_all();
 }
 
+// Makes `device` current for a block of code.
+struct OnDevice {
+  int before = 0;
+  bool moved = false;
+  hipError_t error;
+  explicit OnDevice(int device) {
+    error = hipGetDevice(&before);
+    if (error != hipSuccess || before == device) return;
+    error = hipSetDevice(device);
+    moved = error == hipSuccess;
+  }
+  ~OnDevice() {
+    if (moved) (void)hipSetDevice(before);
+  }
+  OnDevice(const OnDevice &) = delete;
+  OnDevice &operator=(const OnDevice &) = delete;
+};
+
 bool out_of_memory(hipError_t e) {
   return e == hipErrorOutOfMemory || e == hipErrorMemoryAllocation;
 }
@@ -156,11 +174,8 @@ bool idle_thread_runs(Pool &p) {
 
 }  // namespace
 
-hipError_t pool_malloc(void **out, size_t bytes) {
+hipError_t pool_malloc(void **out, size_t bytes, int device) {
   *out = nullptr;
-  int device = 0;
-  hipError_t e = hipGetDevice(&device);
-  if (e != hipSuccess) return e;
   Pool &p = pool();
   {
     std::lock_guard<std::mutex> lk(p.mu);
@@ -174,7 +189,9 @@ hipError_t pool_malloc(void **out, size_t bytes) {
       }
     }
   }
-  e = hipMalloc(out, bytes);
+  const OnDevice on(device);
+  if (on.error != hipSuccess) return on.error;
+  const hipError_t e = hipMalloc(out, bytes);
   if (!out_of_memory(e)) return e;
   (void)hipGetLastError();
   std::unique_lock<std::mutex> lk(p.mu);
@@ -230,11 +247,8 @@ void destroy(Workspace *w) {
 
 }  // namespace
 
-hipError_t workspace_get(Workspace **out) {
+hipError_t workspace_get(Workspace **out, int device) {
   *out = nullptr;
-  int device = 0;
-  hipError_t e = hipGetDevice(&device);
-  if (e != hipSuccess) return e;
   Pool &p = pool();
   {
     std::lock_guard<std::mutex> lk(p.mu);
@@ -247,10 +261,12 @@ hipError_t workspace_get(Workspace **out) {
   }
   Workspace *w = new Workspace();
   w->device = device;
-  e = hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking);
-  if (e == hipSuccess) e = pool_malloc((void **)&w->d_red, kRedDoubles * sizeof(double));
+  const OnDevice on(device);
+  hipError_t e = on.error;
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&w->stream, hipStreamNonBlocking);
+  if (e == hipSuccess) e = pool_malloc((void **)&w->d_red, kRedDoubles * sizeof(double), device);
   if (e == hipSuccess) e = hipHostMalloc((void **)&w->h_red, 64 * sizeof(double));
-  if (e == hipSuccess) e = pool_malloc((void **)&w->d_ring, kRingBytes);
+  if (e == hipSuccess) e = pool_malloc((void **)&w->d_ring, kRingBytes, device);
   if (e == hipSuccess) e = hipHostMalloc((void **)&w->h_ring, kRingBytes);
   // measurement slots that nothing has written read 0
   if (e == hipSuccess)

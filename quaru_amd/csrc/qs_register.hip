@@ -147,7 +147,7 @@ int alloc_register(size_t n, int dtype, qs_register **out) {
   r->dtype = dtype;
   r->len = 1ull << n;
   hipError_t e = hipGetDevice(&r->device);
-  if (e == hipSuccess) e = qs::workspace_get(&r->ws);
+  if (e == hipSuccess) e = qs::workspace_get(&r->ws, r->device);
   if (e == hipSuccess) {
     r->stream = r->ws->stream;
     r->d_red = r->ws->d_red;
@@ -155,7 +155,7 @@ int alloc_register(size_t n, int dtype, qs_register **out) {
     r->d_ring = r->ws->d_ring;
     r->h_ring = r->ws->h_ring;
     r->ring_cap = qs::kRingBytes;
-    e = qs::pool_malloc(&r->psi, r->state_bytes());
+    e = qs::pool_malloc(&r->psi, r->state_bytes(), r->device);
   }
   if (e != hipSuccess) {
     qs_register_free(r);
@@ -175,7 +175,7 @@ hipError_t ensure_big(qs_register *r, size_t bytes, double **out) {
     qs::pool_free(r->d_big, r->d_big_bytes, r->device);
     r->d_big = nullptr;
     r->d_big_bytes = 0;
-    e = qs::pool_malloc((void **)&r->d_big, bytes);
+    e = qs::pool_malloc((void **)&r->d_big, bytes, r->device);
     if (e != hipSuccess) return e;
     r->d_big_bytes = bytes;
   }
@@ -219,7 +219,7 @@ hipError_t big_upload(qs_register *r, const void *src, size_t bytes, void **dev)
     qs::pool_free(r->d_upload, r->d_upload_bytes, r->device);
     r->d_upload = nullptr;
     r->d_upload_bytes = 0;
-    e = qs::pool_malloc(&r->d_upload, bytes);
+    e = qs::pool_malloc(&r->d_upload, bytes, r->device);
     if (e != hipSuccess) return e;
     r->d_upload_bytes = bytes;
   }
@@ -564,7 +564,7 @@ hipError_t launch_one(qs_register *r, const Gate &g) {
                                                      : big_upload(r, buf.data(), buf.size(), &dm);
       if (e != hipSuccess) return e;
       if (!r->scratch) {
-        e = qs::pool_malloc(&r->scratch, r->state_bytes());
+        e = qs::pool_malloc(&r->scratch, r->state_bytes(), r->device);
         if (e != hipSuccess) return e;
       }
       ++r->st_kernels;
@@ -593,7 +593,7 @@ hipError_t launch_one(qs_register *r, const Gate &g) {
                                        : big_upload(r, src, bytes, &dm);
         if (e != hipSuccess) return e;
         if (!r->scratch && qs::dense_needs_scratch(std::is_same<T, float>::value, r->n, g)) {
-          e = qs::pool_malloc(&r->scratch, r->state_bytes());
+          e = qs::pool_malloc(&r->scratch, r->state_bytes(), r->device);
           if (e != hipSuccess) return e;
         }
       }

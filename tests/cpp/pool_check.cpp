@@ -36,9 +36,9 @@ constexpr size_t MiB = 1ull << 20, GiB = 1ull << 30;
     }                                                              \
   } while (0)
 
-void *take(size_t bytes) {
+void *take(size_t bytes, int device = 0) {
   void *p = nullptr;
-  return pool_malloc(&p, bytes) == hipSuccess ? p : nullptr;
+  return pool_malloc(&p, bytes, device) == hipSuccess ? p : nullptr;
 }
 
 void wait_ms(int ms) { std::this_thread::sleep_for(std::chrono::milliseconds(ms)); }
@@ -147,6 +147,22 @@ int freeing() {
   return 0;
 }
 
+// Memory is its owner's device's, whatever device the calling thread has
+// current (a register's buffers grow in calls made at any time).
+int device() {
+  fake::current = 1;
+  void *a = take(GiB, 0);
+  CHECK(fake::device_of(a) == 0 && fake::current == 1);
+  pool_free(a, GiB, 0);
+  void *b = take(GiB, 1);
+  CHECK(fake::device_of(b) == 1 && b != a);
+  fake::current = 0;
+  pool_free(b, GiB, 1);
+  CHECK(take(GiB, 0) == a && take(GiB, 1) == b);
+  CHECK(!take(64 * GiB, 1) && fake::current == 0);
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -156,6 +172,7 @@ int main(int argc, char **argv) {
   if (!std::strcmp(what, "idle")) rc = idle();
   if (!std::strcmp(what, "capture")) rc = capture();
   if (!std::strcmp(what, "freeing")) rc = freeing();
+  if (!std::strcmp(what, "device")) rc = device();
   if (!std::strcmp(what, "no_thread")) rc = no_thread();
   if (rc == 0) std::printf("ok\n");
   return rc;
