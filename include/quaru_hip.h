@@ -82,6 +82,16 @@ int qs_register_clone(qs_register *src, qs_register **out);
 /* Drop.  Accepts NULL. */
 void qs_register_free(qs_register *r);
 
+/* Device memory of freed registers and adjoint passes is kept for the next
+ * ones: at most an eighth of the device's memory, each block for a second (64
+ * MiB and a few workspaces of 8 MiB stay), given back at once when an
+ * allocation of this library fails.  A thread of the library frees what has
+ * lain for a second; such a free waits for the device, and leaves a stream
+ * capture of another thread alone.  Other users of the GPU (another library,
+ * another process) cannot have the kept memory until then:
+ * qs_release_memory() gives all of it back before it returns. */
+void qs_release_memory(void);
+
 /* Register::size (src/register.rs:404-406). */
 size_t qs_register_size(const qs_register *r);
 

@@ -47,6 +47,7 @@ SIGNATURES = {
     "qs_register_from_qubits": (_I, [_P, _P, _S, _I, _PP]),
     "qs_register_clone": (_I, [_P, _PP]),
     "qs_register_free": (None, [_P]),
+    "qs_release_memory": (None, []),
     "qs_register_size": (_S, [_P]),
     "qs_register_dtype": (_I, [_P]),
     "qs_apply": (_I, [_P, _P, _S, _S, _P, _S]),

@@ -77,6 +77,9 @@ constexpr size_t kRingBytes = 8u << 20;
 hipError_t pool_malloc(void **out, size_t bytes, int device);
 void pool_free(void *p, size_t bytes, int device);
 
+// Give back everything that is kept (blocks and workspaces).
+void pool_release();
+
 // What every register and adjoint pass needs beside its states: a stream, an
 // upload ring (pinned host buffer mirrored in device memory) and buffers of
 // the reductions.  put: the stream has been drained.

@@ -13,9 +13,11 @@
 // memory, the oldest leave first; a block that has lain here for a second is
 // given back, whatever goes on with the others, as long as more than
 // kIdleKept bytes are kept; and when an allocation of this library fails,
-// everything kept on the device is given back before it is tried again.  A block is handed in only when no GPU work
-// uses it any more (its owner has drained its stream), so any thread and any
-// stream may take it next.  Contents are whatever was there.
+// everything kept on the device is given back before it is tried again.  A
+// program that needs the memory for something else at once calls
+// qs_release_memory.  A block is handed in only when no GPU work uses it any
+// more (its owner has drained its stream), so any thread and any stream may
+// take it next.  Contents are whatever was there.
 #include <hip/hip_runtime.h>
 
 #include <chrono>
@@ -58,6 +60,7 @@ struct Pool {
   int freeing = 0;               // threads that are giving blocks back
   std::condition_variable freed;
   bool started = false, exits = false, stopping = false;
+  Pool() { spaces.reserve(kMaxSpaces * kMaxDevices); }  // putting one back throws nothing
 };
 
 // Never destroyed: threads may free their registers while the process exits.
@@ -286,12 +289,26 @@ void workspace_put(Workspace *w) {
     std::lock_guard<std::mutex> lk(p.mu);
     size_t n = 0;
     for (const Workspace *s : p.spaces) n += s->device == w->device;
-    if (n < kMaxSpaces) {
+    if (n < kMaxSpaces && p.spaces.size() < p.spaces.capacity()) {
       p.spaces.push_back(w);
       return;
     }
   }
   destroy(w);
+}
+
+void pool_release() {
+  Pool &p = pool();
+  std::unique_lock<std::mutex> lk(p.mu);
+  while (!p.spaces.empty()) {
+    Workspace *w = p.spaces.back();
+    p.spaces.pop_back();
+    lk.unlock();
+    destroy(w);
+    lk.lock();
+  }
+  give_back(p, lk, take_out(p, -1, 0));
+  p.freed.wait(lk, [&] { return p.freeing == 0; });
 }
 
 }  // namespace qs

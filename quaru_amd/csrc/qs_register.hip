@@ -1140,6 +1140,8 @@ void qs_register_free(qs_register *r) {
   delete r;
 }
 
+void qs_release_memory(void) { qs::pool_release(); }
+
 size_t qs_register_size(const qs_register *r) { return r ? (size_t)r->n : 0; }
 
 int qs_register_dtype(const qs_register *r) { return r ? r->dtype : -1; }

@@ -135,6 +135,13 @@ def _call_of(op: Operation):
     return False, (m.ctypes.data, rows, cols, t.ctypes.data, t.size), (m, t)
 
 
+def release_memory() -> None:
+    """Give the device memory that is kept of closed registers and adjoint
+    passes back now (at most an eighth of the device, otherwise after a
+    second), for another library or process that needs it."""
+    _lib.load().qs_release_memory()
+
+
 class Register:
     """A quantum register of ``n`` qubits whose state lives on the GPU."""
 

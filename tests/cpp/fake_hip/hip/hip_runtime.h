@@ -49,6 +49,7 @@ inline Runtime &rt() {
 inline thread_local int current = 0;
 inline thread_local hipStreamCaptureMode mode = hipStreamCaptureModeGlobal;
 inline std::atomic<int> free_ms{0};  // how long a free waits for the device
+inline std::atomic<int> streams{0}, host_blocks{0};
 
 // Device of a live block, -1: none there.
 inline int device_of(void *p) {
@@ -121,18 +122,22 @@ inline hipError_t hipFree(void *p) {
 template <typename T>
 hipError_t hipHostMalloc(T **out, size_t) {
   *out = reinterpret_cast<T *>(new char[16]);
+  ++fake::host_blocks;
   return hipSuccess;
 }
 inline hipError_t hipHostFree(void *p) {
   delete[] static_cast<char *>(p);
+  --fake::host_blocks;
   return hipSuccess;
 }
 inline hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) {
   *s = reinterpret_cast<hipStream_t>(new char[1]);
+  ++fake::streams;
   return hipSuccess;
 }
 inline hipError_t hipStreamDestroy(hipStream_t s) {
   delete[] reinterpret_cast<char *>(s);
+  --fake::streams;
   return hipSuccess;
 }
 inline hipError_t hipMemsetAsync(void *, int, size_t, hipStream_t) { return hipSuccess; }

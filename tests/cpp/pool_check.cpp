@@ -163,6 +163,24 @@ int device() {
   return 0;
 }
 
+// Everything kept goes back when a program asks for it, also what the idle
+// thread leaves and workspaces of closed registers; blocks in use stay.
+int release() {
+  Workspace *w[6];
+  for (Workspace *&x : w) CHECK(workspace_get(&x, &x - w < 3 ? 0 : 1) == hipSuccess);
+  void *a = take(MiB), *b = take(GiB), *mine = take(2 * GiB);
+  pool_free(a, MiB, 0);
+  pool_free(b, GiB, 0);
+  for (Workspace *x : w) workspace_put(x);
+  CHECK(fake::used(0) > 3 * GiB && fake::used(1) > 0);
+  pool_release();
+  CHECK(fake::used(0) == 2 * GiB && fake::used(1) == 0);
+  CHECK(fake::device_of(mine) == 0 && fake::streams == 0 && fake::host_blocks == 0);
+  CHECK(workspace_get(&w[0], 0) == hipSuccess);
+  workspace_put(w[0]);
+  return 0;
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
@@ -173,6 +191,7 @@ int main(int argc, char **argv) {
   if (!std::strcmp(what, "capture")) rc = capture();
   if (!std::strcmp(what, "freeing")) rc = freeing();
   if (!std::strcmp(what, "device")) rc = device();
+  if (!std::strcmp(what, "release")) rc = release();
   if (!std::strcmp(what, "no_thread")) rc = no_thread();
   if (rc == 0) std::printf("ok\n");
   return rc;

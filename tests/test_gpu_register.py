@@ -1184,6 +1184,31 @@ def test_registers_in_turn_share_no_contents():
     assert not failures
 
 
+def test_kept_memory_is_released_on_demand():
+    import ctypes
+
+    from quaru_amd import release_memory
+
+    hip = ctypes.CDLL("libamdhip64.so.7")  # the library's own runtime
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    Register.from_int(26, 0).sync().close()  # loads what the library runs
+    release_memory()
+    before = free()
+    r = Register.from_int(26, 0)  # 1 GiB
+    r.sync()
+    r.close()
+    assert free() <= before - (1 << 30)  # kept for the next one
+    release_memory()
+    assert free() > before - (1 << 27)
+    s = Register.from_int(12, 3)  # what goes on is as before
+    assert s.measure(0) and s.measure(1) and not s.measure(2)
+
+
 @pytest.mark.parametrize("off", [0.0, 1e-9])
 @pytest.mark.parametrize("k", [2, 5, 6, 7])
 def test_products_of_one_qubit_gates(k, off):

@@ -21,7 +21,7 @@ def exe(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("rule", ["bounds", "idle", "capture", "no_thread", "freeing", "device"])
+@pytest.mark.parametrize("rule", ["bounds", "idle", "capture", "no_thread", "freeing", "device", "release"])
 def test_kept_memory(exe, rule):
     res = subprocess.run([exe, rule], capture_output=True, text=True, timeout=60)
     assert res.returncode == 0 and res.stdout == "ok\n", res.stdout + res.stderr
