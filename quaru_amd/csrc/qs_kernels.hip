@@ -629,9 +629,9 @@ __device__ __forceinline__ int stage_phys(int s) { return s ^ ((s >> 5) & 31); }
 
 // K = 3..5 active targets (complex128: those that k_dense_tile does not take)
 // when low index bits are fixed (active or controls): the direct kernel's
-// loads would then stride by 2^(lowest free bit) amplitudes per lane.  One wave stages 64 groups through LDS with
-// loads over the block's lowest index bits, each lane computes its own group
-// from registers (matrix on scalar loads, as in k_gatek), writes its outputs
+// loads would then stride by 2^(lowest free bit) amplitudes per lane.  One
+// wave stages 64 groups through LDS with loads over the block's lowest index
+// bits, each lane computes its own group from registers (matrix on scalar loads, as in k_gatek), writes its outputs
 // back to its own slots, and the wave stores the block the way it loaded it.
 template <typename R, int K, bool kReal, bool kNT>
 __global__ __launch_bounds__(64) void k_gatek_staged(typename V2<R>::T *__restrict__ psi,
@@ -1068,34 +1068,49 @@ __global__ __launch_bounds__(256) void k_dense_f32(float2 *psi, const float2 *sr
 
 // Which kernel a dense gate on na >= 4 qubits takes, nfree index bits being
 // neither its targets nor its controls; low: a fixed bit among the lowest 4;
-// big: a streaming state.  Measured, complex128 (us per gate with its upload):
+// big: a streaming state; eight: eight_streams below.  Measured, complex128
+// (us per gate with its upload):
 //   5 qubits, 15-qubit state: tiles 10-11, k_gatek and its staged form 40;
-//   24 qubits: 80-100 against 114 (free low bits) and 156-184; 27 qubits:
-//   800 against 950-1160 (low bits fixed), but 870-1040 against 780-800 of
-//   k_gatek's long runs (low bits free), which it keeps.
-//   4 qubits: 9.5 against 13-19 up to 18 qubits, 75 against 81-87 at 24; at
-//   28 qubits 1580-1850 against 1460-1600, so streaming states keep theirs.
+//   24 qubits: 95 against 108 (free low bits) and 95-115 against 180; 27
+//   qubits: 800-1020 against 1170 (low bits fixed), but 870-1040 against
+//   780-800 of k_gatek's long runs (low bits free), which it keeps.
+//   4 qubits, free low bits: 13 against 17 up to 19 qubits, 32 against 39 at
+//   20; 18 either way at 21, 27-33 against 25-29 at 22, 44-55 against 42-48 at
+//   23, 75-90 against 72-82 at 24, so k_gatek from 21 on.  Low bits fixed:
+//   27-31 against 37-39 at 22, 42-51 against 53-57 at 23, 74-82 against 83-87
+//   at 24; at 28 qubits 1580-1850 against 1460-1600, so streaming states keep
+//   theirs.
 //   6 qubits: 32 columns per tile from 20 qubits on (33 against 37 at 20, 67
 //   against 74 at 22, 1200 against 1240 at 27), 16 below (24 against 26).
 // Larger products take 32 columns per workgroup when that still fills the
 // chip.  Complex64: 64 x 64 outputs per workgroup from 20 qubits on.
 enum DenseForm { kDenseDirect, kDenseTile, kDenseTileSmall, kDenseWide, kDenseNarrow };
 
-static DenseForm dense_form(bool c64, int na, int nfree, bool low, bool big) {
+static DenseForm dense_form(bool c64, int na, int nfree, bool low, bool big, bool eight) {
   if (c64) {
     if (na <= 5) return kDenseDirect;
     return nfree >= 6 && na + nfree >= 20 ? kDenseWide : kDenseNarrow;
   }
-  if (na == 4) return nfree >= 6 && !big ? kDenseTile : kDenseDirect;
-  if (na == 5) return nfree >= 5 && (low || !big) ? kDenseTile : kDenseDirect;
+  if (na == 4)
+    return nfree >= 6 && !big && !eight && (low || nfree <= 16) ? kDenseTile : kDenseDirect;
+  if (na == 5) return nfree >= 5 && (low || (!big && !eight)) ? kDenseTile : kDenseDirect;
   if (na == 6 && nfree >= 4) return nfree < 14 ? kDenseTileSmall : kDenseTile;
   return nfree >= 5 && na + nfree >= 17 ? kDenseWide : kDenseNarrow;
+}
+
+// Whether a tile's rows are 8 streams 4 MiB or more apart, each a run of a few
+// KiB, of a state just the size of the last-level cache (2^24 amplitudes of
+// complex128).  There, tiles take 91-96 us (4 qubits, low bits fixed; 5
+// qubits, low bits free) and the kernels without tiles 85-91 (4 qubits) and
+// 87-88; with 4 or 16 streams, or shorter runs, tiles are faster as elsewhere.
+static bool eight_streams(int n, uint64_t active) {
+  return n == 24 && __builtin_popcountll(active >> 18) == 3 && (active & 0x3FF00ull) == 0;
 }
 
 bool dense_needs_scratch(bool c64, int n, const Gate &g) {
   if (g.na <= 5) return false;
   const Fixed fx = make_fixed(g.cmask | active_mask(g), g.cval);
-  const DenseForm f = dense_form(c64, g.na, n - fx.nf, false, false);
+  const DenseForm f = dense_form(c64, g.na, n - fx.nf, false, false, false);
   if (c64) return !(g.na == 6 && f == kDenseWide);
   return f != kDenseTile && f != kDenseTileSmall;
 }
@@ -1244,7 +1259,8 @@ hipError_t launch_gate_dense(void *psi_v, int n, const Gate &g, void *d_mat, voi
     for (const cd &v : g.m) real = real && v.im == 0.0;
     if constexpr (std::is_same<R, double>::value) {
       if (g.na >= 4 &&
-          dense_form(false, g.na, nfree, (fx_mask(fx) & 0xFull) != 0, big) == kDenseTile) {
+          dense_form(false, g.na, nfree, (fx_mask(fx) & 0xFull) != 0, big,
+                     eight_streams(n, active_mask(g))) == kDenseTile) {
         if (g.na == 4)
           launch_dense_tile<4, 6>(psi, nfree, fx, ax, real, big, (const double2 *)m, s);
         else
@@ -1299,7 +1315,7 @@ hipError_t launch_gate_dense(void *psi_v, int n, const Gate &g, void *d_mat, voi
   } else {
     const Fixed ax = active_positions(g);
     const T *m = (const T *)d_mat;
-    const DenseForm f = dense_form(std::is_same<R, float>::value, g.na, nfree, false, big);
+    const DenseForm f = dense_form(std::is_same<R, float>::value, g.na, nfree, false, big, false);
     const T *src = psi;
     if (dense_needs_scratch(std::is_same<R, float>::value, n, g)) {
       hipError_t e = hipMemcpyAsync(scratch, psi, sizeof(T) << n, hipMemcpyDeviceToDevice, s);

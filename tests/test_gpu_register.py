@@ -259,6 +259,47 @@ def test_dense_blocks_of_every_form(dtype, k, n):
         assert infid(r.state, ref) < 1e-6
 
 
+@pytest.mark.parametrize("n, targets, real, controls", [
+    # 20 and 21, 24 qubits: either side of the lines between the kernels of
+    # blocks on 4 and 5 qubits; 25: streaming states, the tile kernel's
+    # nontemporal forms (low bits fixed, 6 targets)
+    (20, [16, 5, 9, 12], False, []), (21, [16, 5, 9, 12], False, []),
+    (24, [21, 0, 23, 22], False, []), (24, [0, 17, 23, 22], True, []),
+    (24, [6, 21, 7, 23, 22], False, []), (24, [4, 9, 21, 22, 23], False, []),
+    (25, [0, 24, 3, 11, 7], False, []), (25, [24, 1, 23, 2, 20], True, []),
+    (25, [2, 3, 17, 8, 24], False, [0, 12]), (25, [24, 6, 0, 14, 9, 22], False, []),
+    (25, [5, 4, 3, 2, 1, 0], True, []), (25, [10, 11, 12, 13, 14, 15], False, [3, 24])])
+def test_dense_blocks_on_large_states(n, targets, real, controls):
+    """Blocks of 4 to 6 qubits on states up to a streaming one: groups of
+    amplitudes drawn from the whole state against the product in numpy."""
+    rng = np.random.default_rng(1500 + n + 7 * sum(targets))
+    k = len(targets)
+    m = (random_orthogonal if real else random_unitary)(rng, 1 << k)
+    psi = np.empty((1 << n, 2))
+    rng.standard_normal(out=psi)
+    psi = psi.view(np.complex128).reshape(-1) * 2 ** (-(n + 1) / 2)
+    r = Register.new([False] * n)
+    r.state = psi
+    if controls:
+        r.apply(ops.Operation.controlled(controls, m, targets))
+    else:
+        r.apply(ops.Operation(m, targets))
+    mask = sum(1 << t for t in targets)
+    cmask = sum(1 << c for c in controls)
+    base = rng.integers(0, 1 << n, 3000) & ~mask
+    base[:2] = [0, ((1 << n) - 1) & ~mask]
+    base[1000:] |= cmask
+    off = np.array([sum(1 << t for j, t in enumerate(targets) if (i >> j) & 1)
+                    for i in range(1 << k)])
+    idx = base[:, None] | off[None, :]
+    x = psi[idx]
+    on = (base & cmask) == cmask
+    want = np.where(on[:, None], x @ m.T, x)
+    assert on.any() and np.max(np.abs(r.amplitudes(idx.reshape(-1)).reshape(x.shape) - want)) < TOL
+    assert abs(r.norm_sqr() - np.sum(psi.real ** 2 + psi.imag ** 2)) < 1e-11
+    r.close()
+
+
 @pytest.mark.parametrize("n", [12, 14])
 def test_c64_complex_5q_blocks_matrix_cores(n):
     """Complex 32 x 32 blocks in complex64 with the 5 lowest index bits free
