@@ -1545,20 +1545,36 @@ static inline bool reduce_blocked(uint64_t len) {
   return len >= (uint64_t)kReduceBlocks * kRedTrip;
 }
 
+// What becomes of a split's sums: {prob_0, prob_1} go to `host`, or, with a
+// slot, the outcome is decided here (src/register.rs:317-321: x > prob_0),
+// stored there and left with its scale in `coll` for the collapse.
+__device__ __forceinline__ void split_result(const double (&v)[2], const SplitEnd &end) {
+  if (threadIdx.x != 0) return;
+  if (end.host) {
+    end.host[0] = v[0];
+    end.host[1] = v[1];
+  }
+  if (end.slot) {
+    const int res = end.x > v[0];
+    end.coll[0] = (double)res;
+    end.coll[1] = sqrt(res ? v[1] : v[0]);
+    *end.slot = (unsigned char)res;
+  }
+}
+
 // The end of a split over all blocks: the partials go to `part`, and the
 // block that comes last (it counts them, and leaves the counter at 0) adds
-// them up in the order of k_finish.  {prob_0, prob_1} go to `host`, or, with a
-// slot, the outcome is decided here (src/register.rs:317-321: x > prob_0),
-// stored there and left with its scale in `coll` for the collapse.  Against a
-// kernel of its own for the sums, a copy to the host and a kernel for the
-// decision: a measurement of 12 qubits is one launch of 5.0 us, was three of
-// 6.5; a deferred one of up to 8 qubits one launch of 2.4 us with its
-// collapse, was four of 6.6 (teleportation of one qubit 101 us, 147).
+// them up in the order of k_finish.  Without a counter, k_split_finish does.
 // Returns whether this block was the last; v holds the sums on its threads.
 __device__ __forceinline__ bool split_end(double (&v)[2], double (*sh)[kBlock],
                                           double *__restrict__ part, const SplitEnd &end) {
   __shared__ bool last;
   if (gridDim.x > 1) {
+    if (!end.count) {
+      if (threadIdx.x == 0)
+        for (int c = 0; c < 2; ++c) part[2 * blockIdx.x + c] = v[c];
+      return false;
+    }
     if (threadIdx.x == 0) {
       for (int c = 0; c < 2; ++c)
         __hip_atomic_store(part + 2 * blockIdx.x + c, v[c], __ATOMIC_RELAXED,
@@ -1576,19 +1592,39 @@ __device__ __forceinline__ bool split_end(double (&v)[2], double (*sh)[kBlock],
     if (threadIdx.x == 0)
       __hip_atomic_store(end.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  if (threadIdx.x == 0) {
-    if (end.host) {
-      end.host[0] = v[0];
-      end.host[1] = v[1];
-    }
-    if (end.slot) {
-      const int res = end.x > v[0];
-      end.coll[0] = (double)res;
-      end.coll[1] = sqrt(res ? v[1] : v[0]);
-      *end.slot = (unsigned char)res;
-    }
-  }
+  split_result(v, end);
   return true;
+}
+
+__global__ __launch_bounds__(kBlock) void k_split_finish(const double *__restrict__ part, int nblocks,
+                                                         SplitEnd end) {
+  __shared__ double sh[2][kBlock];
+  double v[2] = {0.0, 0.0};
+  for (int b = threadIdx.x; b < nblocks; b += kBlock)
+    for (int c = 0; c < 2; ++c) v[c] += part[2 * b + c];
+  block_sum<2>(v, sh);
+  split_result(v, end);
+}
+
+// Grids up to which the last block takes the sums itself: each block's count
+// is an atomic and a write-back of its XCD's L2, which a large grid pays for
+// hundreds of times.  Twelve measures, complex128: 14 qubits (64 blocks) 197
+// us in one launch each, 213 in two and a copy to the host; 15 qubits 213 us,
+// 198 in two launches (this kernel writes to the host); 18 qubits 463, 214;
+// 22 qubits 894, 417.  A deferred measure of up to 8 qubits is one launch of
+// 2.4 us with its collapse, in four it was 6.6.
+constexpr int kSplitBlocks = 64;
+
+// Runs a split of g blocks, launch(end) being its kernel.
+template <typename F>
+static hipError_t run_split(int g, const SplitEnd &end, const double *d_part, hipStream_t s,
+                            F &&launch) {
+  SplitEnd mine = end;
+  if (g > kSplitBlocks) mine.count = nullptr;
+  launch(mine);
+  if (g > kSplitBlocks)
+    hipLaunchKernelGGL(k_split_finish, dim3(1), dim3(kBlock), 0, s, d_part, g, end);
+  return hipGetLastError();
 }
 
 // Amplitude a of index i after a collapse on bit `target` of outcome `keep`.
@@ -1670,13 +1706,14 @@ hipError_t launch_prob_split(void *psi, int n, int target, double *d_part, const
                              hipStream_t s) {
   const uint64_t len = 1ull << n;
   const int g = reduce_grid(len);
-  if (reduce_blocked(len))
-    hipLaunchKernelGGL((k_prob_split<R, true>), dim3(g), dim3(kBlock), 0, s,
-                       (typename V2<R>::T *)psi, len, target, d_part, end);
-  else
-    hipLaunchKernelGGL((k_prob_split<R, false>), dim3(g), dim3(kBlock), 0, s,
-                       (typename V2<R>::T *)psi, len, target, d_part, end);
-  return hipGetLastError();
+  return run_split(g, end, d_part, s, [&](const SplitEnd &e) {
+    if (reduce_blocked(len))
+      hipLaunchKernelGGL((k_prob_split<R, true>), dim3(g), dim3(kBlock), 0, s,
+                         (typename V2<R>::T *)psi, len, target, d_part, e);
+    else
+      hipLaunchKernelGGL((k_prob_split<R, false>), dim3(g), dim3(kBlock), 0, s,
+                         (typename V2<R>::T *)psi, len, target, d_part, e);
+  });
 }
 
 // The collapse of try_measure (src/register.rs:324-339): zero the amplitudes
@@ -1758,15 +1795,16 @@ hipError_t launch_collapse_split(void *psi, int n, int ctarget, int keep, double
                                  int target, double *d_part, const SplitEnd &end, hipStream_t s) {
   const uint64_t len = 1ull << n;
   const int g = reduce_grid(len);
-  if (reduce_blocked(len))
-    hipLaunchKernelGGL((k_collapse_split<R, true>), dim3(g), dim3(kBlock), 0, s,
-                       (typename V2<R>::T *)psi, len, ctarget, keep, sqrt(total), target, d_part,
-                       end);
-  else
-    hipLaunchKernelGGL((k_collapse_split<R, false>), dim3(g), dim3(kBlock), 0, s,
-                       (typename V2<R>::T *)psi, len, ctarget, keep, sqrt(total), target, d_part,
-                       end);
-  return hipGetLastError();
+  return run_split(g, end, d_part, s, [&](const SplitEnd &e) {
+    if (reduce_blocked(len))
+      hipLaunchKernelGGL((k_collapse_split<R, true>), dim3(g), dim3(kBlock), 0, s,
+                         (typename V2<R>::T *)psi, len, ctarget, keep, sqrt(total), target, d_part,
+                         e);
+    else
+      hipLaunchKernelGGL((k_collapse_split<R, false>), dim3(g), dim3(kBlock), 0, s,
+                         (typename V2<R>::T *)psi, len, ctarget, keep, sqrt(total), target, d_part,
+                         e);
+  });
 }
 
 // k_collapse with its outcome and scale read from device memory.

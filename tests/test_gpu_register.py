@@ -1158,6 +1158,12 @@ def test_measures_of_one_and_many_blocks(n, dtype):
     b.close()
 
 
+@pytest.mark.parametrize("dtype", ["c128", "c64"])
+@pytest.mark.parametrize("n", [14, 15])
+def test_measures_of_the_largest_one_launch_grid_and_the_next(n, dtype):
+    test_measures_of_one_and_many_blocks(n, dtype)
+
+
 def test_measure_deferred_equals_measure():
     import ctypes
     from quaru_amd import EngineError, _lib
