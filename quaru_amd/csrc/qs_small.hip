@@ -36,6 +36,7 @@ using namespace qs::merge;
 
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallPhases = 8;
+constexpr int kSmallMost = 13;  // qubits, complex128
 
 enum : uint32_t { SM_PAIR = 1, SM_DENSE2 = 2, SM_PHASES = 3 };
 // flags of the 2x2 in place j of a pair pass
@@ -347,7 +348,11 @@ hipError_t execute_small_t(SweepRunner &run, const std::vector<Gate> &gates, uin
   int slot[64];
   for (int q = 0; q < 64; ++q) slot[q] = q < n ? kFirstLaneSlot : -1;
   for (size_t at = 0; at < gates.size();) {
-    if (!Builder<R>::takes(gates[at])) {
+    // (one gate alone on the largest state: its own kernel's many workgroups
+    // are faster than one's loads and stores: a 4x4 on 13 qubits 14.0 us with
+    // its synchronisation, 18.2 here; on 12 qubits 15.6 here, 17.3)
+    const bool alone = n >= kSmallMost && !run.fresh && gates.size() == 1;
+    if (alone || !Builder<R>::takes(gates[at])) {
       hipError_t e = launch();
       if (e == hipSuccess) e = sweep_settle(run);
       if (e == hipSuccess) e = run.single(gates[at]);
@@ -391,7 +396,7 @@ bool small_fits(int n, bool c64) {
     return !(v && v[0] == '0');
   }();
   if (!on || n < 2) return false;
-  return c64 ? n < sweep::kLaneBits + sweep_reg_bits(true) : n <= 13;
+  return c64 ? n < sweep::kLaneBits + sweep_reg_bits(true) : n <= kSmallMost;
 }
 
 hipError_t execute_small(SweepRunner &run, const std::vector<Gate> &gates, uint64_t *sweeps) {

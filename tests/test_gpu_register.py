@@ -1329,6 +1329,20 @@ def small_run_ops(rng, n, count):
     return opl
 
 
+@pytest.mark.parametrize("n", [12, 13])
+def test_small_registers_gate_by_gate(n):
+    """Runs of one gate, the first from a basis state: on the largest state
+    of one compute unit by kernels of their own."""
+    rng = np.random.default_rng(4100 + n)
+    r = Register.from_int(n, 5)
+    ref = np.zeros(1 << n, dtype=np.complex128)
+    ref[5] = 1
+    for op in small_run_ops(rng, n, 25):
+        ref = oracle_run(ref, [op])
+        r.apply(op).sync()
+        assert maxdiff(r.state, ref) < TOL
+
+
 @pytest.mark.parametrize("dtype", ["c128", "c64"])
 @pytest.mark.parametrize("n", [2, 3, 5, 6, 8, 10, 12, 13])
 def test_small_registers_in_one_launch(n, dtype):
