@@ -364,7 +364,7 @@ hipError_t execute_small_t(SweepRunner &run, const std::vector<Gate> &gates, uin
     while (end < gates.size() && Builder<R>::takes(gates[end])) ++end;
     std::vector<SweepOp> items(end - at);
     for (size_t k = at; k < end; ++k) items[k - at].g = &gates[k];
-    if (!exact && sweep_merge_ops()) merge_sweep_ops(items, slot, 0);
+    if (!exact && sweep_merge_ops()) merge_sweep_ops<long double>(items, slot, 0);
     for (const SweepOp &o : items) {
       if (!o.alive) {
         if (run.merged) ++*run.merged;

@@ -3,6 +3,7 @@
 // qs_sweep.hip, and by the CPU check of the merge rules in tests/cpp.
 #pragma once
 
+#include <cmath>
 #include <cstdint>
 #include <deque>
 #include <vector>
@@ -57,16 +58,25 @@ struct SweepOp {
   bool alive = true;
 };
 
-inline cd cmul(const cd &a, const cd &b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
-inline cd cadd(const cd &a, const cd &b) { return {a.re + b.re, a.im + b.im}; }
+// Whether a product with m (X, phases of 1, -1, i, -i) rounds nothing.
+inline bool exact2(const cd *m) {
+  auto zero = [](const cd &v) { return v.re == 0 && v.im == 0; };
+  auto unit = [](const cd &v) { return std::fabs(v.re) + std::fabs(v.im) == 1 && v.re * v.im == 0; };
+  return (zero(m[1]) && zero(m[2]) && unit(m[0]) && unit(m[3])) ||
+         (zero(m[0]) && zero(m[3]) && unit(m[1]) && unit(m[2]));
+}
 
-// c = a * b for row-major 2x2 matrices.
+// c = a * b for row-major 2x2 matrices.  P: the precision of the products,
+// rounded once at the end.
+template <typename P = double>
 inline void mul2(const cd *a, const cd *b, cd *c) {
+  if (sizeof(P) > sizeof(double) && (exact2(a) || exact2(b))) return mul2<double>(a, b, c);
   cd r[4];
-  r[0] = cadd(cmul(a[0], b[0]), cmul(a[1], b[2]));
-  r[1] = cadd(cmul(a[0], b[1]), cmul(a[1], b[3]));
-  r[2] = cadd(cmul(a[2], b[0]), cmul(a[3], b[2]));
-  r[3] = cadd(cmul(a[2], b[1]), cmul(a[3], b[3]));
+  for (int k = 0; k < 4; ++k) {
+    const cd &x = a[k & 2], &y = a[(k & 2) + 1], &u = b[k & 1], &v = b[2 + (k & 1)];
+    r[k].re = (double)(((P)x.re * u.re - (P)x.im * u.im) + ((P)y.re * v.re - (P)y.im * v.im));
+    r[k].im = (double)(((P)x.re * u.im + (P)x.im * u.re) + ((P)y.re * v.im + (P)y.im * v.re));
+  }
   for (int k = 0; k < 4; ++k) c[k] = r[k];
 }
 
@@ -191,6 +201,10 @@ inline void merge_batched(std::vector<SweepOp> &items, std::deque<Gate> &store) 
   }
 }
 
+// P: the precision of the products of merged 2x2s.  A product's rounding is the
+// same for all amplitudes; where the gates ran one by one before, long double
+// keeps the merged run's error below theirs.
+template <typename P = double>
 inline void merge_sweep_ops(std::vector<SweepOp> &items, const int *slot, uint64_t reg_qubits) {
   int last[64], lastx[64];  // last op touching q at all / non-diagonally
   for (int q = 0; q < 64; ++q) last[q] = lastx[q] = -1;
@@ -218,8 +232,8 @@ inline void merge_sweep_ops(std::vector<SweepOp> &items, const int *slot, uint64
           // multiplexed (or merged plain) op at j; t may also be one of its
           // pattern qubits, which is not a merge
           if (J.t == t) {  // u moves back to j
-            mul2(u, J.m0, J.m0);
-            mul2(u, J.m1, J.m1);
+            mul2<P>(u, J.m0, J.m0);
+            mul2<P>(u, J.m1, J.m1);
             // the op at j may have been diagonal on t; with u it may not be
             if (!diagonal2(u)) lastx[t] = j;
             merged = true;
@@ -229,7 +243,7 @@ inline void merge_sweep_ops(std::vector<SweepOp> &items, const int *slot, uint64
           J.g = nullptr;
           J.t = t;
           J.pm = J.pv = 0;
-          mul2(u, uj, J.m1);
+          mul2<P>(u, uj, J.m1);
           for (int k = 0; k < 4; ++k) J.m0[k] = J.m1[k];
           if (!diagonal2(J.m1)) lastx[t] = j;
           merged = true;
@@ -242,7 +256,7 @@ inline void merge_sweep_ops(std::vector<SweepOp> &items, const int *slot, uint64
             J.pm = pm;
             J.pv = pv;
             for (int k = 0; k < 4; ++k) J.m0[k] = u[k];
-            mul2(u, mt, J.m1);
+            mul2<P>(u, mt, J.m1);
             // a phase pattern acted diagonally on t; the merged op does not
             lastx[t] = j;
             merged = true;
@@ -270,7 +284,7 @@ inline void merge_sweep_ops(std::vector<SweepOp> &items, const int *slot, uint64
           G.pm = pm;
           G.pv = pv;
           for (int k = 0; k < 4; ++k) G.m0[k] = uj[k];
-          mul2(mt, uj, G.m1);
+          mul2<P>(mt, uj, G.m1);
           J.alive = false;
           merged = true;
           last[t] = lastx[t] = i;
@@ -280,7 +294,7 @@ inline void merge_sweep_ops(std::vector<SweepOp> &items, const int *slot, uint64
           bool still = true;
           for (uint64_t b = pm; b; b &= b - 1) still = still && lastx[__builtin_ctzll(b)] < j;
           if (!still) continue;
-          mul2(mt, J.m1, J.m1);
+          mul2<P>(mt, J.m1, J.m1);
           G.alive = false;
           merged = true;
         }
