@@ -485,3 +485,46 @@ def test_gradients_as_close_as_one_operation_at_a_time(n, batch, bound):
     ex.forward(th)
     err = ex.backward() - long_gradients(n, ans, masks, coeffs, th)
     assert np.sqrt(np.mean(err ** 2)) < bound
+
+
+@pytest.mark.parametrize("dtype,tol", [("c128", 1e-11), ("c64", 1e-4)])
+@pytest.mark.parametrize("n", [2, 5, 8, 10, 12, 13])
+def test_reverse_blocks_against_the_shift_rule(n, dtype, tol):
+    """Every parameter of circuits with every record of the reverse blocks
+    (rotations about all axes, several Z rotations of one qubit in a row,
+    phases and diagonals on and off the tile, dense and controlled 2x2s, a 4x4
+    in between), of all parameter sets of a batch that is no power of two."""
+    rng = np.random.default_rng(40 + n)
+    pc = ParamCircuit(n)
+    for step in range(90):
+        k = int(rng.integers(0, 10))
+        a, b = (int(q) for q in rng.permutation(n)[:2])
+        if k < 5:
+            pc.rotation("xyzzz"[k], a, pc.nparams)
+            if k == 4:
+                pc.rotation("z", a, pc.nparams)
+        elif k == 5:
+            pc.gate(np.diag(np.exp(1j * rng.random(4) * 6)), [a, b])
+        elif k == 6:
+            pc.gate(ops.cz(a, b).matrix(), [a, b])
+        elif k == 7:
+            pc.gate(np.diag([1, 1, 1, np.exp(0.7j)]), [a, b])
+        elif k == 8:
+            g = ops.cnot(a, b) if step % 2 else ops.to_controlled(ops.Operation(random_u(rng, 2), [a]), b)
+            pc.gate(g.matrix(), g.targets())
+        else:
+            pc.gate(random_u(rng, 4 if step % 3 == 0 else 2), [a, b] if step % 3 == 0 else [a])
+        if step % 30 == 29:
+            pc.layer()
+    masks, coeffs = circuits.zz_chain_observable(n)
+    th = rng.random((3, pc.nparams)) * 6.2
+    want = shift_gradients(Expectation(pc, masks, coeffs), th)
+    for every in (0, 1):
+        ex = Expectation(pc, masks, coeffs, dtype=dtype, checkpoint_every=every)
+        ex.forward(th)
+        assert np.max(np.abs(ex.backward() - want)) < tol
+
+
+def random_u(rng, d):
+    q, r = np.linalg.qr(rng.standard_normal((d, d)) + 1j * rng.standard_normal((d, d)))
+    return q * (np.diag(r) / np.abs(np.diag(r)))
