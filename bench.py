@@ -249,7 +249,10 @@ def adjoint_bench(n: int, layers: int, batch: int, fd_params: int, dtype: str):
     S = float(batch << n) * (16 if dtype == "c128" else 8)
     rstats = run.reverse_stats
     bwd_bytes = rstats["blocks"] * 4 * S - S
-    fwd_bytes = fstats["sweeps"] * 2 * S
+    # forward: each sweep reads and writes the states (2S), but for the first
+    # (the part that its gates reach from |0...0>, a 256th at 20 qubits) and
+    # the second's reads (of that part): both are left out
+    fwd_bytes = max(2 * fstats["sweeps"] - 3, 0) * S
     # central finite differences (h = 1e-4, FP64) on the same GPU for a sample
     # of parameters: each needs two forward passes of the whole batch.
     h = 1e-4
