@@ -393,7 +393,10 @@ hipError_t execute_t(SweepRunner &run, const std::vector<Gate> &gates, uint64_t 
   while (true) {
     while (first < G && done[first]) ++first;
     if (first == G) break;
-    if (!sweepable(gates[first], lowb)) {
+    // (a batched 2x2 of more states than a descriptor has room for is no
+    // sweep's either)
+    if (!sweepable(gates[first], lowb) ||
+        blob_bytes<R>(op_count(gates[first]), pool_count(gates[first])) > kMaxBlobBytes<R>) {
       hipError_t e = sweep_settle(run);
       if (e == hipSuccess) e = run.single(gates[first]);
       if (e != hipSuccess) return e;

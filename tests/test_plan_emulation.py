@@ -12,6 +12,7 @@ GPU tests.
 import ctypes
 import os
 import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -81,6 +82,7 @@ def emu(tmp_path_factory):
         out = dict(zip(["sweeps", "singles", "sweep_ops", "merged"], map(int, stats)))
         out["hist"] = hist
         return st, out
+    run.path = out
     return run
 
 
@@ -169,6 +171,34 @@ def test_batched_rotations_plan(tmp_path):
             for m, t in per_state[b]:
                 ref = oracle.apply_fast(ref, m, t)
             assert np.max(np.abs(st[b << n:(b + 1) << n] - ref)) < TOL[dtype], (dtype, b)
+
+
+@pytest.mark.parametrize("dtype,nb", [("c128", 12), ("c128", 13), ("c64", 10), ("c64", 11)])
+def test_batches_beyond_a_sweeps_descriptor(emu, dtype, nb):
+    """A batched rotation whose matrices alone fill a descriptor runs by
+    itself; the planner goes on behind it.  (Planned in a process of its own,
+    with a time limit.)"""
+    code = f"""
+import ctypes, sys
+import numpy as np
+lib = ctypes.CDLL({emu.path!r})
+B = 1 << {nb}
+one = np.array([0.6, 0.8, -0.8, 0.6], dtype=np.complex128)
+mats = np.concatenate([np.tile(one, B), one, one, one] * 2)
+t = np.array([3, 3, 4, 5, 9, 9, 10, 11], dtype=np.uint64)
+ks = np.ones(8, dtype=np.int32)
+bm = np.array([B - 1, 0, 0, 0] * 2, dtype=np.uint32)
+stats = np.zeros(4, dtype=np.uint64)
+err = ctypes.create_string_buffer(512)
+p = lambda a: ctypes.c_void_p(a.ctypes.data)
+rc = lib.emu_run2(14 + {nb}, {int(dtype == "c64")}, None, 8, p(mats), p(t), p(ks), None, None,
+                  p(bm), 14, p(stats), None, err, 512)
+print(rc, *stats[:2])
+"""
+    out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=60)
+    rc, sweeps, singles = (int(v) for v in out.stdout.split())
+    assert rc == 0 and sweeps >= 1
+    assert singles == (2 if nb in (11, 13) else 0)
 
 
 @pytest.mark.parametrize("dtype", ["c128", "c64"])
