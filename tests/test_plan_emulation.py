@@ -198,7 +198,8 @@ print(rc, *stats[:2])
     out = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=60)
     rc, sweeps, singles = (int(v) for v in out.stdout.split())
     assert rc == 0 and sweeps >= 1
-    assert singles == (2 if nb in (11, 13) else 0)
+    # (the last gate on qubit 9 is alone behind the second rotation)
+    assert singles == (3 if nb in (11, 13) else 0)
 
 
 @pytest.mark.parametrize("dtype", ["c128", "c64"])
