@@ -528,3 +528,21 @@ def test_reverse_blocks_against_the_shift_rule(n, dtype, tol):
 def random_u(rng, d):
     q, r = np.linalg.qr(rng.standard_normal((d, d)) + 1j * rng.standard_normal((d, d)))
     return q * (np.diag(r) / np.abs(np.diag(r)))
+
+
+@pytest.mark.parametrize("dtype,batch,tol", [("c128", 8200, 1e-11), ("c64", 2050, 1e-4)])
+def test_batches_beyond_a_sweeps_descriptor(dtype, batch, tol):
+    """Rotations of so many parameter sets that a sweep has no room for their
+    matrices: energies and gradients of some of the sets alone."""
+    n = 12
+    ans = circuits.hardware_efficient_ansatz(n, 1)
+    masks, coeffs = circuits.zz_chain_observable(n)
+    th = circuits.seeded_thetas(batch, ans.nparams, seed=23)
+    pc = ParamCircuit.from_ansatz(ans)
+    ex = Expectation(pc, masks, coeffs, dtype=dtype)
+    e = ex.forward(th)
+    g = ex.backward()
+    some = [0, batch // 3, batch - 1]
+    one = Expectation(pc, masks, coeffs)
+    assert np.max(np.abs(e[some] - one.forward(th[some]))) < tol * n
+    assert np.max(np.abs(g[some] - one.backward())) < tol * n
