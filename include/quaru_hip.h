@@ -61,7 +61,12 @@ int qs_last_error(size_t *a, size_t *b, const char **message);
 /* Library version string. */
 const char *qs_version(void);
 
-/* ---- construction (src/register.rs:41-102) ------------------------------ */
+/* ---- construction (src/register.rs:41-102) ------------------------------
+ *
+ * qs_register_new and qs_register_from_int allocate the state but write
+ * nothing yet: gates start from the index, and the first call that needs
+ * amplitudes in memory writes them.  A launch that fails there is reported by
+ * that call (a failed allocation still by the constructor). */
 
 /* Register::new (src/register.rs:41-56): bits[i] != 0 sets qubit i. */
 int qs_register_new(const unsigned char *bits, size_t n, int dtype, qs_register **out);

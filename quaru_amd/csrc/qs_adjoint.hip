@@ -568,16 +568,18 @@ __device__ __forceinline__ uint32_t rev_pos(uint32_t j) { return j ^ ((j >> 3) &
 // share of the gradient of the rotation with that row.
 //
 // Bound by vector and LDS work beside the memory pass.  Backward of the
-// 20-qubit, 10-layer, batch-64 ansatz, complex128 (15 blocks, 4 GiB of
-// traffic each, 0.81 ms at the card's copy rate): 24.2 ms, 1.24 ms per block
-// with the vector units 51% busy (1490 instructions per wave).  Steps there:
-// 66 ms (55 blocks of 1.11 ms, operations in strict order, one exchange and
-// one descriptor fetch per rotation); 34.5 ms with commuting blocks and
-// diagonal passes (2280 instructions); 28.4 ms with descriptors fetched
-// ahead, cosines and sines in LDS and sums on the matrix cores (by 16 x 16
-// FP64 products instead of 4 x 4: 35.7 ms); 24.2 ms with one multiply-add per
-// component and tables for signs and lane sums.  Complex64: 45 to 17.8 ms.
-// Tiles of 2^11 complex128 amplitudes, two workgroups per CU: 27.3 ms.
+// 20-qubit, 10-layer, batch-64 ansatz, complex128: 20.7 ms in 15 blocks of
+// 1.34-1.39 ms (4 GiB of traffic each, 0.81 ms at the card's copy rate).
+// Complex64, in strict order: 31 ms in 25 blocks of 1.20 ms.  Steps there in
+// complex128, with 0.44 ms copies at four checkpoints and a kernel for lambda
+// still outside: 66 ms (55 blocks of 1.11 ms, operations in strict order, one
+// exchange and one descriptor fetch per rotation); 34.5 ms with commuting
+// blocks and diagonal passes (2280 instructions per wave); 28.4 ms with
+// descriptors fetched ahead, cosines and sines in LDS and sums on the matrix
+// cores (by 16 x 16 FP64 products instead of 4 x 4: 35.7 ms); 24.2 ms with one
+// multiply-add per component and tables for signs and lane sums (1490
+// instructions, the vector units 51% busy).  Tiles of 2^11 complex128
+// amplitudes, two workgroups per CU: 27.3 ms then.
 template <typename R, int PER>
 __global__ __launch_bounds__(kBlock)
 __attribute__((amdgpu_waves_per_eu(PER < 8 ? 4 : (sizeof(R) == 8 ? 2 : 3)))) void k_reverse_tile(typename AV2<R>::T *__restrict__ psi,
@@ -1566,7 +1568,7 @@ bool adjoint_fused_reverse() {
 
 // Qubits 0 .. low - 1 are on every tile of the reverse blocks: runs of 128
 // bytes.  One qubit more (256-byte runs) measured the same per block (20
-// qubits, batch 64: 24.2 ms backward either way) and leaves one less for the
+// qubits, batch 64) and leaves one less for the
 // pair targets.
 int reverse_low_bits(int dtype) { return dtype == QS_C128 ? 3 : 4; }
 

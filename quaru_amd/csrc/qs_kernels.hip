@@ -824,7 +824,8 @@ __device__ __forceinline__ int tile_phys(int s) { return s ^ (((s >> 4) ^ (s >> 
 // (16 or 32 KiB) keep several workgroups per CU and fill the chip from 15
 // qubits on.  Bound by memory for K = 4 and 5, by the matrix cores' FP64 rate
 // for K = 6: 27 qubits, 6 targets 1.2 ms a gate (57 TFLOP/s, 3.6 TB/s), 29.6
-// ms with one thread per output; 5 targets on low qubits 0.80 ms, 1.17 ms in
+// ms with one thread per output; 5 targets with low qubits among them 0.80 ms
+// (all low) to 1.02 ms (the others spread over far bits), 1.17 ms in
 // k_gatek_staged; 15 qubits, 5 targets 4.9 us, 36 us in k_gatek.
 template <int K, int LC, bool kReal, bool kNT>
 __global__ __launch_bounds__(256, 2) void k_dense_tile(double2 *__restrict__ psi, uint64_t ntiles,
@@ -2313,7 +2314,8 @@ __global__ __launch_bounds__(kBlock) void k_chunk_sums(const typename V2<R>::T *
 // by DPP.  1000 shots of 26 qubits, complex128: 543 us, 620 with every value
 // read from LDS by all lanes (four waves of a CU share its LDS); with the
 // readouts beside it 1.39 ms, against 110 ms with the ~640 hit chunks'
-// probabilities copied to and scanned on the host.
+// probabilities copied to and scanned on the host.  (A few shots are: see
+// sample_on_host.)
 constexpr int kSampleLoads = 16;
 constexpr int kSampleTrip = 64 * kSampleLoads;
 constexpr int kSampleGroup = 64;  // additions between two looks at the sum
